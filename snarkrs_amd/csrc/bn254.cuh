@@ -230,8 +230,18 @@ HD Fp<C> mul(const Fp<C>& a, const Fp<C>& b) {
 // carries lazily (each stays below 2^63: at most 18 products of 2^58 land in one column), so
 // the loop has no carry flags at all, which the 32-bit form above needs on every step. On
 // gfx950 this runs 1.42x the 32-bit form's products per second. Inputs and output are the
-// usual 8 x 32-bit limbs, the output fully reduced. M29 gives the modulus in 29-bit limbs and
-// -modulus^-1 mod 2^29.
+// usual 8 x 32-bit limbs, the output fully reduced. M29 gives the modulus in 29-bit limbs,
+// -modulus^-1 mod 2^29 and w = 2^-29 mod the modulus.
+//
+// Seven of the nine reduction steps drop a column without a quotient digit: a column
+// t = hi 2^32 + lo of weight 2^(29 i) is worth (8 hi + lo w) 2^(29 (i + 1)), since 2^32 = 8 2^29
+// and 1 = 2^29 w. That is ten multiply-adds straight from the column's two words, where a
+// Montgomery step is nine, a product for the digit, a mask, a 64-bit shift and an addition,
+// each waiting for the one before. Each such step adds less than 2^32 w 2^(29 (i + 1)) to the
+// value, 2^-25 modulus in all once divided by 2^261; the last two steps are Montgomery's, so
+// that the quotient keeps its bound (below the product's share plus one modulus).
+// Product chains on the MI355X: 1223 -> 1051 cycles per product with one wave on a SIMD,
+// 1153 -> 956 with three.
 struct Fq29 {
   using Cfg = FqCfg;
   static HD uint32_t p29(int j) {
@@ -240,6 +250,13 @@ struct Fq29 {
     return P[j];
   }
   static constexpr uint32_t N29 = 0x04866389u;
+  // 2^-29 + 2q mod 2^261: of the small multiples of q added to 2^-29 mod q, the one whose
+  // limbs are smallest (any seven consecutive ones sum to at most 1.65 2^29).
+  static HD uint32_t w29(int j) {
+    constexpr uint32_t W[9] = {0x0872952du, 0x0808854au, 0x065124e0u, 0x029b9885u, 0x03f6b850u,
+                               0x148e9764u, 0x02b3e954u, 0x0843f777u, 0x0067a061u};
+    return W[j];
+  }
 };
 
 struct Fr29 {
@@ -250,6 +267,11 @@ struct Fr29 {
     return P[j];
   }
   static constexpr uint32_t N29 = 0x0fffffffu;
+  static HD uint32_t w29(int j) {  // 2^-29 mod r
+    constexpr uint32_t W[9] = {0x18f05361u, 0x012bb1feu, 0x0f5d8135u, 0x1e6275f6u, 0x07e7a880u,
+                               0x10c6bf1fu, 0x11f74a6cu, 0x06fdaecbu, 0x00183227u};
+    return W[j];
+  }
 };
 
 // The 29-bit limbs of an 8 x 32-bit value, and back (a value below 2^256 in limbs < 2^29).
@@ -291,32 +313,46 @@ HD void pack29(const uint32_t R[9], uint32_t out[8]) {
   out[7] = word29_at<7>(R);
 }
 
+// 8, kept from the compiler: it would turn the multiply-add by a known 8 into a 64-bit shift, a
+// mask and a 64-bit addition.
+HD uint32_t opaque8() {
+  uint32_t e = 8u;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("" : "+s"(e));
+#endif
+  return e;
+}
+
 // The product on limbs: A B 2^-261 mod the modulus, in [0, 2 modulus) (any inputs below
 // 2^256), as nine 29-bit limbs.
 template <class M29>
 HD void mont29_limbs(const uint32_t A[9], const uint32_t B[9], uint32_t R[9]) {
   constexpr uint32_t MASK = (1u << 29) - 1u;
-  uint64_t t[10];
+  uint64_t t[17];
 #pragma unroll
-  for (int j = 0; j < 10; ++j) t[j] = 0;
+  for (int k = 0; k < 17; ++k) t[k] = 0;
 #pragma unroll
   for (int i = 0; i < 9; ++i) {
 #pragma unroll
-    for (int j = 0; j < 9; ++j) t[j] += (uint64_t)A[j] * B[i];
-    // m = t0 * N29 mod 2^29; the low 32 bits of the product suffice, unmasked t0 included.
-    const uint32_t m = ((uint32_t)t[0] * M29::N29) & MASK;
+    for (int j = 0; j < 9; ++j) t[i + j] += (uint64_t)A[j] * B[i];
+    if (i < 7) {
+      const uint32_t lo = (uint32_t)t[i], hi = (uint32_t)(t[i] >> 32);
+      t[i + 1] += (uint64_t)hi * opaque8();
 #pragma unroll
-    for (int j = 0; j < 9; ++j) t[j] += (uint64_t)m * M29::p29(j);
-    t[1] += t[0] >> 29;  // t[0] is now a multiple of 2^29
+      for (int j = 0; j < 9; ++j) t[i + 1 + j] += (uint64_t)lo * M29::w29(j);
+    } else {
+      // m = t_i * N29 mod 2^29; the low 32 bits of the product suffice, unmasked t_i included.
+      const uint32_t m = ((uint32_t)t[i] * M29::N29) & MASK;
 #pragma unroll
-    for (int j = 0; j < 9; ++j) t[j] = t[j + 1];
-    t[9] = 0;
+      for (int j = 0; j < 9; ++j) t[i + j] += (uint64_t)m * M29::p29(j);
+      if (i < 8) t[i + 1] += t[i] >> 29;  // t[i] is now a multiple of 2^29
+    }
   }
   // Carry the columns into 29-bit limbs (the value is below 2 modulus < 2^255).
-  uint64_t c = 0;
+  uint64_t c = t[8] >> 29;
 #pragma unroll
   for (int j = 0; j < 9; ++j) {
-    const uint64_t x = t[j] + c;
+    const uint64_t x = (j < 8 ? t[9 + j] : 0) + c;
     c = x >> 29;
     R[j] = (uint32_t)x & MASK;
   }
@@ -343,20 +379,30 @@ HD void wide_msub(uint64_t t[17], const uint32_t A[9], const uint32_t B[9]) {
 }
 
 // t 2^-261 mod the modulus as nine 29-bit limbs in [0, 2 modulus), for a wide value
-// V = sum_k t[k] 2^(29 k) with -2^261 modulus < V < 2^261 modulus whose columns each hold at
-// most 18 partial products of limbs below 2^29 (|t[k]| <= 18 2^58; the reduction's nine
-// products and the carries keep every column below 27 2^58 + 2^34 < 2^63). The quotient
-// (V + M modulus) / 2^261, M < 2^261, lies in (-modulus, 2 modulus); a negative one gets the
+// V = sum_k t[k] 2^(29 k), |V| < (1 - 2^-24) 2^261 modulus, that sums at most two products
+// of each sign (operands below 16 modulus in limbs below 2^29 + 8). A column then holds at most
+// 16 partial products of such limbs and two with a top limb, below 2^26 (|t[k]| < 16.1 2^58);
+// the steps add 2^32 times at most seven consecutive limbs of w (1.65 2^61 = 13.2 2^58 for q),
+// the digits' two products and the carries, so every column stays below
+// 31.4 2^58 < 2^63. The quotient lies in (-modulus, 2 modulus); a negative one gets the
 // modulus added (NEG = false: V >= 0, nothing to add).
 template <class M29, bool NEG = true>
 HD void redc29(uint64_t t[17], uint32_t R[9]) {
   constexpr uint32_t MASK = (1u << 29) - 1u;
 #pragma unroll
   for (int i = 0; i < 9; ++i) {
-    const uint32_t m = ((uint32_t)t[i] * M29::N29) & MASK;
+    if (i < 7) {
+      const uint32_t lo = (uint32_t)t[i];
+      const int32_t hi = (int32_t)(t[i] >> 32);
+      t[i + 1] += (uint64_t)((int64_t)hi * (int64_t)(int32_t)opaque8());
 #pragma unroll
-    for (int j = 0; j < 9; ++j) t[i + j] += (uint64_t)m * M29::p29(j);
-    if (i < 8) t[i + 1] += (uint64_t)((int64_t)t[i] >> 29);  // t[i] is now 0 mod 2^29
+      for (int j = 0; j < 9; ++j) t[i + 1 + j] += (uint64_t)lo * M29::w29(j);
+    } else {
+      const uint32_t m = ((uint32_t)t[i] * M29::N29) & MASK;
+#pragma unroll
+      for (int j = 0; j < 9; ++j) t[i + j] += (uint64_t)m * M29::p29(j);
+      if (i < 8) t[i + 1] += (uint64_t)((int64_t)t[i] >> 29);  // t[i] is now 0 mod 2^29
+    }
   }
   // The quotient's columns are t[9..16] plus the carry out of t[8].
   int64_t c = (int64_t)t[8] >> 29;
@@ -973,6 +1019,40 @@ HD G1L g1l_inf() {
   return r;
 }
 
+HD uint32_t q4_29(int j) {  // 4q, exact limbs
+  constexpr uint32_t K[9] = {0x01f3f51cu, 0x041182dbu, 0x11ca8d3cu, 0x0b548b43u, 0x161765e0u,
+                             0x0b6d0302u, 0x029b8504u, 0x197098d0u, 0x00c19139u};
+  return K[j];
+}
+
+// A value below 9q in limbs below 2^32, to exact limbs and below 5q.
+HD void below5q(uint32_t x[9]) {
+  constexpr uint32_t MASK = (1u << 29) - 1u;
+  uint32_t c = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t v = x[j] + c;
+    x[j] = v & MASK;
+    c = v >> 29;
+  }
+  x[8] += c;
+  uint32_t d[9];
+  int32_t b = 0;
+#pragma unroll
+  for (int j = 0; j < 9; ++j) {
+    const int32_t v = (int32_t)x[j] - (int32_t)q4_29(j) + b;
+    d[j] = (uint32_t)v & MASK;
+    b = v >> 29;  // 0 or -1
+  }
+#pragma unroll
+  for (int j = 0; j < 9; ++j) x[j] = b < 0 ? x[j] : d[j];
+}
+
+HD void wide_zero(uint64_t t[17]) {
+#pragma unroll
+  for (int k = 0; k < 17; ++k) t[k] = 0;
+}
+
 HD Xyzz<Fm> g1l_out(const G1L& p) {
   uint32_t one[9], X[9];
 #pragma unroll
@@ -1132,40 +1212,6 @@ struct Kq6 {  // 6q, b' = 2
     return K[j];
   }
 };
-HD uint32_t q4_29(int j) {  // 4q, exact limbs
-  constexpr uint32_t K[9] = {0x01f3f51cu, 0x041182dbu, 0x11ca8d3cu, 0x0b548b43u, 0x161765e0u,
-                             0x0b6d0302u, 0x029b8504u, 0x197098d0u, 0x00c19139u};
-  return K[j];
-}
-
-// A value below 9q in limbs below 2^32, to exact limbs and below 5q.
-HD void below5q(uint32_t x[9]) {
-  constexpr uint32_t MASK = (1u << 29) - 1u;
-  uint32_t c = 0;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const uint32_t v = x[j] + c;
-    x[j] = v & MASK;
-    c = v >> 29;
-  }
-  x[8] += c;
-  uint32_t d[9];
-  int32_t b = 0;
-#pragma unroll
-  for (int j = 0; j < 9; ++j) {
-    const int32_t v = (int32_t)x[j] - (int32_t)q4_29(j) + b;
-    d[j] = (uint32_t)v & MASK;
-    b = v >> 29;  // 0 or -1
-  }
-#pragma unroll
-  for (int j = 0; j < 9; ++j) x[j] = b < 0 ? x[j] : d[j];
-}
-
-HD void wide_zero(uint64_t t[17]) {
-#pragma unroll
-  for (int k = 0; k < 17; ++k) t[k] = 0;
-}
-
 // r = a b (r must not alias a or b). Both components' sums are formed before either is
 // reduced, so the two reductions' serial chains can interleave.
 HD void f2l_mul(const F2L& a, const F2L& b, F2L& r) {
@@ -1749,18 +1795,25 @@ struct P2L {
   F2L X, Y, Z;
 };
 
-// redc29 for a wide value whose columns are all sums of products (no subtraction): up to 54
-// limb products a column, so that with the reduction's nine they stay below 2^64, and the
-// carries shift unsigned. The value is below 2^261 q, the result below 2q.
+// redc29 for a wide value whose columns are all sums of products (no subtraction): up to 36
+// limb products a column (of limbs below 2^29 + 8: with the reduction 51.3 2^58 < 2^64), and the
+// carries shift unsigned. The value is below (1 - 2^-24) 2^261 q, the result below 2q.
 template <class M29>
 HD void redc29u(uint64_t t[17], uint32_t R[9]) {
   constexpr uint32_t MASK = (1u << 29) - 1u;
 #pragma unroll
   for (int i = 0; i < 9; ++i) {
-    const uint32_t m = ((uint32_t)t[i] * M29::N29) & MASK;
+    if (i < 7) {
+      const uint32_t lo = (uint32_t)t[i], hi = (uint32_t)(t[i] >> 32);
+      t[i + 1] += (uint64_t)hi * opaque8();
 #pragma unroll
-    for (int j = 0; j < 9; ++j) t[i + j] += (uint64_t)m * M29::p29(j);
-    if (i < 8) t[i + 1] += t[i] >> 29;
+      for (int j = 0; j < 9; ++j) t[i + 1 + j] += (uint64_t)lo * M29::w29(j);
+    } else {
+      const uint32_t m = ((uint32_t)t[i] * M29::N29) & MASK;
+#pragma unroll
+      for (int j = 0; j < 9; ++j) t[i + j] += (uint64_t)m * M29::p29(j);
+      if (i < 8) t[i + 1] += t[i] >> 29;
+    }
   }
   uint64_t c = t[8] >> 29;
 #pragma unroll
