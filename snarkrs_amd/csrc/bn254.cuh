@@ -936,7 +936,8 @@ HD Aff<F> xyzz_to_aff(const Xyzz<F>& p) {
 //   X < 9q, limbs below 2^29 + 8 (X3 = R^2 + 7q - PPP - 2Q); Y, ZZ, ZZZ < 2q exact.
 // Each product stays inside mont29_limbs' bound (operands' product below 2^261 q): the largest
 // is P^2 with P = U2 + 10q - X1 < 12q, 144 q^2 < 2^261 q. Every limb sum stays in [0, 2^32).
-// Leaving the loop, X is reduced below 2q by a product with one (g1l_out).
+// Stored for the next kernel, X is taken below 5q (g1l_pack); for the host, below 2q by a
+// product with one (g1l_out).
 struct G1L {
   uint32_t X[9], Y[9], ZZ[9], ZZZ[9];
 };
@@ -1051,6 +1052,23 @@ HD void below5q(uint32_t x[9]) {
 HD void wide_zero(uint64_t t[17]) {
 #pragma unroll
   for (int k = 0; k < 17; ++k) t[k] = 0;
+}
+
+// The form points take between kernels: X below 5q < 2^256, packed by one conditional
+// subtraction of 4q (g1l_out's product is ten times the work, and a wave of the bucket loop
+// stores a lane's run almost every iteration when buckets hold about as many entries as the
+// wave has lanes). g1l_from reads it back; only g1l_out's form goes to the host.
+HD Xyzz<Fm> g1l_pack(const G1L& p) {
+  uint32_t X[9];
+#pragma unroll
+  for (int j = 0; j < 9; ++j) X[j] = p.X[j];
+  below5q(X);
+  Xyzz<Fm> r;
+  pack29(X, r.X.v);
+  pack29(p.Y, r.Y.v);
+  pack29(p.ZZ, r.ZZ.v);
+  pack29(p.ZZZ, r.ZZZ.v);
+  return r;
 }
 
 HD Xyzz<Fm> g1l_out(const G1L& p) {
@@ -1285,6 +1303,20 @@ HD G2L g2l_inf() {
     r.X.c0[j] = r.X.c1[j] = r.Y.c0[j] = r.Y.c1[j] = 0;
     r.ZZ.c0[j] = r.ZZ.c1[j] = r.ZZZ.c0[j] = r.ZZZ.c1[j] = 0;
   }
+  return r;
+}
+
+// The form between kernels (as g1l_pack): X is below 5q in exact limbs already.
+HD Xyzz<Fm2i> g2l_pack(const G2L& p) {
+  Xyzz<Fm2i> r;
+  pack29(p.X.c0, r.X.c0.v);
+  pack29(p.X.c1, r.X.c1.v);
+  pack29(p.Y.c0, r.Y.c0.v);
+  pack29(p.Y.c1, r.Y.c1.v);
+  pack29(p.ZZ.c0, r.ZZ.c0.v);
+  pack29(p.ZZ.c1, r.ZZ.c1.v);
+  pack29(p.ZZZ.c0, r.ZZZ.c0.v);
+  pack29(p.ZZZ.c1, r.ZZZ.c1.v);
   return r;
 }
 

@@ -195,7 +195,7 @@ struct COps<Fm> {
 
 // The tails' additions (merges, heavy buckets, reduction): XOps, or for G1 and G2 the limb
 // forms (LOps): points are loaded into limbs, added there, and packed back to the XYZZ words
-// (X reduced below 2q) when stored.
+// (X below 5q) when stored; `out`, for the host, has X below 2q.
 template <class F>
 struct LOps : XOps<F> {};
 template <>
@@ -207,7 +207,7 @@ struct LOps<Fm> {
     return g1l_from(ld_xyzz<Fm>(base, i));
   }
   static __device__ __forceinline__ void store(uint4* base, size_t i, const P& p) {
-    st_xyzz(base, i, g1l_out(p));
+    st_xyzz(base, i, g1l_pack(p));
   }
   static __device__ __forceinline__ Xyzz<Fm> out(const P& p) { return g1l_out(p); }
 };
@@ -220,7 +220,7 @@ struct LOps<Fm2i> {
     return g2l_from(ld_xyzz<Fm2i>(base, i));
   }
   static __device__ __forceinline__ void store(uint4* base, size_t i, const P& p) {
-    st_xyzz(base, i, g2l_out(p));
+    st_xyzz(base, i, g2l_pack(p));
   }
   static __device__ __forceinline__ Xyzz<Fm2i> out(const P& p) { return g2l_out(p); }
 };
@@ -267,7 +267,7 @@ struct Acc<Fm> {
                                            const uint4*, uint32_t) {
     return g1l_madd(p, a, negate);
   }
-  static __device__ __forceinline__ Xyzz<Fm> out(const T& p) { return g1l_out(p); }
+  static __device__ __forceinline__ Xyzz<Fm> out(const T& p) { return g1l_pack(p); }
 };
 
 template <>
@@ -288,7 +288,7 @@ struct Acc<Fm2i> {
     if (k == 2) return g2l_inf();
     return r;
   }
-  static __device__ __forceinline__ Xyzz<Fm2i> out(const T& p) { return g2l_out(p); }
+  static __device__ __forceinline__ Xyzz<Fm2i> out(const T& p) { return g2l_pack(p); }
 };
 
 // Segment t of the sorted entries: its runs added into XYZZ accumulators, a run whole inside

@@ -4,6 +4,7 @@
 //   q, r    mont29_limbs over Fq / Fr (two operands)
 //   s       redc29 of a b + c d - e f - g h;  p  redc29 of a b + c d, which is never negative
 //   u       redc29u of a b + c d + e f + g h
+//   x       g1l_pack's X (one operand), as eight words
 #include <cstdio>
 
 #include "../../snarkrs_amd/csrc/bn254.cuh"
@@ -13,16 +14,23 @@ using namespace g16;
 int main() {
   char op;
   while (std::scanf(" %c", &op) == 1) {
-    const int n = op == 'q' || op == 'r' ? 2 : op == 'p' ? 4 : 8;
+    const int n = op == 'q' || op == 'r' ? 2 : op == 'x' ? 1 : op == 'p' ? 4 : 8;
     uint32_t v[8][9], R[9] = {};
     for (int i = 0; i < n; ++i)
       for (int j = 0; j < 9; ++j)
         if (std::scanf("%u", &v[i][j]) != 1) return 1;
     uint64_t t[17] = {};
+    int len = 9;
     if (op == 'q') {
       mont29_limbs<Fq29>(v[0], v[1], R);
     } else if (op == 'r') {
       mont29_limbs<Fr29>(v[0], v[1], R);
+    } else if (op == 'x') {
+      G1L p = g1l_inf();
+      for (int j = 0; j < 9; ++j) p.X[j] = v[0][j];
+      const Xyzz<Fm> w = g1l_pack(p);
+      for (int j = 0; j < 8; ++j) R[j] = w.X.v[j];
+      len = 8;
     } else {
       wide_mac(t, v[0], v[1]);
       wide_mac(t, v[2], v[3]);
@@ -38,7 +46,7 @@ int main() {
         redc29u<Fq29>(t, R);
       }
     }
-    for (int j = 0; j < 9; ++j) std::printf("%u ", R[j]);
+    for (int j = 0; j < len; ++j) std::printf("%u ", R[j]);
     std::printf("\n");
   }
   return 0;

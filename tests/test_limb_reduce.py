@@ -1,5 +1,5 @@
 """The limb products' and reductions' results and bounds at their edges (bn254.cuh mont29_limbs,
-redc29, redc29u) against Python integers, on the host: every operand at the top of its
+redc29, redc29u, g1l_pack) against Python integers, on the host: every operand at the top of its
 bound, limbs raised to 2^29 + 7, zero, multiples of the modulus, and random ones."""
 import os
 import random
@@ -94,3 +94,13 @@ def test_sums(run, op, bounds):
         got = value(r)
         assert all(x < 2**29 for x in r)
         assert got < 2 * Q_MOD and (got * 2**261 - want) % Q_MOD == 0
+
+
+def test_pack(run):
+    rng = random.Random(7)
+    xs = operands(Q_MOD, 9, rng)
+    xs += [limbs(k * Q_MOD + d) for k in range(9) for d in (0, 1)]
+    xs += [limbs(k * Q_MOD - 1) for k in range(1, 10)]
+    for x, r in zip(xs, run([("x", [x]) for x in xs])):
+        got = sum(w << (32 * j) for j, w in enumerate(r))
+        assert got < 5 * Q_MOD and (got - value(x)) % Q_MOD == 0
