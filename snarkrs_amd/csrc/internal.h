@@ -149,13 +149,36 @@ size_t msm_accum_scratch_bytes(const MsmPlan& p, int group);
 // merges and after the window reduction.
 void msm_accumulate(const MsmPlan& p, int group, const void* bases, void* scratch,
                     void* window_out, hipStream_t s, hipEvent_t* ev = nullptr);
-// The G1 bucket accumulations of n <= 4 MSMs (plans[k] sorted, bases[k] in the MSM form,
-// scratch[k] of msm_accum_scratch_bytes) as ONE persistent launch whose workgroups take tiles
-// of segments of every job from a device-side counter (a device word of the caller, 16 bytes,
-// cleared by a kernel here), then each MSM's merges and reduction into window_out[k].
+// The G1 bucket accumulations of n <= TAIL_JOBS variable-work MSMs (plans[k] sorted, bases[k] in
+// the MSM form, scratch[k] of msm_accum_scratch_bytes), then their merges and reductions into
+// window_out[k], every launch over all of them. _together: MSMs over one plan's entries, side by
+// side (ev as msm_accumulate's). _queue: ONE persistent accumulation launch whose workgroups
+// take tiles of segments of every job from a device-side counter (a device word of the caller,
+// 16 bytes, cleared by a kernel here).
+void msm_accumulate_g1_together(const MsmPlan& p, const void* const* bases, void* const* scratch,
+                                void* const* window_out, int n, hipStream_t s, hipEvent_t* ev);
 void msm_accumulate_g1_queue(const MsmPlan* const* plans, const void* const* bases,
                              void* const* scratch, void* const* window_out, int n,
                              uint32_t* counter, hipStream_t s);
+
+// The tail of a variable-work MSM (kernels_msm_tail.hip): K = sets nb buckets from their pieces
+// (the accumulation's whole buckets, first and last partial sums per segment of `seg` entries),
+// then per set `rows` rows over its G groups of B buckets, in S slices each. One launch of each
+// kernel serves every job.
+constexpr int TAIL_JOBS = 4;
+struct TailJob {
+  const uint32_t* offset;
+  uint32_t K, seg, sets, B, G, rows, S;
+  uint32_t avg_pieces;  // entries the plan holds at most, per segment and bucket
+  uint4 *buckets, *pfirst, *plast, *task_sum, *gT, *gU, *parts, *out;
+  uint32_t *heavy, *tasks, *cnt;
+};
+struct TailJobs {
+  TailJob job[TAIL_JOBS];
+  int n;
+};
+void tail_merge_jobs(int group, const TailJobs& t, hipStream_t s);
+void tail_reduce_jobs(int group, const TailJobs& t, hipStream_t s);
 void msm_reduce_shape(const MsmPlan& p, int* rows, int* lg);
 // The MSM kernels keep coordinates in Montgomery form with R' = 2^261 (bn254.cuh Fm): bases go
 // in as 32 x mod q. dst may equal src; n_fq counts 32-byte coordinates.

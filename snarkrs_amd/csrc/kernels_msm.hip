@@ -10,10 +10,11 @@
 //               into XYZZ accumulators (madd-2008-s); a run that fills its bucket inside
 //               the segment is stored as the bucket, the partial runs at a segment's ends go
 //               to side arrays and a merge pass folds them (heavy buckets, e.g. every 1
-//               scalar in bucket 0 of window 0, are cut into tasks summed by LDS trees);
+//               scalar in bucket 0 of window 0, are cut into tasks summed by trees);
 //   4. reduce:  per window S_w = sum_j (j+1) B_j, as group sums and weighted group sums of
-//               8 buckets, then one LDS tree per (window, bit of the group index); the host
+//               4 buckets, then one tree per (window, bit of the group index); the host
 //               finishes with one Horner pass over every window and bit.
+// Merges and reduction (kernels_msm_tail.hip) work on points spread over lanes (msm_quad.cuh).
 // Zero scalars produce no entries and a scalar equal to 1 produces one (window 0, bucket 0),
 // which is the reference prescan's effect (crates/msm/src/lib.rs:534-690) without a pass of
 // its own; bases at infinity are skipped where they are loaded.
@@ -760,14 +761,14 @@ size_t msm_accum_scratch_bytes(const MsmPlan& p, int group) {
 }
 
 template <>
-void Tail<Fm>::merge(const MsmPlan& p, const AccumPtrs& a, hipStream_t s) {
-  tail_merge_impl<Fm>(p, a, s);
+void ConstTail<Fm>::fold(const AccumPtrs& a, hipStream_t s) {
+  tail_fold_const<Fm>(a, s);
 }
 
 template <>
-void Tail<Fm>::reduce(const MsmPlan& p, const AccumPtrs& a, uint32_t B, void* window_out,
-                      hipStream_t s) {
-  tail_reduce_impl<Fm>(p, a, B, window_out, s);
+void ConstTail<Fm>::reduce(const MsmPlan& p, const AccumPtrs& a, uint32_t B, void* window_out,
+                           hipStream_t s) {
+  tail_reduce_ops<Fm, COps<Fm>>(p, a, B, window_out, s);
 }
 
 // Window tables: entry w n + i = 2^(c w) P_i from P_i at entry i, one thread per point.
@@ -820,13 +821,22 @@ static int queue_grid() {
 void msm_accumulate_g1_queue(const MsmPlan* const* plans, const void* const* bases,
                              void* const* scratch, void* const* window_out, int n,
                              uint32_t* counter, hipStream_t s) {
-  accumulate_queue_impl<Fm>(plans, bases, scratch, window_out, n, counter, queue_grid(), s);
+  accumulate_jobs_impl<Fm>(1, plans, bases, scratch, window_out, n, counter, queue_grid(), s,
+                           nullptr);
+}
+
+void msm_accumulate_g1_together(const MsmPlan& p, const void* const* bases, void* const* scratch,
+                                void* const* window_out, int n, hipStream_t s, hipEvent_t* ev) {
+  const MsmPlan* plans[TAIL_JOBS];
+  for (int k = 0; k < TAIL_JOBS; ++k) plans[k] = &p;
+  accumulate_jobs_impl<Fm>(1, plans, bases, scratch, window_out, n, nullptr, 0, s, ev);
 }
 
 void msm_accumulate(const MsmPlan& p, int group, const void* bases, void* scratch,
                     void* window_out, hipStream_t s, hipEvent_t* ev) {
-  if (group == 1) accumulate_impl<Fm>(p, bases, scratch, window_out, s, ev);
-  else msm_accumulate_g2(p, bases, scratch, window_out, s, ev);
+  if (group == 2) msm_accumulate_g2(p, bases, scratch, window_out, s, ev);
+  else if (p.constant) accumulate_const_impl<Fm>(p, bases, scratch, window_out, s, ev);
+  else msm_accumulate_g1_together(p, &bases, &scratch, &window_out, 1, s, ev);
 }
 
 }  // namespace g16

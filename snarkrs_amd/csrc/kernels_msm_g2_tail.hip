@@ -1,11 +1,11 @@
-// G2 bucket merges (spanning and heavy buckets) on Fm2i: see msm_accum.cuh.
+// G2 constant-work fold on Fm2i: see msm_accum.cuh.
 #include "msm_accum.cuh"
 
 namespace g16 {
 
 template <>
-void Tail<Fm2i>::merge(const MsmPlan& p, const AccumPtrs& a, hipStream_t s) {
-  tail_merge_impl<Fm2i>(p, a, s);
+void ConstTail<Fm2i>::fold(const AccumPtrs& a, hipStream_t s) {
+  tail_fold_const<Fm2i>(a, s);
 }
 
 }  // namespace g16

@@ -1,6 +1,7 @@
-// Bucket accumulation, merge and window reduction kernels (templated on the coordinate field),
-// shared by kernels_msm.hip (G1) and kernels_msm_g2.hip (G2). See kernels_msm.hip for the
-// pipeline.
+// Bucket accumulation kernels, the constant-work fold and reduction (templated on the coordinate
+// field), shared by kernels_msm.hip (G1) and kernels_msm_g2*.hip (G2), and the layout of an
+// accumulation's scratch. The variable-work merges and reduction are in kernels_msm_tail.hip.
+// See kernels_msm.hip for the pipeline.
 #pragma once
 #include <algorithm>
 #include <string>
@@ -29,10 +30,11 @@ template <int = 0>
 __global__ void k_clear_cnt(uint32_t* cnt) {
   if (threadIdx.x < 4) cnt[threadIdx.x] = 0;
 }
-// Segments a merge thread folds itself, as a chain of dependent additions; a bucket past it
-// goes to the heavy path's parallel trees. At 32 a few dense buckets (the narrow top window of
-// the standalone G2 MSM) kept the merge running ~450 us with most SIMDs idle.
-static constexpr int HEAVY_SPAN = 8;
+// Segments past its first beyond which a bucket goes to the heavy path's parallel sums, per
+// point that merges it (k_tail_merge): a chain of dependent additions runs on few waves. At 32
+// the dense buckets of the standalone G2 MSM's narrow top window kept its merge running with
+// most SIMDs idle.
+static constexpr uint32_t MERGE_SPAN = 8;
 
 __device__ __forceinline__ Fr ld_fr(const uint4* p) {
   uint4 a = p[0], b = p[1];
@@ -115,19 +117,9 @@ __device__ __forceinline__ void st_xyzz(uint4* base, size_t i, const Xyzz<F>& r)
   st_f(p + 3 * W, r.ZZZ);
 }
 
-// How the merge and reduction kernels see a point: XYZZ with the exceptional-case shortcuts
-// (XOps), or, for constant-work MSMs, (X : Y : Z) with the complete formulas (POps in words;
-// COps below runs them on limbs), stored in an XYZZ-sized slot as (X, Y, Z, 0). `out` is the
-// form the host reads (XYZZ).
-template <class F>
-struct XOps {
-  using P = Xyzz<F>;
-  static __device__ __forceinline__ P inf() { return xyzz_inf<F>(); }
-  static __device__ __forceinline__ P add(const P& a, const P& b) { return xyzz_add(a, b); }
-  static __device__ __forceinline__ P load(const uint4* base, size_t i) { return ld_xyzz<F>(base, i); }
-  static __device__ __forceinline__ void store(uint4* base, size_t i, const P& p) { st_xyzz(base, i, p); }
-  static __device__ __forceinline__ Xyzz<F> out(const P& p) { return p; }
-};
+// How the constant-work kernels see a point: (X : Y : Z) with the complete formulas (POps in
+// words; COps below runs them on limbs), stored in an XYZZ-sized slot as (X, Y, Z, 0). `out` is
+// the form the host reads (XYZZ).
 template <class F>
 struct POps {
   using P = Proj<F>;
@@ -191,38 +183,6 @@ struct COps<Fm> {
     limbs29_of(a.y.v, y);
     return p1l_add_aff(p, x, y);
   }
-};
-
-// The tails' additions (merges, heavy buckets, reduction): XOps, or for G1 and G2 the limb
-// forms (LOps): points are loaded into limbs, added there, and packed back to the XYZZ words
-// (X below 5q) when stored; `out`, for the host, has X below 2q.
-template <class F>
-struct LOps : XOps<F> {};
-template <>
-struct LOps<Fm> {
-  using P = G1L;
-  static __device__ __forceinline__ P inf() { return g1l_inf(); }
-  static __device__ __forceinline__ P add(const P& a, const P& b) { return g1l_add(a, b); }
-  static __device__ __forceinline__ P load(const uint4* base, size_t i) {
-    return g1l_from(ld_xyzz<Fm>(base, i));
-  }
-  static __device__ __forceinline__ void store(uint4* base, size_t i, const P& p) {
-    st_xyzz(base, i, g1l_pack(p));
-  }
-  static __device__ __forceinline__ Xyzz<Fm> out(const P& p) { return g1l_out(p); }
-};
-template <>
-struct LOps<Fm2i> {
-  using P = G2L;
-  static __device__ __forceinline__ P inf() { return g2l_inf(); }
-  static __device__ __forceinline__ P add(const P& a, const P& b) { return g2l_add(a, b); }
-  static __device__ __forceinline__ P load(const uint4* base, size_t i) {
-    return g2l_from(ld_xyzz<Fm2i>(base, i));
-  }
-  static __device__ __forceinline__ void store(uint4* base, size_t i, const P& p) {
-    st_xyzz(base, i, g2l_pack(p));
-  }
-  static __device__ __forceinline__ Xyzz<Fm2i> out(const P& p) { return g2l_out(p); }
 };
 
 // Window tables for merged MSMs (msm_window_tables): entry w n + i = 2^(c w) P_i, affine, from
@@ -344,15 +304,33 @@ __device__ __forceinline__ void accumulate_segment(size_t t, const uint2* __rest
   }
 }
 
+// The accumulations one launch works on: MSMs over the same or other sorted entries, each with
+// its bases and its scratch.
+static constexpr int QUEUE_JOBS = TAIL_JOBS;
+
+struct AccQueueJob {
+  const uint2* ent;
+  const uint32_t* total;
+  const uint4* bases;
+  uint4 *buckets, *pfirst, *plast;
+  uint32_t* cnt;  // heavy buckets and tasks, cleared here for the merges that follow
+  uint64_t nseg;
+  uint32_t seg;
+};
+
+struct AccQueue {
+  AccQueueJob job[QUEUE_JOBS];
+  uint32_t start[QUEUE_JOBS + 1];
+  int n;
+};
+
+// One launch over jobs of the same segment count (blockIdx.y picks the job).
 template <class F>
-__global__ void __launch_bounds__(128) k_accumulate(const uint2* __restrict__ ent,
-                                                    const uint32_t* total, size_t nseg,
-                                                    uint32_t seg,
-                                                    const uint4* __restrict__ bases,
-                                                    uint4* buckets, uint4* pfirst,
-                                                    uint4* plast) {
-  accumulate_segment<F>((size_t)blockIdx.x * blockDim.x + threadIdx.x, ent, total, nseg, seg,
-                        bases, buckets, pfirst, plast);
+__global__ void __launch_bounds__(128) k_accumulate(const AccQueue q) {
+  const AccQueueJob& j = q.job[blockIdx.y];
+  if (blockIdx.x == 0 && threadIdx.x < 4) j.cnt[threadIdx.x] = 0;
+  accumulate_segment<F>((size_t)blockIdx.x * blockDim.x + threadIdx.x, j.ent, j.total, j.nseg,
+                        j.seg, j.bases, j.buckets, j.pfirst, j.plast);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -536,28 +514,14 @@ __global__ void k_fill_proj_inf(uint4* buckets, size_t K) {
 // the grid is sized to what the device holds at once, and each workgroup takes tiles of 128
 // segments from a shared counter until every job's segments are done. Tile t belongs to job
 // d with start[d] <= t < start[d + 1]; segments past a job's device-side entry count end at once.
-static constexpr int QUEUE_JOBS = 4;
 static constexpr uint32_t QUEUE_TILE = 128;  // segments per tile = threads per workgroup
-
-struct AccQueueJob {
-  const uint2* ent;
-  const uint32_t* total;
-  const uint4* bases;
-  uint4 *buckets, *pfirst, *plast;
-  uint64_t nseg;
-  uint32_t seg;
-};
-
-struct AccQueue {
-  AccQueueJob job[QUEUE_JOBS];
-  uint32_t start[QUEUE_JOBS + 1];
-  int n;
-};
 
 template <class F>
 __global__ void __launch_bounds__(QUEUE_TILE) k_accumulate_queue(AccQueue q, uint32_t* counter) {
   __shared__ uint32_t tile;
   const uint32_t tiles = q.start[q.n];
+  if (blockIdx.x == 0 && threadIdx.x < 4)
+    for (int d = 0; d < q.n; ++d) q.job[d].cnt[threadIdx.x] = 0;
   for (;;) {
     if (threadIdx.x == 0) tile = atomicAdd(counter, 1u);
     __syncthreads();
@@ -572,113 +536,8 @@ __global__ void __launch_bounds__(QUEUE_TILE) k_accumulate_queue(AccQueue q, uin
   }
 }
 
-// Buckets that span segments: one thread folds a short span; a heavy one (e.g. every scalar
-// equal to 1, in bucket 0 of window 0) is cut into tasks of HEAVY_TASK interior segments
-// that a two-level tree sums (k_heavy_tasks, k_heavy_finish): depth log2 instead of a chain.
-// cnt[0] = heavy buckets, cnt[1] = tasks; heavy[h] = {bucket, first task, task count};
-// tasks[t] = {first segment, end segment}.
-static constexpr int HEAVY_TASK = 256;
-
-template <class F>
-__global__ void __launch_bounds__(256) k_merge(const uint32_t* offset, uint32_t K, uint4* buckets,
-                                               const uint4* pfirst, const uint4* plast,
-                                               uint32_t* cnt, uint32_t* heavy, uint32_t* tasks,
-                                               uint32_t seg) {
-  uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= K) return;
-  uint32_t s = offset[k], e = offset[k + 1];
-  if (s == e) {
-    st_xyzz(buckets, k, xyzz_inf<F>());
-    return;
-  }
-  uint32_t sa = s / seg, sb = (e - 1) / seg;
-  if (sa == sb) return;  // stored whole by the accumulation
-  if (sb - sa > HEAVY_SPAN) {
-    uint32_t interior = sb - sa - 1;
-    uint32_t ntask = (interior + HEAVY_TASK - 1) / HEAVY_TASK;
-    uint32_t slot = atomicAdd(&cnt[0], 1u);
-    uint32_t tb = atomicAdd(&cnt[1], ntask);
-    heavy[3 * slot] = k;
-    heavy[3 * slot + 1] = tb;
-    heavy[3 * slot + 2] = ntask;
-    for (uint32_t t = 0; t < ntask; ++t) {
-      uint32_t lo = sa + 1 + t * HEAVY_TASK;
-      tasks[2 * (tb + t)] = lo;
-      tasks[2 * (tb + t) + 1] = lo + HEAVY_TASK < sb ? lo + HEAVY_TASK : sb;
-    }
-    return;
-  }
-  // One addition site: a G2 addition is over 100 KB of code.
-  using O = LOps<F>;
-  typename O::P acc = O::load(plast, sa);
-  for (uint32_t t = sa + 1; t <= sb; ++t) acc = O::add(acc, O::load(pfirst, t));
-  O::store(buckets, k, acc);
-}
-
-// Merged windows: every bucket holds many entries and spans many segments (11-32 at the
-// 1.1M-constraint size), so a bucket gets MERGE_LANES lanes: each sums every MERGE_LANES-th of
-// the bucket's segment pieces (plast of its first segment, pfirst of the rest), then the lanes
-// of a bucket add up through LDS. 256-lane workgroups take 256 / MERGE_LANES buckets. A bucket
-// past WIDE_SPAN segments (the ones of a boolean witness pile into one; a skewed witness's
-// small values would make more) is handed to the heavy path instead, as k_merge does, so no
-// lane folds more than WIDE_SPAN / MERGE_LANES pieces in a row. Four lanes measured best
-// inside the prove (the GPU is full there, so the tree's extra additions cost more than the
-// shorter chains save): 16 lanes 73, 8 lanes 76, 4 lanes 78, 2 lanes 77 proofs/s at the
-// 1.1M-constraint size.
-static constexpr int MERGE_LANES = 4;
-static constexpr uint32_t WIDE_SPAN = 64;
-
-template <class F>
-__global__ void __launch_bounds__(256) k_merge_wide(const uint32_t* offset, uint32_t K,
-                                                    uint4* buckets, const uint4* pfirst,
-                                                    const uint4* plast, uint32_t* cnt,
-                                                    uint32_t* heavy, uint32_t* tasks,
-                                                    uint32_t seg) {
-  using O = LOps<F>;
-  __shared__ typename O::P sh[256];
-  const uint32_t lane = threadIdx.x % MERGE_LANES;
-  const uint32_t k = blockIdx.x * (256 / MERGE_LANES) + threadIdx.x / MERGE_LANES;
-  typename O::P acc = O::inf();
-  bool store = false;  // the bucket's sum is merged here
-  uint32_t s = 0, e = 0;
-  if (k < K) {
-    s = offset[k];
-    e = offset[k + 1];
-    if (s != e) {
-      const uint32_t sa = s / seg, sb = (e - 1) / seg;
-      if (sb - sa > WIDE_SPAN) {
-        if (lane == 0) {
-          uint32_t interior = sb - sa - 1;
-          uint32_t ntask = (interior + HEAVY_TASK - 1) / HEAVY_TASK;
-          uint32_t slot = atomicAdd(&cnt[0], 1u);
-          uint32_t tb = atomicAdd(&cnt[1], ntask);
-          heavy[3 * slot] = k;
-          heavy[3 * slot + 1] = tb;
-          heavy[3 * slot + 2] = ntask;
-          for (uint32_t t = 0; t < ntask; ++t) {
-            uint32_t lo = sa + 1 + t * HEAVY_TASK;
-            tasks[2 * (tb + t)] = lo;
-            tasks[2 * (tb + t) + 1] = lo + HEAVY_TASK < sb ? lo + HEAVY_TASK : sb;
-          }
-        }
-      } else if (sa != sb) {
-        store = true;
-        for (uint32_t t = sa + lane; t <= sb; t += MERGE_LANES)
-          acc = O::add(acc, O::load(t == sa ? plast : pfirst, t));
-      }
-    }
-  }
-  sh[threadIdx.x] = acc;
-  for (int off = MERGE_LANES / 2; off > 0; off >>= 1) {
-    __syncthreads();
-    if (lane < (uint32_t)off) sh[threadIdx.x] = O::add(sh[threadIdx.x], sh[threadIdx.x + off]);
-  }
-  __syncthreads();
-  if (k < K && lane == 0) {
-    if (s == e) st_xyzz(buckets, k, xyzz_inf<F>());
-    else if (store) O::store(buckets, k, sh[threadIdx.x]);
-  }
-}
+// Interior segments per heavy-bucket task (kernels_msm_tail.hip).
+static constexpr uint32_t HEAVY_TASK = 256;
 
 // Sum of BLOCK per-thread values in LDS, left in sh[0].
 template <class Ops, int BLOCK>
@@ -688,52 +547,6 @@ __device__ __forceinline__ void block_tree(typename Ops::P* sh) {
     if ((int)threadIdx.x < off) sh[threadIdx.x] = Ops::add(sh[threadIdx.x], sh[threadIdx.x + off]);
   }
   __syncthreads();
-}
-
-// Level 1: each task's interior segment partials (one per thread) summed by an LDS tree.
-template <class F, int BLOCK>
-__global__ void __launch_bounds__(BLOCK) k_heavy_tasks(const uint32_t* cnt, const uint32_t* tasks,
-                                                       const uint4* pfirst, uint4* task_sum) {
-  static_assert(BLOCK == HEAVY_TASK, "one segment partial per thread");
-  using O = LOps<F>;
-  __shared__ typename O::P sh[BLOCK];
-  uint32_t nt = cnt[1];
-  for (uint32_t t = blockIdx.x; t < nt; t += gridDim.x) {
-    uint32_t lo = tasks[2 * t], hi = tasks[2 * t + 1];
-    uint32_t seg = lo + threadIdx.x;
-    sh[threadIdx.x] = seg < hi ? O::load(pfirst, seg) : O::inf();
-    block_tree<O, BLOCK>(sh);
-    if (threadIdx.x == 0) O::store(task_sum, t, sh[0]);
-    __syncthreads();
-  }
-}
-
-// Level 2: a heavy bucket's task sums and its two end pieces (item nt: plast of the first
-// segment, nt + 1: pfirst of the last), strided over the block, then a tree.
-template <class F, int BLOCK>
-__global__ void __launch_bounds__(BLOCK) k_heavy_finish(const uint32_t* offset,
-                                                        const uint32_t* cnt,
-                                                        const uint32_t* heavy,
-                                                        const uint4* task_sum, uint4* buckets,
-                                                        const uint4* pfirst, const uint4* plast,
-                                                        uint32_t seg) {
-  using O = LOps<F>;
-  __shared__ typename O::P sh[BLOCK];
-  uint32_t nh = cnt[0];
-  for (uint32_t h = blockIdx.x; h < nh; h += gridDim.x) {
-    uint32_t k = heavy[3 * h], tb = heavy[3 * h + 1], nt = heavy[3 * h + 2];
-    uint32_t sa = offset[k] / seg, sb = (offset[k + 1] - 1) / seg;
-    typename O::P acc = O::inf();
-    for (uint32_t t = threadIdx.x; t < nt + 2; t += BLOCK) {
-      const uint4* src = t < nt ? task_sum : (t == nt ? plast : pfirst);
-      const size_t i = t < nt ? (size_t)tb + t : (t == nt ? sa : sb);
-      acc = O::add(acc, O::load(src, i));
-    }
-    sh[threadIdx.x] = acc;
-    block_tree<O, BLOCK>(sh);
-    if (threadIdx.x == 0) O::store(buckets, k, sh[0]);
-    __syncthreads();
-  }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -751,7 +564,7 @@ __global__ void __launch_bounds__(BLOCK) k_heavy_finish(const uint32_t* offset,
 // buckets: 8192 groups) costs two short trees rather than one long strided chain. Every
 // chain is short; the doublings of the bit weights happen once, in the host's Horner pass
 // over all windows.
-template <class F, class Ops = LOps<F>>
+template <class F, class Ops>
 __global__ void __launch_bounds__(128) k_reduce_groups(const uint4* buckets, uint32_t nb,
                                                        int W, uint32_t B, uint4* T,
                                                        uint4* U) {
@@ -770,7 +583,7 @@ __global__ void __launch_bounds__(128) k_reduce_groups(const uint4* buckets, uin
 
 // Workgroup x = ((w rows + r) S + slice); writes out[x] (the host's XYZZ when S = 1, else a
 // slice sum in the policy's form for k_reduce_slices).
-template <class F, int BLOCK, class Ops = LOps<F>>
+template <class F, int BLOCK, class Ops>
 __global__ void __launch_bounds__(BLOCK) k_reduce_rows(const uint4* T, const uint4* U,
                                                        uint32_t G, uint32_t rows, uint32_t S,
                                                        uint4* out) {
@@ -797,7 +610,7 @@ __global__ void __launch_bounds__(BLOCK) k_reduce_rows(const uint4* T, const uin
 }
 
 // Row x = w rows + r: out[x] = sum of parts[x S .. x S + S), in the host's XYZZ.
-template <class F, int BLOCK, class Ops = LOps<F>>
+template <class F, int BLOCK, class Ops>
 __global__ void __launch_bounds__(BLOCK) k_reduce_slices(const uint4* parts, uint32_t S,
                                                          uint4* out) {
   __shared__ typename Ops::P sh[BLOCK];
@@ -819,10 +632,10 @@ inline int ilog2_u32(uint32_t x) {
   return l;
 }
 
-// Slices per row of G groups over `sets` bucket sets: rows hold G or G / 2 items, at least
-// 512 and 256 per slice, and no more than 256 workgroups of four waves (one wave per SIMD):
-// past that, waves share SIMDs and every tree level slows by as much as slicing saves. In
-// practice only a single bucket set (merged windows) is sliced.
+// Slices per row of G groups over `sets` bucket sets (constant work: one lane per point): rows
+// hold G or G / 2 items, at least 512 and 256 per slice, and no more than 256 workgroups of four
+// waves (one wave per SIMD): past that, waves share SIMDs and every tree level slows by as much
+// as slicing saves. In practice only a single bucket set (merged windows) is sliced.
 // Past 8192 groups (bucket sets of 2^15 and more: widths above 16) a row is cut into slices of
 // about 2048 groups, up to 256 per row, so that the row sums run across the device instead of
 // in a few long chains.
@@ -837,10 +650,23 @@ inline uint32_t reduce_slices(uint32_t G, uint32_t sets) {
   return S;
 }
 
+// The same where a point takes `lanes` lanes (k_tail_rows: 256 / lanes points per workgroup). A
+// slice costs its chain of additions and a tree of log2(points): with at least two items per
+// point while the device has room (512 workgroups), eight beyond.
+inline uint32_t tail_slices(uint32_t G, uint32_t sets, uint32_t lanes) {
+  const uint32_t rows = 1 + (uint32_t)ilog2_u32(G), points = 256 / lanes;
+  uint32_t S = 1;
+  for (;;) {
+    const uint64_t blocks = (uint64_t)2 * S * rows * sets;
+    if (S >= 256 || 2 * S > G / 2 || 2 * S * (blocks <= 512 ? 2 : 8) * points > G) return S;
+    S *= 2;
+  }
+}
+
 // Scratch of one accumulation (one base vector over one sorted entry list): buckets, the
 // segment end partials, heavy-bucket bookkeeping, task sums, reduction groups, counters.
 struct AccumLayout {
-  size_t buckets, pfirst, plast, heavy, tasks, task_sum, gT, gU, parts, cnt;
+  size_t buckets, pfirst, plast, heavy, tasks, task_sum, gT, gU, cnt;
   size_t fold0, frows0, fold1, frows1;  // constant work: the fold's two levels of slots
   size_t total;
 };
@@ -853,7 +679,7 @@ inline AccumLayout accum_layout(const MsmPlan& p, size_t pt) {
   size_t K = (size_t)msm_bucket_sets(p) * p.nb;
   const uint32_t seg = accum_seg(p, pt);
   size_t nseg = (p.max_entries + seg - 1) / seg;
-  size_t max_heavy = nseg / HEAVY_SPAN + 2;
+  size_t max_heavy = nseg / MERGE_SPAN + 2;
   size_t max_tasks = nseg / HEAVY_TASK + max_heavy + 2;
   uint32_t B = reduce_group_size(p);
   size_t G = p.nb / B;
@@ -872,8 +698,6 @@ inline AccumLayout accum_layout(const MsmPlan& p, size_t pt) {
   L.task_sum = take(pt * max_tasks);
   L.gT = take(pt * G * msm_bucket_sets(p));
   L.gU = take(pt * G * msm_bucket_sets(p));
-  const uint32_t S = reduce_slices((uint32_t)G, (uint32_t)msm_bucket_sets(p));
-  L.parts = take(S > 1 ? pt * S * (1 + ilog2_u32((uint32_t)G)) * msm_bucket_sets(p) : 0);
   L.cnt = take(16);
   L.fold0 = take(p.constant ? pt * fold_slots0(nseg) : 0);
   L.frows0 = take(p.constant ? 4 * fold_slots0(nseg) : 0);
@@ -889,7 +713,11 @@ inline size_t msm_accum_scratch_bytes_impl(const MsmPlan& p, int group) {
 
 // Pointers into one accumulation's scratch.
 struct AccumPtrs {
-  uint4 *buckets, *pfirst, *plast, *task_sum, *gT, *gU, *parts;
+  uint4 *buckets, *pfirst, *plast, *task_sum, *gT, *gU;
+  // The reduction's slice sums: S per row, in the segment partials' place (no longer needed by
+  // then), so S is cut to what they hold.
+  uint4* parts;
+  uint32_t S;
   uint32_t *heavy, *tasks, *cnt;
   uint4 *fold0, *fold1;
   uint32_t *frows0, *frows1;
@@ -897,13 +725,13 @@ struct AccumPtrs {
   size_t nseg;
 };
 
-// Launchers of the merge and reduction kernels over field F. The G1 ones are defined here;
+// Launchers of the constant-work fold and reduction over field F. The G1 ones are defined here;
 // the G2 ones (F = Fm2i, products expanded in place so the latency-bound tail does not spill)
 // live in kernels_msm_g2_tail.hip and kernels_msm_g2_reduce.hip, so the slow G2 kernels
 // compile in parallel translation units.
 template <class F>
-struct Tail {
-  static void merge(const MsmPlan& p, const AccumPtrs& a, hipStream_t s);
+struct ConstTail {
+  static void fold(const AccumPtrs& a, hipStream_t s);
   static void reduce(const MsmPlan& p, const AccumPtrs& a, uint32_t B, void* window_out,
                      hipStream_t s);
 };
@@ -935,38 +763,6 @@ inline void tail_fold_const(const AccumPtrs& a, hipStream_t s) {
   G16_LAUNCH_CHECK("msm fold scan (constant work)");
 }
 
-template <class F>
-inline void tail_merge_impl(const MsmPlan& p, const AccumPtrs& a, hipStream_t s) {
-  if (p.constant) {
-    tail_fold_const<F>(a, s);
-    return;
-  }
-  size_t K = (size_t)msm_bucket_sets(p) * p.nb;
-  hipLaunchKernelGGL(k_clear_cnt<0>, dim3(1), dim3(64), 0, s, a.cnt);
-  G16_LAUNCH_CHECK("msm clear counters");
-  // Merged windows give a bucket many segments in a large MSM (11-32 at the 1.1M-constraint
-  // size: MERGE_LANES lanes each); a wave of small proofs gives most buckets one segment or
-  // none, where lanes that mostly exit at once only cost launches: one thread per bucket then.
-  const size_t avg_segs = p.max_entries / ((size_t)a.seg * (K ? K : 1));
-  if (p.merged && avg_segs >= 4) {
-    constexpr unsigned per_block = 256 / MERGE_LANES;
-    hipLaunchKernelGGL(k_merge_wide<F>, dim3((unsigned)((K + per_block - 1) / per_block)),
-                       dim3(256), 0, s, p.offset, (uint32_t)K, a.buckets, a.pfirst, a.plast,
-                       a.cnt, a.heavy, a.tasks, a.seg);
-    G16_LAUNCH_CHECK("msm merge (wide)");
-  } else {
-    hipLaunchKernelGGL(k_merge<F>, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s, p.offset,
-                       (uint32_t)K, a.buckets, a.pfirst, a.plast, a.cnt, a.heavy, a.tasks, a.seg);
-    G16_LAUNCH_CHECK("msm merge");
-  }
-  hipLaunchKernelGGL((k_heavy_tasks<F, HEAVY_TASK>), dim3(1024), dim3(HEAVY_TASK), 0, s, a.cnt,
-                     a.tasks, a.pfirst, a.task_sum);
-  G16_LAUNCH_CHECK("msm heavy tasks");
-  hipLaunchKernelGGL((k_heavy_finish<F, 64>), dim3(256), dim3(64), 0, s, p.offset, a.cnt, a.heavy,
-                     a.task_sum, a.buckets, a.pfirst, a.plast, a.seg);
-  G16_LAUNCH_CHECK("msm heavy finish");
-}
-
 template <class F, class Ops>
 inline void tail_reduce_ops(const MsmPlan& p, const AccumPtrs& a, uint32_t B, void* window_out,
                             hipStream_t s) {
@@ -977,7 +773,7 @@ inline void tail_reduce_ops(const MsmPlan& p, const AccumPtrs& a, uint32_t B, vo
   hipLaunchKernelGGL((k_reduce_groups<F, Ops>), dim3((nthreads + 127) / 128), dim3(128), 0, s,
                      a.buckets, p.nb, sets, B, a.gT, a.gU);
   G16_LAUNCH_CHECK("msm reduce groups");
-  const uint32_t S = reduce_slices(G, (uint32_t)sets);
+  const uint32_t S = a.S;
   uint4* wout = static_cast<uint4*>(window_out);
   hipLaunchKernelGGL((k_reduce_rows<F, 256, Ops>), dim3((unsigned)sets * rows * S), dim3(256), 0,
                      s, a.gT, a.gU, G, rows, S, S > 1 ? a.parts : wout);
@@ -987,14 +783,6 @@ inline void tail_reduce_ops(const MsmPlan& p, const AccumPtrs& a, uint32_t B, vo
                        a.parts, S, wout);
     G16_LAUNCH_CHECK("msm reduce slices");
   }
-}
-
-// Constant-work plans reduce their projective buckets with the complete formulas.
-template <class F>
-inline void tail_reduce_impl(const MsmPlan& p, const AccumPtrs& a, uint32_t B, void* window_out,
-                             hipStream_t s) {
-  if (p.constant) tail_reduce_ops<F, COps<F>>(p, a, B, window_out, s);
-  else tail_reduce_ops<F, LOps<F>>(p, a, B, window_out, s);
 }
 
 // F: the coordinate field in the MSM's Montgomery form R' = 2^261 (Fm, or Fm2i for G2); the
@@ -1013,7 +801,7 @@ inline AccumPtrs accum_ptrs(const MsmPlan& p, void* scratch) {
   a.task_sum = reinterpret_cast<uint4*>(q + L.task_sum);
   a.gT = reinterpret_cast<uint4*>(q + L.gT);
   a.gU = reinterpret_cast<uint4*>(q + L.gU);
-  a.parts = reinterpret_cast<uint4*>(q + L.parts);
+  a.parts = a.pfirst;
   a.cnt = reinterpret_cast<uint32_t*>(q + L.cnt);
   a.fold0 = reinterpret_cast<uint4*>(q + L.fold0);
   a.frows0 = reinterpret_cast<uint32_t*>(q + L.frows0);
@@ -1021,72 +809,102 @@ inline AccumPtrs accum_ptrs(const MsmPlan& p, void* scratch) {
   a.frows1 = reinterpret_cast<uint32_t*>(q + L.frows1);
   a.seg = accum_seg(p, PT);
   a.nseg = (p.max_entries + a.seg - 1) / a.seg;
+  const uint32_t G = p.nb / reduce_group_size(p), sets = (uint32_t)msm_bucket_sets(p);
+  const uint64_t rows = (uint64_t)(1 + ilog2_u32(G)) * sets;
+  a.S = p.constant ? reduce_slices(G, sets) : tail_slices(G, sets, PT == 128 ? 4 : 8);
+  while (a.S > 1 && a.S * rows > 2 * (a.nseg + 1)) a.S /= 2;
   return a;
 }
 
-// The G1 bucket accumulations of up to QUEUE_JOBS MSMs (each: plan, bases, scratch) as one
-// persistent launch, then each job's merges and reduction into its window_out. `counter` is a
-// device word the launch takes tiles from (cleared here by a kernel first).
-template <class F>
-inline void accumulate_queue_impl(const MsmPlan* const* plans, const void* const* bases,
-                                  void* const* scratch, void* const* window_out, int n,
-                                  uint32_t* counter, int grid, hipStream_t s) {
-  if (n < 1 || n > QUEUE_JOBS) throw ArgError{"accumulation queue of " + std::to_string(n) + " jobs"};
-  for (int d = 0; d < n; ++d)
-    if (plans[d]->constant) throw ArgError{"constant-work MSMs do not go through the queue"};
-  AccQueue q{};
-  q.n = n;
-  q.start[0] = 0;
-  AccumPtrs a[QUEUE_JOBS];
-  for (int d = 0; d < n; ++d) {
-    a[d] = accum_ptrs<F>(*plans[d], scratch[d]);
-    const size_t nseg = (plans[d]->max_entries + a[d].seg - 1) / a[d].seg;
-    q.job[d] = AccQueueJob{plans[d]->ent, plans[d]->total, static_cast<const uint4*>(bases[d]),
-                           a[d].buckets, a[d].pfirst, a[d].plast, nseg, a[d].seg};
-    const size_t tiles = (nseg + QUEUE_TILE - 1) / QUEUE_TILE;
-    if (q.start[d] + tiles >= (1ull << 32)) throw ArgError{"accumulation queue too long"};
-    q.start[d + 1] = q.start[d] + (uint32_t)tiles;
-  }
-  hipLaunchKernelGGL(k_clear_cnt<0>, dim3(1), dim3(64), 0, s, counter);
-  G16_LAUNCH_CHECK("msm queue counter");
-  if (q.start[n]) {
-    const unsigned blocks = (unsigned)std::min<size_t>((size_t)grid, q.start[n]);
-    hipLaunchKernelGGL(k_accumulate_queue<F>, dim3(blocks), dim3(QUEUE_TILE), 0, s, q, counter);
-    G16_LAUNCH_CHECK("msm accumulate (queue)");
-  }
-  for (int d = 0; d < n; ++d) {
-    Tail<F>::merge(*plans[d], a[d], s);
-    Tail<F>::reduce(*plans[d], a[d], reduce_group_size(*plans[d]), window_out[d], s);
-  }
+inline TailJob tail_job(const MsmPlan& p, const AccumPtrs& a, void* window_out) {
+  TailJob j{};
+  j.offset = p.offset;
+  j.sets = (uint32_t)msm_bucket_sets(p);
+  j.K = j.sets * p.nb;
+  j.seg = a.seg;
+  j.B = reduce_group_size(p);
+  j.G = p.nb / j.B;
+  j.rows = 1 + (uint32_t)ilog2_u32(j.G);
+  j.S = a.S;
+  j.avg_pieces = (uint32_t)(p.max_entries / ((size_t)a.seg * j.K));
+  j.buckets = a.buckets;
+  j.pfirst = a.pfirst;
+  j.plast = a.plast;
+  j.task_sum = a.task_sum;
+  j.gT = a.gT;
+  j.gU = a.gU;
+  j.parts = a.parts;
+  j.out = static_cast<uint4*>(window_out);
+  j.heavy = a.heavy;
+  j.tasks = a.tasks;
+  j.cnt = a.cnt;
+  return j;
 }
 
+// The bucket accumulations of up to QUEUE_JOBS variable-work MSMs of one group (each: plan,
+// bases, scratch), then their merges and reductions into window_out, all jobs in each launch.
+// With `counter` (a device word, cleared here by a kernel first) the accumulation is one
+// persistent launch of `grid` workgroups that take tiles of segments from it; without, the jobs
+// have the same entries and run side by side.
 template <class F>
-inline void accumulate_impl(const MsmPlan& p, const void* bases, void* scratch, void* window_out,
-                            hipStream_t s, hipEvent_t* ev) {
+inline void accumulate_jobs_impl(int group, const MsmPlan* const* plans, const void* const* bases,
+                                 void* const* scratch, void* const* window_out, int n,
+                                 uint32_t* counter, int grid, hipStream_t s, hipEvent_t* ev) {
+  if (n < 1 || n > QUEUE_JOBS) throw ArgError{"accumulation of " + std::to_string(n) + " jobs"};
+  AccQueue q{};
+  TailJobs t{};
+  q.n = t.n = n;
+  for (int d = 0; d < n; ++d) {
+    if (plans[d]->constant) throw ArgError{"constant-work MSMs accumulate on their own"};
+    const AccumPtrs a = accum_ptrs<F>(*plans[d], scratch[d]);
+    q.job[d] = AccQueueJob{plans[d]->ent, plans[d]->total, static_cast<const uint4*>(bases[d]),
+                           a.buckets, a.pfirst, a.plast, a.cnt, a.nseg, a.seg};
+    const size_t tiles = (a.nseg + QUEUE_TILE - 1) / QUEUE_TILE;
+    if (q.start[d] + tiles >= (1ull << 32)) throw ArgError{"accumulation queue too long"};
+    q.start[d + 1] = q.start[d] + (uint32_t)tiles;
+    t.job[d] = tail_job(*plans[d], a, window_out[d]);
+  }
+  if (ev) G16_CHECK(hipEventRecord(ev[0], s));
+  if (counter) {
+    hipLaunchKernelGGL(k_clear_cnt<0>, dim3(1), dim3(64), 0, s, counter);
+    G16_LAUNCH_CHECK("msm queue counter");
+    const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>((size_t)grid, q.start[n]));
+    hipLaunchKernelGGL(k_accumulate_queue<F>, dim3(blocks), dim3(QUEUE_TILE), 0, s, q, counter);
+  } else {
+    uint64_t nseg = 1;  // at least one workgroup: it clears the counters
+    for (int d = 0; d < n; ++d) nseg = std::max(nseg, q.job[d].nseg);
+    hipLaunchKernelGGL(k_accumulate<F>, dim3((unsigned)((nseg + 127) / 128), n), dim3(128), 0, s, q);
+  }
+  G16_LAUNCH_CHECK("msm accumulate");
+  if (ev) G16_CHECK(hipEventRecord(ev[1], s));
+  tail_merge_jobs(group, t, s);
+  if (ev) G16_CHECK(hipEventRecord(ev[2], s));
+  tail_reduce_jobs(group, t, s);
+  if (ev) G16_CHECK(hipEventRecord(ev[3], s));
+}
+
+// One constant-work MSM.
+template <class F>
+inline void accumulate_const_impl(const MsmPlan& p, const void* bases, void* scratch,
+                                  void* window_out, hipStream_t s, hipEvent_t* ev) {
   const AccumPtrs a = accum_ptrs<F>(p, scratch);
   const uint32_t B = reduce_group_size(p);
   auto bp = static_cast<const uint4*>(bases);
   const unsigned grid = (unsigned)((a.nseg + 127) / 128);
+  const size_t K = (size_t)msm_bucket_sets(p) * p.nb;
   if (ev) G16_CHECK(hipEventRecord(ev[0], s));
-  if (p.constant) {
-    const size_t K = (size_t)msm_bucket_sets(p) * p.nb;
-    hipLaunchKernelGGL(k_fill_proj_inf<F>, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s,
-                       a.buckets, K);
-    G16_LAUNCH_CHECK("msm buckets (constant work)");
-    if (a.nseg) {
-      hipLaunchKernelGGL(k_accumulate_const<F>, dim3(grid), dim3(128), 0, s, p.ent, p.total,
-                         a.nseg, a.seg, bp, a.buckets, a.fold0, a.frows0);
-      G16_LAUNCH_CHECK("msm accumulate (constant work)");
-    }
-  } else if (a.nseg) {
-    hipLaunchKernelGGL(k_accumulate<F>, dim3(grid), dim3(128), 0, s, p.ent, p.total, a.nseg,
-                       a.seg, bp, a.buckets, a.pfirst, a.plast);
-    G16_LAUNCH_CHECK("msm accumulate");
+  hipLaunchKernelGGL(k_fill_proj_inf<F>, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s,
+                     a.buckets, K);
+  G16_LAUNCH_CHECK("msm buckets (constant work)");
+  if (a.nseg) {
+    hipLaunchKernelGGL(k_accumulate_const<F>, dim3(grid), dim3(128), 0, s, p.ent, p.total,
+                       a.nseg, a.seg, bp, a.buckets, a.fold0, a.frows0);
+    G16_LAUNCH_CHECK("msm accumulate (constant work)");
   }
   if (ev) G16_CHECK(hipEventRecord(ev[1], s));
-  Tail<F>::merge(p, a, s);
+  ConstTail<F>::fold(a, s);
   if (ev) G16_CHECK(hipEventRecord(ev[2], s));
-  Tail<F>::reduce(p, a, B, window_out, s);
+  ConstTail<F>::reduce(p, a, B, window_out, s);
   if (ev) G16_CHECK(hipEventRecord(ev[3], s));
 }
 
