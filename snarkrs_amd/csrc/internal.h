@@ -104,6 +104,8 @@ struct MsmPlan {
   // discarded, and the accumulation computes its addition and keeps the old sum by a select.
   // Entry values are then index << 2 | discard << 1 | sign (index < 2^30).
   bool constant = false;
+  // Entries per accumulation segment, for G1 and G2 bases (msm_segments).
+  uint32_t seg[2] = {0, 0};
   // device scratch (owned by the caller)
   uint32_t* offset = nullptr;   // [K + 1] first entry of each bucket (K = sets * nb); [K] = total
   uint32_t* block_sums = nullptr;
@@ -130,8 +132,12 @@ inline MsmPlan msm_vector_view(const MsmPlan& p) {
   return v;
 }
 size_t msm_sort_scratch_bytes(uint32_t n, int c, uint32_t batch = 1);
+// `at_once`: entries the device works on together in the launches this plan is for (0: as many
+// as fill it). Fewer than fill it are cut into shorter segments, which take more scratch
+// (msm_accum_scratch_bytes); a caller short of memory passes 0. A wave passes the same count for
+// its cap and every smaller number of proofs, so that all fit the scratch sized for the cap.
 void msm_plan_bind(MsmPlan& p, void* scratch, uint32_t n, int c, bool merged = false,
-                   bool constant = false, uint32_t batch = 1);
+                   bool constant = false, uint32_t batch = 1, size_t at_once = 0);
 // Window tables for merged MSMs: `table` holds n affine bases (MSM form) at [0, n); fills
 // entries w n + i = 2^(c w) P_i for 1 <= w < windows. group 1 = G1, 2 = G2.
 void msm_window_tables(int group, void* table, size_t n, int c, int windows, hipStream_t s);

@@ -640,8 +640,31 @@ size_t msm_sort_scratch_bytes(uint32_t n, int c, uint32_t batch) {
          align_up(4 * E) + align_up(16);
 }
 
+// Entries per segment: 32, and 40 for a G1 MSM over per-window buckets, whose merges are one or
+// two additions per bucket, so fewer and longer segments pay there (the 2^20 G1 MSM: 2.13
+// against 2.25-2.30 ms; G2 and the prove's merged MSMs were slower).
+// Constant-work MSMs over window tables (the prove's) take 64: their accumulation runs the
+// same number of rounds of waves at the prove's sizes and the fold starts from half the slots
+// (47.8-47.9 against 47.4-47.5 proofs/s).
+// A segment is a chain of dependent additions on one lane, 5 us each in G1 and 13 in G2 while
+// the device is not full, so a variable-work MSM whose segments would not fill it halves them
+// until they do, down to 8 (G1 over per-window buckets: 10). MI355X: G1 MSM of 4099 points
+// 562 -> 405 us, G2 of 1021 points 956 -> 622, 22k-constraint prove 1035 -> 850, 65k resident
+// 1616 -> 1530. 131072 lanes for G1 gave 868 and 1576 on the last two; 32768 for G2 966 and
+// 1652, 131072 the same as 65536; segments of 4 gained 3 % on the two MSMs and lost as much on
+// the proofs.
+static constexpr size_t SEG_LANES[2] = {262144, 65536};  // G1: four waves per SIMD; G2: one
+
+static uint32_t segment_length(const MsmPlan& p, int g, size_t at_once) {
+  if (p.constant && p.merged) return 64u;
+  uint32_t seg = !p.merged && g == 0 ? 40u : 32u;
+  if (p.constant || !at_once) return seg;
+  while (seg >= 16 && at_once / seg < SEG_LANES[g]) seg /= 2;
+  return seg;
+}
+
 void msm_plan_bind(MsmPlan& p, void* scratch, uint32_t n, int c, bool merged, bool constant,
-                   uint32_t batch) {
+                   uint32_t batch, size_t at_once) {
   if (c < 2 || c > MSM_MAX_C) throw ArgError{"MSM window width must be in [2, 20]"};
   if (batch == 0) throw ArgError{"MSM batch of zero vectors"};
   p.merged = merged;
@@ -665,6 +688,7 @@ void msm_plan_bind(MsmPlan& p, void* scratch, uint32_t n, int c, bool merged, bo
   p.q = g.q;
   p.groups = g.groups;
   p.max_slices = g.max_slices;
+  for (int g = 0; g < 2; ++g) p.seg[g] = segment_length(p, g, at_once);
   const size_t K = (size_t)msm_bucket_sets(p) * p.nb;
   char* q = static_cast<char*>(scratch);
   auto take = [&](size_t bytes) {

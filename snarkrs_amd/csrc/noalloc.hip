@@ -49,14 +49,19 @@ extern "C" g16hip_status g16hip_msm_device_noalloc(g16hip_device* d, int group, 
     set_device(d);
     char* base = static_cast<char*>(device_scratch(d));
     const int w = msm_width((uint32_t)n, c);
-    const MsmScratchSizes z = msm_scratch_sizes(group, (uint32_t)n, w, d->constant_work);
+    bool lean = false;
+    MsmScratchSizes z = msm_scratch_sizes(group, (uint32_t)n, w, d->constant_work, lean);
+    if (z.total() > G16HIP_NOALLOC_SCRATCH_BYTES) {
+      lean = true;
+      z = msm_scratch_sizes(group, (uint32_t)n, w, d->constant_work, lean);
+    }
     if (z.total() > G16HIP_NOALLOC_SCRATCH_BYTES)
       throw StatusError{G16HIP_DEVICE_MEMORY,
                         "an MSM of " + std::to_string(n) + " points at window width " +
                             std::to_string(w) + " needs " + std::to_string(z.total()) +
                             " bytes of scratch and the static scratch holds " +
                             std::to_string((size_t)G16HIP_NOALLOC_SCRATCH_BYTES)};
-    msm_device_on_scratch(d, group, bases, scalars, (uint32_t)n, w,
+    msm_device_on_scratch(d, group, bases, scalars, (uint32_t)n, w, lean,
                           MsmScratch{base, base + z.sort, base + z.sort + z.accum}, out);
     return G16HIP_OK;
   });

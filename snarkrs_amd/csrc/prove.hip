@@ -35,6 +35,10 @@ struct Slot {
   hipEvent_t mev[5][4] = {};   // per MSM: before accumulation, after it, after merges, after reduction
   DevBuf witness, abc, hbuf, sort_w, sort_h, accum_w1, accum_w2, accum_h;
   MsmPlan plan_w, plan_h;
+  // Short segments where few entries would not fill the device, and scratch for A, B1 and L
+  // side by side (accum_w1 holds three), so that they share every launch; or the least scratch,
+  // one after the other, where the device budget holds no more.
+  bool fast = false;
   // Pinned, device-mapped host memory: the reduction kernels write each MSM's rows straight
   // here (no copy on the stream, which would wait for CUs behind other streams' kernels).
   uint8_t* host_wout = nullptr;
@@ -48,6 +52,10 @@ struct Slot {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   size_t bytes = 0;
+
+  bool together() const {  // accum_w1 holds three MSMs' scratch
+    return fast && accum_w1.bytes >= 3 * msm_accum_scratch_bytes(plan_w, 1);
+  }
 
   ~Slot() {
     for (hipStream_t st : {stream, side[0], side[1]})
@@ -79,6 +87,7 @@ struct Slot {
 // device runs wave i + 1.
 struct Wave {
   uint32_t cap = 0;
+  bool fast = false;  // short segments where the cap's entries would not fill the device
   hipStream_t stream = nullptr;
   hipEvent_t done[2] = {};
   DevBuf witness, abc, hbuf, sort_w, sort_h;
@@ -191,12 +200,14 @@ static void validate_key(const g16hip_key* k) {
 struct KeyPlan {
   int cw = 0, ch = 0;
   bool merged = false;
-  size_t key_bytes = 0, slot_bytes = 0;
+  size_t key_bytes = 0, slot_bytes = 0;  // slot_bytes: the least scratch a slot works with
+  size_t fast_slot_bytes = 0;            // with short segments and shared launches
+  bool fast = false;                     // the budget holds those
   size_t total() const { return key_bytes + slot_bytes; }
 };
 
 static size_t slot_bytes_for(uint32_t nv, uint32_t n, uint32_t nh, int cw, int ch, bool merged,
-                             bool constant);
+                             bool constant, bool fast);
 
 static KeyPlan plan_key(const g16hip_key* k, bool merged, bool constant) {
   const size_t n = k->domain_size, nv = k->n_vars, nh = k->h_basis == 1 ? n - 1 : n;
@@ -226,7 +237,9 @@ static KeyPlan plan_key(const g16hip_key* k, bool merged, bool constant) {
        (k->h_basis == 1 ? dev_pages(32 * n) : 0) + dev_pages(32 * (n / 2 ? n / 2 : 1));
   P.key_bytes = b;
   P.slot_bytes = slot_bytes_for((uint32_t)nv, (uint32_t)n, (uint32_t)nh, P.cw, P.ch, merged,
-                                constant);
+                                constant, false);
+  P.fast_slot_bytes = slot_bytes_for((uint32_t)nv, (uint32_t)n, (uint32_t)nh, P.cw, P.ch, merged,
+                                     constant, true);
   return P;
 }
 
@@ -238,11 +251,15 @@ static KeyPlan choose_plan(const g16hip_device* d, const g16hip_key* k) {
   const char* wt = std::getenv("G16HIP_WINDOW_TABLES");
   if (!(wt && wt[0] == '0')) {
     KeyPlan P = plan_key(k, true, d->constant_work);
-    if (P.total() + (8ull << 30) <= budget) return P;
+    if (P.total() + (8ull << 30) <= budget) {
+      P.fast = P.key_bytes + P.fast_slot_bytes <= budget;
+      return P;
+    }
   }
   KeyPlan P = plan_key(k, false, d->constant_work);
   if (P.total() > budget)
     throw too_big(P.total(), budget, "this key's resident data and one proof's stage scratch");
+  P.fast = P.key_bytes + P.fast_slot_bytes <= budget;
   return P;
 }
 
@@ -349,17 +366,36 @@ static std::unique_ptr<Slot> new_slot() {
   return S;
 }
 
+// A, B1 and L share their launches while their scratch together stays below this: past it one
+// of them fills the device, and its tail runs beside the next one's accumulation.
+static constexpr size_t TOGETHER_BYTES = 256ull << 20;
+
+// A slot's two plans: the witness's (A, B1, L and B2), H's.
+static void slot_plans(MsmPlan& w, MsmPlan& h, void* sort_w, void* sort_h, uint32_t nv,
+                       uint32_t nh, int cw, int ch, bool merged, bool constant, bool fast) {
+  const size_t ew = (size_t)nv * ((255 + cw - 1) / cw), eh = (size_t)nh * ((255 + ch - 1) / ch);
+  msm_plan_bind(w, sort_w, nv, cw, merged, constant, 1, fast ? ew : 0);
+  msm_plan_bind(h, sort_h, nh, ch, merged, constant, 1, fast ? eh : 0);
+}
+
+// Bytes of a slot's G1 witness scratch: one MSM's, or three when they run together.
+static size_t accum_w1_bytes(const MsmPlan& w, bool fast) {
+  const size_t one = (msm_accum_scratch_bytes(w, 1) + 255) & ~(size_t)255;
+  return fast && !w.constant && 3 * one <= TOGETHER_BYTES ? 3 * one : one;
+}
+
 // Per-proof scratch for one slot, sized once so a proof allocates nothing.
-static void size_slot(const g16hip_circuit* C, Slot* S) {
+static void size_slot(const g16hip_circuit* C, Slot* S, bool fast) {
   size_t nv = C->n_vars, n = C->domain;
+  S->fast = fast;
   S->witness.alloc(32 * nv);
   S->abc.alloc(32 * 3 * n);
   S->hbuf.alloc(32 * n);
   S->sort_w.alloc(msm_sort_scratch_bytes((uint32_t)nv, C->cw));
   S->sort_h.alloc(msm_sort_scratch_bytes(C->n_h, C->ch));
-  msm_plan_bind(S->plan_w, S->sort_w.p, (uint32_t)nv, C->cw, C->merged, C->constant);
-  msm_plan_bind(S->plan_h, S->sort_h.p, C->n_h, C->ch, C->merged, C->constant);
-  S->accum_w1.alloc(msm_accum_scratch_bytes(S->plan_w, 1));
+  slot_plans(S->plan_w, S->plan_h, S->sort_w.p, S->sort_h.p, (uint32_t)nv, C->n_h, C->cw, C->ch,
+             C->merged, C->constant, fast);
+  S->accum_w1.alloc(accum_w1_bytes(S->plan_w, fast));
   S->accum_w2.alloc(msm_accum_scratch_bytes(S->plan_w, 2));
   S->accum_h.alloc(msm_accum_scratch_bytes(S->plan_h, 1));
   size_t wbytes = 256 * (4 * msm_out_points(S->plan_w) + msm_out_points(S->plan_h));
@@ -375,27 +411,26 @@ static void size_slot(const g16hip_circuit* C, Slot* S) {
   for (auto b : bufs) S->bytes += b->bytes;
 }
 
-static std::unique_ptr<Slot> make_slot(const g16hip_circuit* C) {
+static std::unique_ptr<Slot> make_slot(const g16hip_circuit* C, bool fast) {
   auto S = new_slot();
-  size_slot(C, S.get());
+  size_slot(C, S.get(), fast);
   return S;
 }
 
 // Device bytes of one slot (what size_slot allocates), rounded up to pages.
 static size_t slot_bytes_for(uint32_t nv, uint32_t n, uint32_t nh, int cw, int ch, bool merged,
-                             bool constant) {
+                             bool constant, bool fast) {
   MsmPlan pw, ph;
   static char anchor;  // the plans are bound only to size their pieces
-  msm_plan_bind(pw, &anchor, nv, cw, merged, constant);
-  msm_plan_bind(ph, &anchor, nh, ch, merged, constant);
+  slot_plans(pw, ph, &anchor, &anchor, nv, nh, cw, ch, merged, constant, fast);
   return dev_pages(32 * (size_t)nv) + dev_pages(32 * 3 * (size_t)n) + dev_pages(32 * (size_t)n) +
          dev_pages(msm_sort_scratch_bytes(nv, cw)) + dev_pages(msm_sort_scratch_bytes(nh, ch)) +
-         dev_pages(msm_accum_scratch_bytes(pw, 1)) + dev_pages(msm_accum_scratch_bytes(pw, 2)) +
+         dev_pages(accum_w1_bytes(pw, fast)) + dev_pages(msm_accum_scratch_bytes(pw, 2)) +
          dev_pages(msm_accum_scratch_bytes(ph, 1));
 }
 
-static size_t slot_bytes_estimate(const g16hip_circuit* C) {
-  return slot_bytes_for(C->n_vars, C->domain, C->n_h, C->cw, C->ch, C->merged, C->constant);
+static size_t slot_bytes_estimate(const g16hip_circuit* C, bool fast) {
+  return slot_bytes_for(C->n_vars, C->domain, C->n_h, C->cw, C->ch, C->merged, C->constant, fast);
 }
 
 static bool try_add_slot(g16hip_circuit* C, size_t reserve);
@@ -616,8 +651,8 @@ static WinLayout win_layout(const Slot* S) {
 }
 
 // Enqueues stages (0-4 if `with_h`) 5-9 on the slot's three streams: side[0] sorts the
-// witness digits once and accumulates A, B1 and L; side[1] accumulates B2 on the same
-// entries; the main stream runs stages 0-4 and then the H sort and MSM. Each MSM's reduction
+// witness digits once and accumulates A, B1 and L (together while they are small); side[1]
+// accumulates B2 on the same entries; the main stream runs stages 0-4 and then the H sort and MSM. Each MSM's reduction
 // rows are written by its kernel into pinned host memory. With `timed`, events bracket every
 // phase (done_ev[k] marks MSM k's rows on the host) and the entry counts are copied out at
 // the end for the kernel statistics; a graph capture passes timed = false.
@@ -650,12 +685,21 @@ static void enqueue_stages(const g16hip_circuit* C, Slot* S, bool with_h, void* 
   msm_accumulate(pw, 2, C->b2_q.p, S->accum_w2.p, wout + L.off[3], s2, mev3);
   rows_done(3, s2);
   G16_CHECK(hipEventRecord(S->sync_ev[3], s2));
-  msm_accumulate(pw, 1, C->a_q.p, S->accum_w1.p, wout + L.off[0], s1, mev0);
-  rows_done(0, s1);
-  msm_accumulate(pw, 1, C->b1_q.p, S->accum_w1.p, wout + L.off[1], s1, mev1);
-  rows_done(1, s1);
-  msm_accumulate(pw, 1, C->l_q.p, S->accum_w1.p, wout + L.off[2], s1, mev2);
-  rows_done(2, s1);
+  const void* g1_bases[3] = {C->a_q.p, C->b1_q.p, C->l_q.p};
+  void* g1_rows[3] = {wout + L.off[0], wout + L.off[1], wout + L.off[2]};
+  if (S->together()) {
+    const size_t each = S->accum_w1.bytes / 3;
+    void* scratch[3];
+    for (int k = 0; k < 3; ++k) scratch[k] = S->accum_w1.as<char>() + k * each;
+    msm_accumulate_g1_together(pw, g1_bases, scratch, g1_rows, 3, s1, mev0);
+    for (int k = 0; k < 3; ++k) rows_done(k, s1);
+  } else {
+    hipEvent_t* mev[3] = {mev0, mev1, mev2};
+    for (int k = 0; k < 3; ++k) {
+      msm_accumulate(pw, 1, g1_bases[k], S->accum_w1.p, g1_rows[k], s1, mev[k]);
+      rows_done(k, s1);
+    }
+  }
   G16_CHECK(hipEventRecord(S->sync_ev[2], s1));
   if (with_h) stages_0_4(C, S, h, timed, rows);
   msm_sort(ph, h, s0);
@@ -744,9 +788,14 @@ static void run_timed(g16hip_circuit* C, Slot* S, bool with_h, void* h, g16hip_m
   if (rows) check_gnark_h(C, S);
   WinLayout L = win_layout(S);
   const uint32_t* totals = reinterpret_cast<const uint32_t*>(S->host_wout + L.totals);
-  for (size_t k = 0; k < kMsmCount; ++k)
-    note_accumulate(C->dev, k == 3 ? 2 : 1, k == 4 ? totals[1] : totals[0],
-                    ev_ms(S->mev[k][0], S->mev[k][1]));
+  // A, B1 and L in one launch have one pair of events.
+  const auto mev = [&](size_t k) { return S->mev[S->together() && k < 3 ? 0 : k]; };
+  for (size_t k = 0; k < kMsmCount; ++k) {
+    if (S->together() && (k == 1 || k == 2)) continue;
+    const uint64_t entries = k == 4 ? totals[1] : totals[0];
+    note_accumulate(C->dev, k == 3 ? 2 : 1, S->together() && k == 0 ? 3 * entries : entries,
+                    ev_ms(mev(k)[0], mev(k)[1]));
+  }
   if (timeline_on()) {
     // Milliseconds from the witness arriving on the device, per stream (the
     // G16_CUDA_MEMORY_TRACE kind of switch, crates/cuda/src/backend.rs:89-93).
@@ -763,8 +812,8 @@ static void run_timed(g16hip_circuit* C, Slot* S, bool with_h, void* h, g16hip_m
                    ev_ms(S->ev[4], S->ev[2]), ev_ms(S->ev[4], S->ev[3]));
     for (size_t k = 0; k < kMsmCount; ++k)
       std::fprintf(stderr, " %s acc %.2f-%.2f merge %.2f reduce %.2f |", names[k],
-                   ev_ms(S->ev[4], S->mev[k][0]), ev_ms(S->ev[4], S->mev[k][1]),
-                   ev_ms(S->ev[4], S->mev[k][2]), ev_ms(S->ev[4], S->mev[k][3]));
+                   ev_ms(S->ev[4], mev(k)[0]), ev_ms(S->ev[4], mev(k)[1]),
+                   ev_ms(S->ev[4], mev(k)[2]), ev_ms(S->ev[4], mev(k)[3]));
     std::fprintf(stderr, " end %.2f\n", ev_ms(S->ev[4], S->ev[5]));
   }
   if (t) {
@@ -924,10 +973,14 @@ struct WavePlans {
   size_t rw = 0, rh = 0;  // reduction rows per proof
 };
 
-static WavePlans wave_plans(const g16hip_circuit* C, void* sort_w, void* sort_h, uint32_t m) {
+// The plans of a wave of m proofs, m <= cap: segments follow the cap's entries, whatever m is.
+static WavePlans wave_plans(const g16hip_circuit* C, void* sort_w, void* sort_h, uint32_t m,
+                            uint32_t cap, bool fast) {
   WavePlans P;
-  msm_plan_bind(P.w, sort_w, C->n_vars, C->cw, C->merged, C->constant, m);
-  msm_plan_bind(P.h, sort_h, C->n_h, C->ch, C->merged, C->constant, m);
+  const size_t ew = (size_t)cap * C->n_vars * ((255 + C->cw - 1) / C->cw);
+  const size_t eh = (size_t)cap * C->n_h * ((255 + C->ch - 1) / C->ch);
+  msm_plan_bind(P.w, sort_w, C->n_vars, C->cw, C->merged, C->constant, m, fast ? ew : 0);
+  msm_plan_bind(P.h, sort_h, C->n_h, C->ch, C->merged, C->constant, m, fast ? eh : 0);
   P.vw = msm_vector_view(P.w);
   P.vh = msm_vector_view(P.h);
   P.rw = msm_out_points(P.vw);
@@ -948,9 +1001,9 @@ static size_t wave_rows_bytes(const WavePlans& P, uint32_t cap) {
   return wave_rows_offset(P, cap, 4, cap);
 }
 
-static size_t wave_bytes_for(const g16hip_circuit* C, uint32_t cap) {
+static size_t wave_bytes_for(const g16hip_circuit* C, uint32_t cap, bool fast) {
   static char anchor;  // bound only to size the pieces
-  const WavePlans P = wave_plans(C, &anchor, &anchor, cap);
+  const WavePlans P = wave_plans(C, &anchor, &anchor, cap, cap, fast);
   const size_t nv = C->n_vars, n = C->domain;
   return dev_pages(32 * nv * cap) + dev_pages(96 * n * cap) + dev_pages(32 * n * cap) +
          dev_pages(msm_sort_scratch_bytes((uint32_t)nv, C->cw, cap)) +
@@ -973,11 +1026,13 @@ static uint32_t wave_cap_of(const g16hip_circuit* C) {
 
 // Builds a wave for cap proofs, refused before allocating when the device budget cannot hold it.
 static std::unique_ptr<Wave> make_wave(g16hip_circuit* C, uint32_t cap) {
-  const size_t need = wave_bytes_for(C, cap);
   const size_t budget = device_budget(C->dev);
+  const bool fast = wave_bytes_for(C, cap, true) <= budget;
+  const size_t need = wave_bytes_for(C, cap, fast);
   if (need > budget) throw too_big(need, budget, "a wave of " + std::to_string(cap) + " proofs");
   auto W = std::make_unique<Wave>();
   W->cap = cap;
+  W->fast = fast;
   G16_CHECK(hipStreamCreateWithFlags(&W->stream, hipStreamNonBlocking));
   for (auto& e : W->done) G16_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   const size_t nv = C->n_vars, n = C->domain;
@@ -986,7 +1041,7 @@ static std::unique_ptr<Wave> make_wave(g16hip_circuit* C, uint32_t cap) {
   W->hbuf.alloc(32 * n * cap);
   W->sort_w.alloc(msm_sort_scratch_bytes((uint32_t)nv, C->cw, cap));
   W->sort_h.alloc(msm_sort_scratch_bytes(C->n_h, C->ch, cap));
-  const WavePlans P = wave_plans(C, W->sort_w.p, W->sort_h.p, cap);
+  const WavePlans P = wave_plans(C, W->sort_w.p, W->sort_h.p, cap, cap, fast);
   for (int j = 0; j < 3; ++j) W->accum_g1[j].alloc(msm_accum_scratch_bytes(P.w, 1));
   W->accum_g1[3].alloc(msm_accum_scratch_bytes(P.h, 1));
   W->accum_w2.alloc(msm_accum_scratch_bytes(P.w, 2));
@@ -1015,7 +1070,7 @@ static void wave_device(g16hip_circuit* C, Wave* W, uint32_t m, int b) {
   const size_t nv = C->n_vars, wb = 32 * nv;
   hipStream_t s = W->stream;
   G16_CHECK(hipMemcpyAsync(W->witness.p, W->staging[b], wb * m, hipMemcpyHostToDevice, s));
-  WavePlans P = wave_plans(C, W->sort_w.p, W->sort_h.p, m);
+  WavePlans P = wave_plans(C, W->sort_w.p, W->sort_h.p, m, W->cap, W->fast);
   // The buffers are sized for the wave's cap; a plan for m <= cap proofs must fit them.
   if (msm_accum_scratch_bytes(P.w, 1) > W->accum_g1[0].bytes ||
       msm_accum_scratch_bytes(P.h, 1) > W->accum_g1[3].bytes ||
@@ -1095,7 +1150,7 @@ static void finish_wave(g16hip_circuit* C, Wave* W, const std::vector<WaveItem>&
   G16_CHECK(hipEventSynchronize(W->done[b]));
   const uint32_t m = (uint32_t)it.size(), cap = W->cap;
   static char anchor;
-  const WavePlans P = wave_plans(C, &anchor, &anchor, m);
+  const WavePlans P = wave_plans(C, &anchor, &anchor, m, cap, W->fast);
   const uint8_t* rows = W->host_wout[b];
   auto g1 = [&](int j, uint32_t k, const MsmPlan& v) {
     return msm_combine(reinterpret_cast<const G1X*>(rows + wave_rows_offset(P, cap, j, k)), v);
@@ -1217,8 +1272,9 @@ namespace g16 {
 // Adds one slot to `C` if the device keeps `reserve` bytes free after it (admission by free
 // device memory); returns whether it did.
 static bool try_add_slot(g16hip_circuit* C, size_t reserve) {
-  if (device_budget(C->dev) < slot_bytes_estimate(C) + reserve) return false;
-  auto S = make_slot(C);
+  const size_t budget = device_budget(C->dev);
+  if (budget < slot_bytes_estimate(C, false) + reserve) return false;
+  auto S = make_slot(C, budget >= slot_bytes_estimate(C, true) + reserve);
   std::lock_guard<std::mutex> lk(C->mu);
   C->slots.push_back(std::move(S));
   C->busy.push_back(false);
@@ -1326,7 +1382,7 @@ g16hip_status g16hip_prepare(g16hip_device* d, const g16hip_key* key, g16hip_cir
     // its streams first).
     auto S = new_slot();
     upload_key(C.get(), key, plan, S->stream);
-    size_slot(C.get(), S.get());
+    size_slot(C.get(), S.get(), plan.fast);
     C->slots.push_back(std::move(S));
     C->busy.push_back(false);
     *out = C.release();
@@ -1649,7 +1705,7 @@ g16hip_status g16hip_batch_autotune(g16hip_circuit* C, const uint8_t* w, size_t 
     for (uint32_t cap = 1; cap <= max_cap; cap *= 2) {
       {
         std::lock_guard<std::mutex> lk(C->wave_mu);
-        if (wave_bytes_for(C, cap) > device_budget(C->dev)) break;
+        if (wave_bytes_for(C, cap, false) > device_budget(C->dev)) break;
         C->wave_cap = cap;
       }
       // one warm wave, then two timed ones, all of the caller's witness

@@ -120,10 +120,16 @@ NttTables& ntt_tables_for(g16hip_device* d, int L) {
 
 static size_t round256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-MsmScratchSizes msm_scratch_sizes(int group, uint32_t n, int c, bool constant) {
+static void bind_standalone(MsmPlan& plan, void* scratch, uint32_t n, int c, bool constant,
+                            bool lean) {
+  const size_t entries = (size_t)n * ((255 + c - 1) / c);
+  msm_plan_bind(plan, scratch, n, c, false, constant, 1, lean ? 0 : entries);
+}
+
+MsmScratchSizes msm_scratch_sizes(int group, uint32_t n, int c, bool constant, bool lean) {
   MsmPlan plan;
   static char anchor;  // the plan is bound only to size its pieces
-  msm_plan_bind(plan, &anchor, n, c, false, constant);
+  bind_standalone(plan, &anchor, n, c, constant, lean);
   const size_t pt = group == 1 ? 128 : 256;  // XYZZ point
   MsmScratchSizes z;
   z.sort = round256(msm_sort_scratch_bytes(n, c));
@@ -142,9 +148,9 @@ int msm_width(uint32_t n, int c) {
 // statistics).
 template <class F>
 static Xyzz<F> run_msm_on(g16hip_device* d, int group, const void* bases, const void* scalars,
-                          uint32_t n, int c, const MsmScratch& sc) {
+                          uint32_t n, int c, bool lean, const MsmScratch& sc) {
   MsmPlan plan;
-  msm_plan_bind(plan, sc.sort, n, c, false, d->constant_work);
+  bind_standalone(plan, sc.sort, n, c, d->constant_work, lean);
   const size_t npts = msm_out_points(plan);
   const size_t coords = (size_t)n * (group == 1 ? 2 : 4);
   G16_CHECK(hipEventRecord(d->ev[0], d->stream));
@@ -175,33 +181,33 @@ static Xyzz<F> run_msm_on(g16hip_device* d, int group, const void* bases, const 
 // The same with scratch the device owns and grows as needed.
 template <class F>
 static Xyzz<F> run_msm(g16hip_device* d, int group, const void* bases, const void* scalars,
-                       uint32_t n, int c) {
+                       uint32_t n, int c, bool lean = false) {
   c = msm_width(n, c);
-  const MsmScratchSizes z = msm_scratch_sizes(group, n, c, d->constant_work);
+  const MsmScratchSizes z = msm_scratch_sizes(group, n, c, d->constant_work, lean);
   d->scratch_d.alloc(z.sort);
   d->scratch_e.alloc(z.accum);
   d->msm_bases.alloc(z.bases);
-  return run_msm_on<F>(d, group, bases, scalars, n, c,
+  return run_msm_on<F>(d, group, bases, scalars, n, c, lean,
                        MsmScratch{d->scratch_d.p, d->scratch_e.p, d->msm_bases.p});
 }
 
 // One device MSM on caller-provided scratch, result affine in the wire encoding (the caller
 // holds d->mu and has made d's device current).
 void msm_device_on_scratch(g16hip_device* d, int group, const void* bases, const void* scalars,
-                           uint32_t n, int c, const MsmScratch& sc, uint8_t* out) {
-  if (group == 1) g1_store(out, host_to_aff(run_msm_on<Fq>(d, 1, bases, scalars, n, c, sc)));
-  else g2_store(out, host_to_aff(run_msm_on<Fq2>(d, 2, bases, scalars, n, c, sc)));
+                           uint32_t n, int c, bool lean, const MsmScratch& sc, uint8_t* out) {
+  if (group == 1) g1_store(out, host_to_aff(run_msm_on<Fq>(d, 1, bases, scalars, n, c, lean, sc)));
+  else g2_store(out, host_to_aff(run_msm_on<Fq2>(d, 2, bases, scalars, n, c, lean, sc)));
 }
 
 
 // Device bytes one standalone MSM of n points at width c takes: the uploaded bases and
 // scalars, the bases in the MSM form, the sort scratch and the accumulation scratch (with
-// the fold's slots under constant work).
-static size_t msm_run_bytes(int group, uint32_t n, int c, bool constant) {
+// the fold's slots under constant work). With `lean` false the scratch of short segments.
+static size_t msm_run_bytes(int group, uint32_t n, int c, bool constant, bool lean = true) {
   size_t pw = group == 1 ? 64 : 128;
   MsmPlan plan;
   static char anchor;  // the plan is bound only to size its pieces
-  msm_plan_bind(plan, &anchor, n, c, false, constant);
+  bind_standalone(plan, &anchor, n, c, constant, lean);
   return 2 * pw * (size_t)n + 32 * (size_t)n + msm_sort_scratch_bytes(n, c) +
          msm_accum_scratch_bytes(plan, group) + 256 * msm_out_points(plan);
 }
@@ -209,11 +215,11 @@ static size_t msm_run_bytes(int group, uint32_t n, int c, bool constant) {
 // One MSM over host slices: upload, run, result in XYZZ (the caller holds d->mu).
 template <class F>
 static Xyzz<F> msm_from_host(g16hip_device* d, int group, const uint8_t* bases,
-                             const uint8_t* scalars, size_t n) {
+                             const uint8_t* scalars, size_t n, bool lean = false) {
   size_t pw = group == 1 ? 64 : 128;
   upload(d->scratch_a, bases, n * pw, d->stream);
   upload(d->scratch_b, scalars, n * 32, d->stream);
-  return run_msm<F>(d, group, d->scratch_a.p, d->scratch_b.p, (uint32_t)n, 0);
+  return run_msm<F>(d, group, d->scratch_a.p, d->scratch_b.p, (uint32_t)n, 0, lean);
 }
 
 static Fq fq_small(uint32_t k) {
@@ -268,8 +274,11 @@ template <class F>
 static Xyzz<F> ceremony_run(g16hip_ceremony* cer, int group, const uint8_t* bases,
                             const uint8_t* scalars, size_t n) {
   g16hip_device* d = cer->dev;
+  bool lean = false;
   if (cer->vram_limit) {
-    size_t need = msm_run_bytes(group, (uint32_t)n, msm_default_c((uint32_t)n), d->constant_work);
+    const int c = msm_default_c((uint32_t)n);
+    const size_t need = msm_run_bytes(group, (uint32_t)n, c, d->constant_work);
+    lean = msm_run_bytes(group, (uint32_t)n, c, d->constant_work, false) > cer->vram_limit;
     if (need > cer->vram_limit)
       throw StatusError{G16HIP_DEVICE_MEMORY,
                         "a run of " + std::to_string(n) + " points needs " + std::to_string(need) +
@@ -280,7 +289,7 @@ static Xyzz<F> ceremony_run(g16hip_ceremony* cer, int group, const uint8_t* base
     {
       std::lock_guard<std::mutex> lk(d->mu);
       set_device(d);
-      p = msm_from_host<F>(d, group, bases, scalars, n);
+      p = msm_from_host<F>(d, group, bases, scalars, n, lean);
     }
     if (xyzz_on_curve(p)) return p;
     cer->tally.retries += 1;

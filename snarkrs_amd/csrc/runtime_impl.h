@@ -457,12 +457,13 @@ struct MsmScratchSizes {
   size_t sort = 0, accum = 0, bases = 0;
   size_t total() const { return sort + accum + bases; }
 };
-MsmScratchSizes msm_scratch_sizes(int group, uint32_t n, int c, bool constant);
+// `lean`: the least scratch (long segments), for callers that the usual one does not fit.
+MsmScratchSizes msm_scratch_sizes(int group, uint32_t n, int c, bool constant, bool lean);
 // c, or the library's width for n when c <= 0; throws outside [2, 16].
 int msm_width(uint32_t n, int c);
 // One device MSM (group 1 or 2) on caller-provided scratch, result affine in the wire
 // encoding; the caller holds d->mu with d's device current.
 void msm_device_on_scratch(g16hip_device* d, int group, const void* bases, const void* scalars,
-                           uint32_t n, int c, const MsmScratch& sc, uint8_t* out);
+                           uint32_t n, int c, bool lean, const MsmScratch& sc, uint8_t* out);
 
 }  // namespace g16

@@ -29,3 +29,21 @@ def test_one_bucket_per_window(dev, group, kind):
         got = dev.msm(group, bases, fr_array([s] * n))
         total = sum(ks) * s % R_MOD
         assert (got == dev.fixed_base(group, fr_array([total]))[0]).all(), (n, s)
+
+
+@pytest.mark.parametrize("group,n", [(1, 1021), (1, 4099), (2, 1021), (2, 5003)])
+def test_least_scratch_runs_in_one_piece(dev, group, n):
+    # A limit of exactly scratch_bytes holds the run (long segments); without one the same sum
+    # comes from short segments.
+    from snarkrs_amd.native import CeremonyMsm
+
+    rng = SplitMix64(40 + n)
+    ks = [rng.next_fr() for _ in range(n)]
+    ss = [rng.next_fr() if i % 3 else i % 2 for i in range(n)]
+    bases, scalars = dev.fixed_base(group, fr_array(ks)), fr_array(ss)
+    want = dev.fixed_base(group, fr_array([sum(k * s for k, s in zip(ks, ss)) % R_MOD]))[0]
+    lean = CeremonyMsm(dev, vram_limit=CeremonyMsm.scratch_bytes(group, n))
+    for cer in (lean, CeremonyMsm(dev)):
+        got = (cer.msm_g1 if group == 1 else cer.msm_g2)(bases, scalars)
+        assert cer.last_runs() == 1
+        assert (got == want).all()
