@@ -131,13 +131,15 @@ inline MsmPlan msm_vector_view(const MsmPlan& p) {
   v.max_entries = (size_t)p.n * p.windows;
   return v;
 }
-size_t msm_sort_scratch_bytes(uint32_t n, int c, uint32_t batch = 1);
-// `at_once`: entries the device works on together in the launches this plan is for (0: as many
-// as fill it). Fewer than fill it are cut into shorter segments, which take more scratch
-// (msm_accum_scratch_bytes); a caller short of memory passes 0. A wave passes the same count for
-// its cap and every smaller number of proofs, so that all fit the scratch sized for the cap.
+// For `batch` vectors and every smaller number (a plan's cap).
+size_t msm_sort_scratch_bytes(uint32_t n, int c, bool lean, uint32_t batch = 1);
+// `cap`: the vectors the scratch is sized for (0: `batch`). Every smaller batch cuts its digits
+// and entries the same way, so that it fits. An MSM too small to fill the device is cut into
+// smaller pieces than a large one, which takes more scratch (msm_sort_scratch_bytes,
+// msm_accum_scratch_bytes); a caller short of memory passes `lean` for the least.
 void msm_plan_bind(MsmPlan& p, void* scratch, uint32_t n, int c, bool merged = false,
-                   bool constant = false, uint32_t batch = 1, size_t at_once = 0);
+                   bool constant = false, uint32_t batch = 1, uint32_t cap = 0,
+                   bool lean = false);
 // Window tables for merged MSMs: `table` holds n affine bases (MSM form) at [0, n); fills
 // entries w n + i = 2^(c w) P_i for 1 <= w < windows. group 1 = G1, 2 = G2.
 void msm_window_tables(int group, void* table, size_t n, int c, int windows, hipStream_t s);

@@ -102,7 +102,8 @@ static bool short_digits(const MsmPlan& p) { return p.c <= 15 && !p.constant; }
 //      entries with their full keys, in order of bucket, inside the group's range.
 // A set is a digit row (per-window buckets) or a vector's W rows (merged windows). Entries of a
 // bucket come out in any order; its sum does not depend on it.
-static constexpr uint32_t SORT_CHUNK = 65536;  // scalars per coarse workgroup (at least)
+static constexpr uint32_t SORT_CHUNK = 65536;  // scalars per coarse workgroup
+static constexpr uint32_t SORT_CHUNK_MIN = 8192;
 static constexpr int SORT_THREADS = 1024;
 static constexpr int SORT_ITEMS = 8;           // digits per thread per round (loads first)
 static constexpr int FINE_THREADS = 256;
@@ -530,6 +531,113 @@ __global__ void k_scan_fix(uint32_t* offset, const uint32_t* bsum, uint32_t K) {
   if (i == 0) offset[K] = bsum[1024];
 }
 
+// The whole sort of a small MSM in one workgroup: every bucket's count in LDS, a scan, then the
+// entries to their places (the digits are computed twice instead of stored). It is bound by one
+// compute unit's instruction issue, 35 us for 30 thousand entries, as long as the general path's
+// ten kernels together, but those spend as much again between their launches: the
+// 1000-constraint prove, which sorts twice, 895 -> 810 us (MI355X). Up to TINY_ENTRIES entries
+// and TINY_BUCKETS buckets.
+static constexpr uint32_t TINY_ENTRIES = 131072;
+static constexpr uint32_t TINY_BUCKETS = 15360;  // 60 KB of LDS
+
+__global__ void __launch_bounds__(SORT_THREADS) k_sort_tiny(const uint4* scalars, uint32_t n,
+                                                            uint32_t batch, int c, int W,
+                                                            uint32_t nb, uint32_t K, int merged,
+                                                            int constant, uint2* ent,
+                                                            uint32_t* offset, uint32_t* total) {
+  extern __shared__ uint32_t hist[];  // K words
+  __shared__ uint32_t scan_sh[SORT_THREADS / 64];
+  for (uint32_t j = threadIdx.x; j < K; j += SORT_THREADS) hist[j] = 0;
+  __syncthreads();
+  const uint32_t all = n * batch;
+  for (int pass = 0; pass < 2; ++pass) {
+    for (uint32_t i = threadIdx.x; i < all; i += SORT_THREADS) {
+      const uint32_t k = i / n, j = i - k * n;  // scalar j of vector k
+      const Fr x = to_std(ld_fr(scalars + 2 * (size_t)i));
+      const uint32_t zero = constant ? (j & (nb - 1u)) | DIGIT_DISCARD : DIGIT_ZERO;
+      using D = Digit<uint32_t>;
+      // Four windows at a time, their atomics in flight together. Window 0 holds the ones of a
+      // boolean witness, all in one bucket: there a wave takes them with one atomic.
+      for (int w0 = 0; w0 < W; w0 += 4) {
+        uint32_t e[4], key[4], pos[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int w = w0 + u;
+          e[u] = w < W ? D::make(signed_digit(x.v, w, c), zero) : DIGIT_ZERO;
+          key[u] = (merged ? k : k * W + w) * nb + D::bucket(e[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (!D::zero(e[u]))
+            pos[u] = w0 + u == 0 ? lds_take(hist, key[u]) : atomicAdd(&hist[key[u]], 1u);
+        if (!pass) continue;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (D::zero(e[u])) continue;
+          const uint32_t idx = merged ? (uint32_t)(w0 + u) * n + j : j;
+          ent[pos[u]] = make_uint2(key[u], constant ? (idx << 2) | D::discard(e[u]) | D::sign(e[u])
+                                                    : (idx << 1) | D::sign(e[u]));
+        }
+      }
+    }
+    __syncthreads();
+    if (pass) return;
+    // counts to first positions
+    const uint32_t per = (K + SORT_THREADS - 1) / SORT_THREADS;
+    const uint32_t j0 = threadIdx.x * per, j1 = j0 + per < K ? j0 + per : K;
+    uint32_t loc = 0;
+    for (uint32_t j = j0; j < j1; ++j) loc += hist[j];
+    uint32_t sum;
+    uint32_t run = block_exclusive<SORT_THREADS>(loc, scan_sh, &sum);
+    for (uint32_t j = j0; j < j1; ++j) {
+      const uint32_t v = hist[j];
+      hist[j] = run;
+      offset[j] = run;
+      run += v;
+    }
+    if (threadIdx.x == 0) {
+      offset[K] = sum;
+      total[0] = sum;
+    }
+    __syncthreads();
+  }
+}
+
+// The scan of at most SCAN_ONE counts and the slice prefix in one workgroup: one launch for
+// k_scan_blocks, k_scan_top, k_scan_fix and k_slice_scan.
+static constexpr uint32_t SCAN_ONE = 32768;
+__global__ void __launch_bounds__(1024) k_scan_one(const uint32_t* count, uint32_t q,
+                                                   uint32_t* cpos, uint32_t per_group,
+                                                   uint32_t groups, uint32_t* sprefix) {
+  __shared__ uint32_t sh[16];
+  const uint32_t per = (q + 1023) / 1024;
+  const uint32_t j0 = threadIdx.x * per < q ? threadIdx.x * per : q;
+  const uint32_t j1 = j0 + per < q ? j0 + per : q;
+  uint32_t loc = 0;
+  for (uint32_t j = j0; j < j1; ++j) loc += count[j];
+  uint32_t all;
+  uint32_t run = block_exclusive<1024>(loc, sh, &all);
+  for (uint32_t j = j0; j < j1; ++j) {
+    const uint32_t v = count[j];
+    cpos[j] = run;
+    run += v;
+  }
+  if (threadIdx.x == 0) cpos[q] = all;
+  __syncthreads();  // this workgroup's own stores are read below
+  const uint32_t pg = (groups + 1023) / 1024;
+  const uint32_t g0 = threadIdx.x * pg < groups ? threadIdx.x * pg : groups;
+  const uint32_t g1 = g0 + pg < groups ? g0 + pg : groups;
+  uint32_t slices = 0;
+  for (uint32_t g = g0; g < g1; ++g)
+    slices += slices_of(cpos[(size_t)(g + 1) * per_group] - cpos[(size_t)g * per_group]);
+  uint32_t before = block_exclusive<1024>(slices, sh, &all);
+  for (uint32_t g = g0; g < g1; ++g) {
+    sprefix[g] = before;
+    before += slices_of(cpos[(size_t)(g + 1) * per_group] - cpos[(size_t)g * per_group]);
+  }
+  if (threadIdx.x == 0) sprefix[groups] = all;
+}
+
 int msm_choose_c(uint32_t n, int g1, int g2) {
   // The reference's cost model (crates/msm/src/lib.rs:160-172) prices a window at
   // n + 2 * buckets points. Here the weights are fitted to this build's measurements on gfx950
@@ -575,8 +683,10 @@ int msm_choose_c_merged(uint32_t n, int g1, int g2) {
 static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // The sort's geometry: coarse bins per set (fine bins per coarse bin at most 2^MAX_FINE_SHIFT,
-// coarse bins at most MAX_CBINS), and chunks of at
-// least SORT_CHUNK scalars, doubled until the count array fits the scan (1024 SCAN_BLOCK).
+// coarse bins at most MAX_CBINS), and chunks of SORT_CHUNK scalars, doubled until the count array
+// fits the scan (1024 SCAN_BLOCK), or halved, down to SORT_CHUNK_MIN, while the coarse kernels
+// would have under 256 workgroups (the counts' scratch grows; `lean` keeps SORT_CHUNK):
+// coarse count and scatter of H at 65k constraints 18 + 44 us with 32 workgroups, 6 + 13 with 256.
 struct SortGeom {
   int shift = 0;
   uint32_t cbins = 1, rows_per_set = 1, sets = 1, rows = 1, cs = SORT_CHUNK, chunks = 1;
@@ -586,7 +696,10 @@ struct SortGeom {
   size_t fine_words() const { return ((size_t)1 << shift) * max_slices; }
 };
 
-static SortGeom sort_geom(uint32_t n, int c, uint32_t batch, bool merged) {
+// Everything but the counts' length follows `cap`, not the vectors sorted now: a smaller batch's
+// pieces fit the scratch sized for the cap.
+static SortGeom sort_geom(uint32_t n, int c, uint32_t batch, bool merged, uint32_t cap_batch,
+                          bool lean) {
   SortGeom g;
   const int W = (RECODE_BITS + c - 1) / c;
   const uint32_t nb = 1u << (c - 1);
@@ -605,11 +718,13 @@ static SortGeom sort_geom(uint32_t n, int c, uint32_t batch, bool merged) {
   while (cb > 1 && (size_t)cb * 1024 > per_set) cb /= 2;
   if (cb < lo) cb = lo;
   const size_t cap = (size_t)1024 * SCAN_BLOCK - 1;
+  const size_t rows_cap = (size_t)cap_batch * W;
   uint32_t cs = SORT_CHUNK;
   auto chunks_of = [&](uint32_t x) { return n ? (uint32_t)(((size_t)n + x - 1) / x) : 1u; };
-  while ((size_t)g.rows * cb * chunks_of(cs) > cap && cs < (1u << 30)) cs *= 2;
-  while ((size_t)g.rows * cb * chunks_of(cs) > cap && cb > lo) cb /= 2;
-  if ((size_t)g.rows * cb * chunks_of(cs) > cap) throw ArgError{"MSM too large for the sort's scan"};
+  while (!lean && cs > SORT_CHUNK_MIN && rows_cap * chunks_of(cs) < 256) cs /= 2;
+  while (rows_cap * cb * chunks_of(cs) > cap && cs < (1u << 30)) cs *= 2;
+  while (rows_cap * cb * chunks_of(cs) > cap && cb > lo) cb /= 2;
+  if (rows_cap * cb * chunks_of(cs) > cap) throw ArgError{"MSM too large for the sort's scan"};
   g.cbins = cb;
   g.shift = 0;
   while ((cb << g.shift) < nb) ++g.shift;
@@ -623,13 +738,14 @@ static SortGeom sort_geom(uint32_t n, int c, uint32_t batch, bool merged) {
   return g;
 }
 
-size_t msm_sort_scratch_bytes(uint32_t n, int c, uint32_t batch) {
+size_t msm_sort_scratch_bytes(uint32_t n, int c, bool lean, uint32_t batch) {
   const int W = (RECODE_BITS + c - 1) / c;
   const size_t nb = (size_t)1 << (c - 1);
   const size_t E = (size_t)batch * n * W;
   // Sized for per-window sets (the larger key count) and the geometry of either layout.
   const size_t K = (size_t)batch * W * nb;
-  const SortGeom a = sort_geom(n, c, batch, false), b = sort_geom(n, c, batch, true);
+  const SortGeom a = sort_geom(n, c, batch, false, batch, lean),
+                 b = sort_geom(n, c, batch, true, batch, lean);
   const size_t q = std::max(a.q, b.q);
   const size_t groups = std::max(a.groups, b.groups);
   const size_t fine = std::max(a.fine_words(), b.fine_words());
@@ -658,15 +774,16 @@ static constexpr size_t SEG_LANES[2] = {262144, 65536};  // G1: four waves per S
 static uint32_t segment_length(const MsmPlan& p, int g, size_t at_once) {
   if (p.constant && p.merged) return 64u;
   uint32_t seg = !p.merged && g == 0 ? 40u : 32u;
-  if (p.constant || !at_once) return seg;
+  if (p.constant || !at_once) return seg;  // constant work, or the least scratch
   while (seg >= 16 && at_once / seg < SEG_LANES[g]) seg /= 2;
   return seg;
 }
 
 void msm_plan_bind(MsmPlan& p, void* scratch, uint32_t n, int c, bool merged, bool constant,
-                   uint32_t batch, size_t at_once) {
+                   uint32_t batch, uint32_t cap, bool lean) {
   if (c < 2 || c > MSM_MAX_C) throw ArgError{"MSM window width must be in [2, 20]"};
   if (batch == 0) throw ArgError{"MSM batch of zero vectors"};
+  if (cap < batch) cap = batch;
   p.merged = merged;
   p.constant = constant;
   p.c = c;
@@ -679,7 +796,7 @@ void msm_plan_bind(MsmPlan& p, void* scratch, uint32_t n, int c, bool merged, bo
   if (p.max_entries >= (1ull << 31)) throw ArgError{"MSM entry count exceeds 2^31"};
   if (constant && (merged ? (size_t)n * p.windows : (size_t)n) >= (1ull << 30))
     throw ArgError{"constant-work MSM: base indices must stay below 2^30"};
-  const SortGeom g = sort_geom(n, c, batch, merged);
+  const SortGeom g = sort_geom(n, c, batch, merged, cap, lean);
   p.shift = g.shift;
   p.cbins = g.cbins;
   p.rows_per_set = g.rows_per_set;
@@ -688,7 +805,7 @@ void msm_plan_bind(MsmPlan& p, void* scratch, uint32_t n, int c, bool merged, bo
   p.q = g.q;
   p.groups = g.groups;
   p.max_slices = g.max_slices;
-  for (int g = 0; g < 2; ++g) p.seg[g] = segment_length(p, g, at_once);
+  for (int g = 0; g < 2; ++g) p.seg[g] = segment_length(p, g, lean ? 0 : (size_t)cap * n * p.windows);
   const size_t K = (size_t)msm_bucket_sets(p) * p.nb;
   char* q = static_cast<char*>(scratch);
   auto take = [&](size_t bytes) {
@@ -733,6 +850,14 @@ static void sort_coarse_scatter(MsmPlan& p, hipStream_t s) {
 
 void msm_sort(MsmPlan& p, const void* scalars, hipStream_t s) {
   const uint32_t Q = (uint32_t)p.q;
+  const size_t K = (size_t)msm_bucket_sets(p) * p.nb;
+  if (p.n && p.max_entries <= TINY_ENTRIES && K <= TINY_BUCKETS) {
+    hipLaunchKernelGGL(k_sort_tiny, dim3(1), dim3(SORT_THREADS), 4 * K, s,
+                       static_cast<const uint4*>(scalars), p.n, p.batch, p.c, p.windows, p.nb,
+                       (uint32_t)K, (int)p.merged, (int)p.constant, p.ent, p.offset, p.total);
+    G16_LAUNCH_CHECK("msm sort (one workgroup)");
+    return;
+  }
   if (p.n) {
     if (short_digits(p)) sort_coarse_count<uint16_t>(p, scalars, s);
     else sort_coarse_count<uint32_t>(p, scalars, s);
@@ -741,22 +866,31 @@ void msm_sort(MsmPlan& p, const void* scalars, hipStream_t s) {
                        (size_t)Q, 0u);
     G16_LAUNCH_CHECK("msm clear counts");
   }
-  const uint32_t nblk = (Q + SCAN_BLOCK - 1) / SCAN_BLOCK;
-  hipLaunchKernelGGL(k_scan_blocks, dim3(nblk), dim3(256), 0, s, p.ccount, Q, p.cpos,
-                     p.block_sums);
-  G16_LAUNCH_CHECK("msm scan");
-  hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, p.block_sums, nblk);
-  G16_LAUNCH_CHECK("msm scan top");
-  hipLaunchKernelGGL(k_scan_fix, dim3((Q + 255) / 256), dim3(256), 0, s, p.cpos, p.block_sums, Q);
-  G16_LAUNCH_CHECK("msm scan fix");
+  const uint32_t per_group = p.rows_per_set * p.chunks;
+  const bool one = Q <= SCAN_ONE;
+  if (one) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(1024), 0, s, p.ccount, Q, p.cpos, per_group,
+                       p.groups, p.sprefix);
+    G16_LAUNCH_CHECK("msm scan (one workgroup)");
+  } else {
+    const uint32_t nblk = (Q + SCAN_BLOCK - 1) / SCAN_BLOCK;
+    hipLaunchKernelGGL(k_scan_blocks, dim3(nblk), dim3(256), 0, s, p.ccount, Q, p.cpos,
+                       p.block_sums);
+    G16_LAUNCH_CHECK("msm scan");
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, s, p.block_sums, nblk);
+    G16_LAUNCH_CHECK("msm scan top");
+    hipLaunchKernelGGL(k_scan_fix, dim3((Q + 255) / 256), dim3(256), 0, s, p.cpos, p.block_sums, Q);
+    G16_LAUNCH_CHECK("msm scan fix");
+  }
   if (p.n) {
     if (short_digits(p)) sort_coarse_scatter<uint16_t>(p, s);
     else sort_coarse_scatter<uint32_t>(p, s);
   }
-  const uint32_t per_group = p.rows_per_set * p.chunks;
-  hipLaunchKernelGGL(k_slice_scan, dim3(1), dim3(1024), 0, s, p.cpos, per_group, p.groups,
-                     p.sprefix);
-  G16_LAUNCH_CHECK("msm slice scan");
+  if (!one) {
+    hipLaunchKernelGGL(k_slice_scan, dim3(1), dim3(1024), 0, s, p.cpos, per_group, p.groups,
+                       p.sprefix);
+    G16_LAUNCH_CHECK("msm slice scan");
+  }
   hipLaunchKernelGGL(k_fine_count, dim3(p.max_slices), dim3(FINE_THREADS), 0, s, p.tmp, p.cpos,
                      per_group, p.groups, p.sprefix, p.shift, p.fcnt);
   G16_LAUNCH_CHECK("msm fine count");

@@ -373,9 +373,8 @@ static constexpr size_t TOGETHER_BYTES = 256ull << 20;
 // A slot's two plans: the witness's (A, B1, L and B2), H's.
 static void slot_plans(MsmPlan& w, MsmPlan& h, void* sort_w, void* sort_h, uint32_t nv,
                        uint32_t nh, int cw, int ch, bool merged, bool constant, bool fast) {
-  const size_t ew = (size_t)nv * ((255 + cw - 1) / cw), eh = (size_t)nh * ((255 + ch - 1) / ch);
-  msm_plan_bind(w, sort_w, nv, cw, merged, constant, 1, fast ? ew : 0);
-  msm_plan_bind(h, sort_h, nh, ch, merged, constant, 1, fast ? eh : 0);
+  msm_plan_bind(w, sort_w, nv, cw, merged, constant, 1, 1, !fast);
+  msm_plan_bind(h, sort_h, nh, ch, merged, constant, 1, 1, !fast);
 }
 
 // Bytes of a slot's G1 witness scratch: one MSM's, or three when they run together.
@@ -391,8 +390,8 @@ static void size_slot(const g16hip_circuit* C, Slot* S, bool fast) {
   S->witness.alloc(32 * nv);
   S->abc.alloc(32 * 3 * n);
   S->hbuf.alloc(32 * n);
-  S->sort_w.alloc(msm_sort_scratch_bytes((uint32_t)nv, C->cw));
-  S->sort_h.alloc(msm_sort_scratch_bytes(C->n_h, C->ch));
+  S->sort_w.alloc(msm_sort_scratch_bytes((uint32_t)nv, C->cw, !fast));
+  S->sort_h.alloc(msm_sort_scratch_bytes(C->n_h, C->ch, !fast));
   slot_plans(S->plan_w, S->plan_h, S->sort_w.p, S->sort_h.p, (uint32_t)nv, C->n_h, C->cw, C->ch,
              C->merged, C->constant, fast);
   S->accum_w1.alloc(accum_w1_bytes(S->plan_w, fast));
@@ -424,7 +423,8 @@ static size_t slot_bytes_for(uint32_t nv, uint32_t n, uint32_t nh, int cw, int c
   static char anchor;  // the plans are bound only to size their pieces
   slot_plans(pw, ph, &anchor, &anchor, nv, nh, cw, ch, merged, constant, fast);
   return dev_pages(32 * (size_t)nv) + dev_pages(32 * 3 * (size_t)n) + dev_pages(32 * (size_t)n) +
-         dev_pages(msm_sort_scratch_bytes(nv, cw)) + dev_pages(msm_sort_scratch_bytes(nh, ch)) +
+         dev_pages(msm_sort_scratch_bytes(nv, cw, !fast)) +
+         dev_pages(msm_sort_scratch_bytes(nh, ch, !fast)) +
          dev_pages(accum_w1_bytes(pw, fast)) + dev_pages(msm_accum_scratch_bytes(pw, 2)) +
          dev_pages(msm_accum_scratch_bytes(ph, 1));
 }
@@ -973,14 +973,12 @@ struct WavePlans {
   size_t rw = 0, rh = 0;  // reduction rows per proof
 };
 
-// The plans of a wave of m proofs, m <= cap: segments follow the cap's entries, whatever m is.
+// The plans of a wave of m proofs, m <= cap, over scratch sized for cap.
 static WavePlans wave_plans(const g16hip_circuit* C, void* sort_w, void* sort_h, uint32_t m,
                             uint32_t cap, bool fast) {
   WavePlans P;
-  const size_t ew = (size_t)cap * C->n_vars * ((255 + C->cw - 1) / C->cw);
-  const size_t eh = (size_t)cap * C->n_h * ((255 + C->ch - 1) / C->ch);
-  msm_plan_bind(P.w, sort_w, C->n_vars, C->cw, C->merged, C->constant, m, fast ? ew : 0);
-  msm_plan_bind(P.h, sort_h, C->n_h, C->ch, C->merged, C->constant, m, fast ? eh : 0);
+  msm_plan_bind(P.w, sort_w, C->n_vars, C->cw, C->merged, C->constant, m, cap, !fast);
+  msm_plan_bind(P.h, sort_h, C->n_h, C->ch, C->merged, C->constant, m, cap, !fast);
   P.vw = msm_vector_view(P.w);
   P.vh = msm_vector_view(P.h);
   P.rw = msm_out_points(P.vw);
@@ -1006,8 +1004,8 @@ static size_t wave_bytes_for(const g16hip_circuit* C, uint32_t cap, bool fast) {
   const WavePlans P = wave_plans(C, &anchor, &anchor, cap, cap, fast);
   const size_t nv = C->n_vars, n = C->domain;
   return dev_pages(32 * nv * cap) + dev_pages(96 * n * cap) + dev_pages(32 * n * cap) +
-         dev_pages(msm_sort_scratch_bytes((uint32_t)nv, C->cw, cap)) +
-         dev_pages(msm_sort_scratch_bytes(C->n_h, C->ch, cap)) +
+         dev_pages(msm_sort_scratch_bytes((uint32_t)nv, C->cw, !fast, cap)) +
+         dev_pages(msm_sort_scratch_bytes(C->n_h, C->ch, !fast, cap)) +
          3 * dev_pages(msm_accum_scratch_bytes(P.w, 1)) + dev_pages(msm_accum_scratch_bytes(P.w, 2)) +
          dev_pages(msm_accum_scratch_bytes(P.h, 1)) + dev_pages(256);
 }
@@ -1039,8 +1037,8 @@ static std::unique_ptr<Wave> make_wave(g16hip_circuit* C, uint32_t cap) {
   W->witness.alloc(32 * nv * cap);
   W->abc.alloc(96 * n * cap);
   W->hbuf.alloc(32 * n * cap);
-  W->sort_w.alloc(msm_sort_scratch_bytes((uint32_t)nv, C->cw, cap));
-  W->sort_h.alloc(msm_sort_scratch_bytes(C->n_h, C->ch, cap));
+  W->sort_w.alloc(msm_sort_scratch_bytes((uint32_t)nv, C->cw, !fast, cap));
+  W->sort_h.alloc(msm_sort_scratch_bytes(C->n_h, C->ch, !fast, cap));
   const WavePlans P = wave_plans(C, W->sort_w.p, W->sort_h.p, cap, cap, fast);
   for (int j = 0; j < 3; ++j) W->accum_g1[j].alloc(msm_accum_scratch_bytes(P.w, 1));
   W->accum_g1[3].alloc(msm_accum_scratch_bytes(P.h, 1));

@@ -122,8 +122,7 @@ static size_t round256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 static void bind_standalone(MsmPlan& plan, void* scratch, uint32_t n, int c, bool constant,
                             bool lean) {
-  const size_t entries = (size_t)n * ((255 + c - 1) / c);
-  msm_plan_bind(plan, scratch, n, c, false, constant, 1, lean ? 0 : entries);
+  msm_plan_bind(plan, scratch, n, c, false, constant, 1, 1, lean);
 }
 
 MsmScratchSizes msm_scratch_sizes(int group, uint32_t n, int c, bool constant, bool lean) {
@@ -132,7 +131,7 @@ MsmScratchSizes msm_scratch_sizes(int group, uint32_t n, int c, bool constant, b
   bind_standalone(plan, &anchor, n, c, constant, lean);
   const size_t pt = group == 1 ? 128 : 256;  // XYZZ point
   MsmScratchSizes z;
-  z.sort = round256(msm_sort_scratch_bytes(n, c));
+  z.sort = round256(msm_sort_scratch_bytes(n, c, lean));
   z.accum = round256(msm_accum_scratch_bytes(plan, group) + pt * msm_out_points(plan));
   z.bases = round256(32 * (size_t)n * (group == 1 ? 2 : 4));
   return z;
@@ -208,7 +207,7 @@ static size_t msm_run_bytes(int group, uint32_t n, int c, bool constant, bool le
   MsmPlan plan;
   static char anchor;  // the plan is bound only to size its pieces
   bind_standalone(plan, &anchor, n, c, constant, lean);
-  return 2 * pw * (size_t)n + 32 * (size_t)n + msm_sort_scratch_bytes(n, c) +
+  return 2 * pw * (size_t)n + 32 * (size_t)n + msm_sort_scratch_bytes(n, c, lean) +
          msm_accum_scratch_bytes(plan, group) + 256 * msm_out_points(plan);
 }
 

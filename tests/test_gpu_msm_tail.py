@@ -47,3 +47,22 @@ def test_least_scratch_runs_in_one_piece(dev, group, n):
         got = (cer.msm_g1 if group == 1 else cer.msm_g2)(bases, scalars)
         assert cer.last_runs() == 1
         assert (got == want).all()
+
+
+@pytest.mark.parametrize("constant", [False, True])
+@pytest.mark.parametrize("n", [1, 63, 1023, 1024, 1025, 4095, 4096, 4097, 6000])
+def test_sort_of_small_msms(dev, n, constant):
+    # The one-workgroup sort and the general one either side of their limits, on boolean-heavy
+    # scalars (most entries in one bucket).
+    rng = SplitMix64(70 + n)
+    ks = [rng.next_fr() for _ in range(n)]
+    ss = [rng.next_fr() if i % 4 == 0 else i % 2 for i in range(n)]
+    ss[0] = 0
+    bases = dev.fixed_base(1, fr_array(ks))
+    dev.set_constant_work(constant)
+    try:
+        got = dev.msm(1, bases, fr_array(ss))
+    finally:
+        dev.set_constant_work(False)
+    total = sum(k * s for k, s in zip(ks, ss)) % R_MOD
+    assert (got == dev.fixed_base(1, fr_array([total]))[0]).all()
