@@ -47,17 +47,17 @@ void launch_fr_to_rp(void* data, size_t n, hipStream_t s);  // R form -> R' form
 // multiplied by prescale[p] (the coset table in bit-reversed order, R' form). With
 // `natural_src` the input is read from there in natural order (the bit reversal folded into
 // the first pass's loads; natural_src may be data) and `tmp` (n elements per vector, distinct
-// from data and natural_src) holds the first pass's output.
+// from data and natural_src) holds the first pass's output. With `factor` (R' form; L > 0) the
+// last pass multiplies the result by it.
 void ntt_dif_inverse(void* data, int nvec, int log_n, const void* tw_inv, hipStream_t s);
 void ntt_dit_forward(void* data, int nvec, int log_n, const void* tw_fwd, const void* prescale,
-                     hipStream_t s, const void* natural_src = nullptr, void* tmp = nullptr);
+                     hipStream_t s, const void* natural_src = nullptr, void* tmp = nullptr,
+                     const void* factor = nullptr);
 // ntt_dif_inverse then ntt_dit_forward with `coset` as the prescale, the inverse's lowest pass
 // and the forward's first pass fused into one (the same tiles, in LDS). With h_out (nvec = 3:
 // A, B, C back to back), H = A B - C goes to h_out from the last pass and C is not stored.
 void ntt_coset_pipeline(void* data, int nvec, int log_n, const void* tw_inv, const void* tw_fwd,
                         const void* coset, hipStream_t s, void* h_out = nullptr);
-void launch_bitrev_permute(void* dst, const void* src, int log_n, hipStream_t s);
-void launch_scale(void* data, size_t n, const void* factor, hipStream_t s);
 void launch_scale_rp(void* data, size_t n, const void* factor_rp, hipStream_t s);
 void launch_mul_table_rp(void* data, size_t n, const void* table_rp, hipStream_t s);
 

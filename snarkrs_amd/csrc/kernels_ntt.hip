@@ -93,21 +93,35 @@ __device__ __forceinline__ uint32_t bitrev(uint32_t x, int L) {
 // The prover's iNTT -> coset shift -> NTT runs as three passes: the inverse's high stages, one
 // fused pass that does the inverse's low stages, multiplies by the coset table and does the
 // forward's low stages on the same tile in LDS, then the forward's high stages.
-static constexpr int NTT_LOG_TILE = 12;
-static constexpr int NTT_TILE = 1 << NTT_LOG_TILE;  // elements per workgroup
-static constexpr int NTT_THREADS = 512;
-static constexpr int NTT_HIGH_PASS = 10;  // stages per pass above the low pass: runs >= 4
+//
+// Transforms that would leave most of the device idle at that size (2^12 to 2^18 elements, under
+// 2^20 over the launch's vectors: at most 256 tiles) take tiles of 1024 elements, one radix-4
+// unit per thread and stage pair instead of two, on four times the compute units: forward 2^13
+// 72 -> 26 us of kernels, the three vectors of a 2^15 domain 190 -> 108 us (MI355X). A tile of
+// either size makes a 2^13 to 2^18 transform two passes.
+static constexpr int NTT_LOG_TILE = 12;       // large tiles
+static constexpr int NTT_LOG_TILE_SMALL = 10;
 
-struct NttLds {
-  uint4 lo[NTT_TILE];  // words 0-3 of each element
-  uint4 hi[NTT_TILE];  // words 4-7
+template <int LT>
+struct NttTile {
+  static constexpr int SIZE = 1 << LT;                      // elements per workgroup
+  static constexpr int THREADS = LT == NTT_LOG_TILE ? 512 : SIZE / 4;
+  static constexpr int HIGH_PASS = LT - 2;  // stages per pass above the low pass: runs >= 4
 };
 
-__device__ __forceinline__ void lds_put(NttLds& t, int e, const Fr& x) {
+template <int LT>
+struct NttLds {
+  uint4 lo[1 << LT];  // words 0-3 of each element
+  uint4 hi[1 << LT];  // words 4-7
+};
+
+template <int LT>
+__device__ __forceinline__ void lds_put(NttLds<LT>& t, int e, const Fr& x) {
   t.lo[e] = make_uint4(x.v[0], x.v[1], x.v[2], x.v[3]);
   t.hi[e] = make_uint4(x.v[4], x.v[5], x.v[6], x.v[7]);
 }
-__device__ __forceinline__ Fr lds_get(const NttLds& t, int e) {
+template <int LT>
+__device__ __forceinline__ Fr lds_get(const NttLds<LT>& t, int e) {
   const uint4 a = t.lo[e], b = t.hi[e];
   return {{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
 }
@@ -121,9 +135,10 @@ __device__ __forceinline__ Fr twiddle(const uint4* tw, int s0, int m, uint32_t k
 
 // The B stages of one tile in LDS (element e = k tlo + l). DIT: stages ascending,
 // (a, b) -> (a + b w, a - b w). DIF: descending, (a, b) -> (a + b, (a - b) w).
-template <bool DIF>
-__device__ __forceinline__ void tile_stages(NttLds& t, int lt, int s0, int B, uint32_t lo0,
+template <bool DIF, int LT>
+__device__ __forceinline__ void tile_stages(NttLds<LT>& t, int lt, int s0, int B, uint32_t lo0,
                                             const uint4* tw) {
+  constexpr int NTT_THREADS = NttTile<LT>::THREADS;
   const int tlo = 1 << lt, E = tlo << B;
   auto radix2 = [&](int m) {
     for (int u = threadIdx.x; u < E / 2; u += NTT_THREADS) {
@@ -239,20 +254,22 @@ struct NttVecs {
 // Where a pass reads and what it stores: src (nullptr: the pass works in place on data) read at
 // bit-reversed indices when brev is set (the first pass of a natural-order forward transform:
 // the permutation folded into its loads, out of place), and full = the stored values are a
-// transform's result (reduced below r).
+// transform's result (reduced below r), MODE 1's multiplied by *factor (R' form) when given.
 struct NttIo {
   const uint4* src = nullptr;
   int brev = 0;
   int full = 0;
+  const uint4* factor = nullptr;
 };
 
-template <int MODE>
-__global__ void __launch_bounds__(NTT_THREADS) k_ntt_pass(uint4* data, int L, int s0, int B,
+template <int MODE, int LT>
+__global__ void __launch_bounds__(NttTile<LT>::THREADS) k_ntt_pass(uint4* data, int L, int s0, int B,
                                                           int lt, const uint4* tw,
                                                           const uint4* prescale,
                                                           const uint4* tw2, NttVecs vs,
                                                           NttIo io) {
-  __shared__ NttLds t;
+  __shared__ NttLds<LT> t;
+  constexpr int NTT_THREADS = NttTile<LT>::THREADS;
   const int tlo = 1 << lt, E = tlo << B;  // elements in this tile
   const uint32_t tiles_lo = 1u << (s0 - lt);
   const uint32_t hi = blockIdx.x >> (s0 - lt);
@@ -271,16 +288,16 @@ __global__ void __launch_bounds__(NTT_THREADS) k_ntt_pass(uint4* data, int L, in
     lds_put(t, e, x);
   }
   __syncthreads();
-  if (MODE == 0) tile_stages<true>(t, lt, s0, B, lo0, tw);
-  if (MODE == 1 || MODE == 3) tile_stages<false>(t, lt, s0, B, lo0, tw);
+  if (MODE == 0) tile_stages<true, LT>(t, lt, s0, B, lo0, tw);
+  if (MODE == 1 || MODE == 3) tile_stages<false, LT>(t, lt, s0, B, lo0, tw);
   if (MODE == 2) {
-    tile_stages<true>(t, lt, s0, B, lo0, tw);
+    tile_stages<true, LT>(t, lt, s0, B, lo0, tw);
     for (int e = threadIdx.x; e < E; e += NTT_THREADS) {
       const size_t idx = base + ((size_t)(e >> lt) << s0) + (e & (tlo - 1));
       lds_put(t, e, tmul(lds_get(t, e), ldfr(prescale + 2 * idx)));
     }
     __syncthreads();
-    tile_stages<false>(t, lt, s0, B, lo0, tw2);
+    tile_stages<false, LT>(t, lt, s0, B, lo0, tw2);
   }
   for (int e = threadIdx.x; e < E; e += NTT_THREADS) {
     const int k = e >> lt, l = e & (tlo - 1);
@@ -293,70 +310,84 @@ __global__ void __launch_bounds__(NTT_THREADS) k_ntt_pass(uint4* data, int L, in
       uint4* h = vs.h + (((size_t)y << L) * 2);
       stfr(h + 2 * idx, sub(mul(ldfr(a + 2 * idx), ldfr(b + 2 * idx)), tfull(lds_get(t, e))));
     } else {
-      const Fr x = lds_get(t, e);
+      Fr x = lds_get(t, e);
+      if (MODE == 1 && io.factor) x = tmul(x, ldfr(io.factor));
       stfr(v + 2 * idx, io.full ? tfull(x) : x);
     }
   }
 }
 
 template <int MODE>
-static void launch_pass(void* data, int nvec, int L, int s0, int B, const void* tw,
+static void launch_pass(int log_tile, void* data, int nvec, int L, int s0, int B, const void* tw,
                         const void* prescale, const void* tw2, hipStream_t s,
                         NttVecs vs = NttVecs{}, NttIo io = NttIo{}) {
-  int lt = NTT_LOG_TILE - B;  // log2 of the consecutive lo per tile
+  int lt = log_tile - B;  // log2 of the consecutive lo per tile
   if (lt > s0) lt = s0;
   if (lt < 0) throw ArgError{"NTT pass of more stages than a tile holds"};
-  const uint32_t tiles = 1u << (L - B - lt);
-  hipLaunchKernelGGL(k_ntt_pass<MODE>, dim3(tiles, nvec), dim3(NTT_THREADS), 0, s,
-                     static_cast<uint4*>(data), L, s0, B, lt, static_cast<const uint4*>(tw),
-                     static_cast<const uint4*>(prescale), static_cast<const uint4*>(tw2), vs, io);
+  const dim3 grid(1u << (L - B - lt), nvec);
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, static_cast<uint4*>(data), L, s0, B, lt,
+                       static_cast<const uint4*>(tw), static_cast<const uint4*>(prescale),
+                       static_cast<const uint4*>(tw2), vs, io);
+  };
+  if (log_tile == NTT_LOG_TILE)
+    launch(k_ntt_pass<MODE, NTT_LOG_TILE>, NttTile<NTT_LOG_TILE>::THREADS);
+  else
+    launch(k_ntt_pass<MODE, NTT_LOG_TILE_SMALL>, NttTile<NTT_LOG_TILE_SMALL>::THREADS);
   G16_LAUNCH_CHECK("ntt pass");
 }
 
-// Pass plan: the lowest min(L, 12) stages in one pass over contiguous tiles; the stages above
-// in passes of at most NTT_HIGH_PASS, as equal as they can be.
-static int high_passes(int rest) { return (rest + NTT_HIGH_PASS - 1) / NTT_HIGH_PASS; }
-
-static int low_stages(int L) { return L < NTT_LOG_TILE ? L : NTT_LOG_TILE; }
-
-// Stages [low, L) in ascending passes: pass p covers [start(p), start(p + 1)).
-static int high_start(int L, int p) {
-  const int low = low_stages(L), rest = L - low, np = high_passes(rest);
-  return low + (rest * p) / np;
-}
+// Pass plan of nvec transforms of 2^L: the tile (log2 elements), the lowest min(L, tile) stages
+// in one pass over contiguous tiles, the stages above in np passes of at most HIGH_PASS, as
+// equal as they can be: pass p covers stages [start(p), start(p + 1)).
+struct NttPlan {
+  int tile, low, rest, np;
+  NttPlan(int L, int nvec) {
+    const bool small = L >= 12 && L <= 18 && ((uint64_t)nvec << L) < (1ull << 20);
+    tile = small ? NTT_LOG_TILE_SMALL : NTT_LOG_TILE;
+    const int hp = small ? NttTile<NTT_LOG_TILE_SMALL>::HIGH_PASS : NttTile<NTT_LOG_TILE>::HIGH_PASS;
+    low = L < tile ? L : tile;
+    rest = L - low;
+    np = (rest + hp - 1) / hp;
+  }
+  int start(int p) const { return low + (rest * p) / np; }
+};
 
 void ntt_dif_inverse(void* data, int nvec, int L, const void* tw, hipStream_t s) {
   if (L == 0) return;
-  const int np = high_passes(L - low_stages(L));
+  const NttPlan plan(L, nvec);
+  const int np = plan.np;
   for (int p = np - 1; p >= 0; --p) {
-    const int a = high_start(L, p), b = high_start(L, p + 1);
-    launch_pass<0>(data, nvec, L, a, b - a, tw, nullptr, nullptr, s);
+    const int a = plan.start(p), b = plan.start(p + 1);
+    launch_pass<0>(plan.tile, data, nvec, L, a, b - a, tw, nullptr, nullptr, s);
   }
-  launch_pass<0>(data, nvec, L, 0, low_stages(L), tw, nullptr, nullptr, s, NttVecs{},
+  launch_pass<0>(plan.tile, data, nvec, L, 0, plan.low, tw, nullptr, nullptr, s, NttVecs{},
                  NttIo{nullptr, 0, 1});
 }
 
 void ntt_dit_forward(void* data, int nvec, int L, const void* tw, const void* prescale,
-                     hipStream_t s, const void* natural_src, void* tmp) {
+                     hipStream_t s, const void* natural_src, void* tmp, const void* factor) {
   if (L == 0) {
     if (natural_src && natural_src != data)
       G16_CHECK(hipMemcpyAsync(data, natural_src, 32 * (size_t)nvec, hipMemcpyDeviceToDevice, s));
     if (prescale) launch_scale_rp(data, (size_t)nvec, prescale, s);  // n == 1: one factor
     return;
   }
-  const int np = high_passes(L - low_stages(L));
+  const NttPlan plan(L, nvec);
+  const int np = plan.np;
   // With natural_src, the first pass gathers it at bit-reversed indices into tmp (np > 0) or
   // into data (np == 0), and the high passes go from tmp back to data.
   void* first = natural_src ? (np > 0 ? tmp : data) : data;
-  launch_pass<1>(first, nvec, L, 0, low_stages(L), tw, prescale, nullptr, s, NttVecs{},
+  launch_pass<1>(plan.tile, first, nvec, L, 0, plan.low, tw, prescale, nullptr, s, NttVecs{},
                  NttIo{static_cast<const uint4*>(natural_src), natural_src ? 1 : 0,
-                       np == 0 ? 1 : 0});
+                       np == 0 ? 1 : 0, np == 0 ? static_cast<const uint4*>(factor) : nullptr});
   for (int p = 0; p < np; ++p) {
-    const int a = high_start(L, p), b = high_start(L, p + 1);
+    const int a = plan.start(p), b = plan.start(p + 1);
     const bool from_tmp = natural_src && p == 0;
-    launch_pass<1>(data, nvec, L, a, b - a, tw, nullptr, nullptr, s, NttVecs{},
+    launch_pass<1>(plan.tile, data, nvec, L, a, b - a, tw, nullptr, nullptr, s, NttVecs{},
                    NttIo{from_tmp ? static_cast<const uint4*>(tmp) : nullptr, 0,
-                         p == np - 1 ? 1 : 0});
+                         p == np - 1 ? 1 : 0,
+                         p == np - 1 ? static_cast<const uint4*>(factor) : nullptr});
   }
 }
 
@@ -365,29 +396,30 @@ void ntt_coset_pipeline(void* data, int nvec, int L, const void* tw_inv, const v
   const size_t n = (size_t)1 << L;
   if (h_out && nvec % 3) throw ArgError{"H from the transforms needs (A, B, C) triples"};
   uint4* v = static_cast<uint4*>(data);
-  const int np = L == 0 ? 0 : high_passes(L - low_stages(L));
+  const NttPlan plan(L, nvec);
+  const int np = L == 0 ? 0 : plan.np;
   if (L == 0) {
     launch_scale_rp(data, (size_t)nvec, coset, s);
   } else {
     for (int p = np - 1; p >= 0; --p) {
-      const int a = high_start(L, p), b = high_start(L, p + 1);
-      launch_pass<0>(data, nvec, L, a, b - a, tw_inv, nullptr, nullptr, s);
+      const int a = plan.start(p), b = plan.start(p + 1);
+      launch_pass<0>(plan.tile, data, nvec, L, a, b - a, tw_inv, nullptr, nullptr, s);
     }
     // Without high passes the fused pass is the last: its output is the result (and with
     // h_out the H below reads it fully reduced).
-    launch_pass<2>(data, nvec, L, 0, low_stages(L), tw_inv, coset, tw_fwd, s, NttVecs{},
+    launch_pass<2>(plan.tile, data, nvec, L, 0, plan.low, tw_inv, coset, tw_fwd, s, NttVecs{},
                    NttIo{nullptr, 0, np == 0 ? 1 : 0});
     for (int p = 0; p < np; ++p) {
-      const int a = high_start(L, p), b = high_start(L, p + 1);
+      const int a = plan.start(p), b = plan.start(p + 1);
       if (h_out && p == np - 1) {
         // Every A and B first (left below 2r: only the H pass reads them), then the C passes
         // store H from the final A and B.
         const int m = nvec / 3;
-        launch_pass<1>(data, 2 * m, L, a, b - a, tw_fwd, nullptr, nullptr, s, NttVecs{2, 0});
-        launch_pass<3>(data, m, L, a, b - a, tw_fwd, nullptr, nullptr, s,
+        launch_pass<1>(plan.tile, data, 2 * m, L, a, b - a, tw_fwd, nullptr, nullptr, s, NttVecs{2, 0});
+        launch_pass<3>(plan.tile, data, m, L, a, b - a, tw_fwd, nullptr, nullptr, s,
                        NttVecs{1, 2, static_cast<uint4*>(h_out)});
       } else {
-        launch_pass<1>(data, nvec, L, a, b - a, tw_fwd, nullptr, nullptr, s, NttVecs{},
+        launch_pass<1>(plan.tile, data, nvec, L, a, b - a, tw_fwd, nullptr, nullptr, s, NttVecs{},
                        NttIo{nullptr, 0, p == np - 1 ? 1 : 0});
       }
     }
@@ -445,34 +477,6 @@ void launch_coset_table(void* out, const void* shift, const void* scale, int L, 
                      static_cast<uint4*>(out), static_cast<const uint4*>(shift),
                      static_cast<const uint4*>(scale), L);
   G16_LAUNCH_CHECK("coset table");
-}
-
-__global__ void k_bitrev_permute(uint4* dst, const uint4* src, int L) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (1u << L)) return;
-  uint32_t j = bitrev(i, L);
-  dst[2 * (size_t)j] = src[2 * (size_t)i];
-  dst[2 * (size_t)j + 1] = src[2 * (size_t)i + 1];
-}
-
-void launch_bitrev_permute(void* dst, const void* src, int L, hipStream_t s) {
-  uint32_t n = 1u << L;
-  hipLaunchKernelGGL(k_bitrev_permute, dim3((n + 255) / 256), dim3(256), 0, s,
-                     static_cast<uint4*>(dst), static_cast<const uint4*>(src), L);
-  G16_LAUNCH_CHECK("bitrev permute");
-}
-
-__global__ void k_scale(uint4* data, size_t n, const uint4* fp) {
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  stfr(data + 2 * i, mul(ldfr(data + 2 * i), ldfr(fp)));
-}
-
-void launch_scale(void* data, size_t n, const void* factor, hipStream_t s) {
-  if (n == 0) return;
-  hipLaunchKernelGGL(k_scale, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                     static_cast<uint4*>(data), n, static_cast<const uint4*>(factor));
-  G16_LAUNCH_CHECK("scale");
 }
 
 __global__ void k_scale_rp(uint4* data, size_t n, const uint4* fp) {

@@ -382,7 +382,8 @@ struct HostTask {
 // ---- devices ---------------------------------------------------------------------------
 struct NttTables {
   // fwd, inv: per-pass twiddle tables (2^L - 1 entries); coset: shift^bitrev(p) / n; both in
-  // the R' = 2^261 form. scalars (R form): [w, w^-1, shift, 1/n, 1, 0, shift^-1, -1/(2n)].
+  // the R' = 2^261 form. scalars (R form): [w, w^-1, shift, 1/n, 1, 0, shift^-1, -1/(2n)],
+  // then 1/n in the R' form.
   // gnark (built for gnark-basis keys only): -shift^-bitrev(p) / (2n), R' form.
   DevBuf fwd, inv, coset, scalars, gnark;
 };
