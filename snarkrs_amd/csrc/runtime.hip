@@ -156,15 +156,13 @@ static Xyzz<F> run_msm_on(g16hip_device* d, int group, const void* bases, const 
   G16_CHECK(hipEventRecord(d->ev[0], d->stream));
   msm_to_msm_form(bases, sc.bases, coords, d->stream);
   msm_sort(plan, scalars, d->stream);
-  char* wout = static_cast<char*>(sc.accum) + msm_accum_scratch_bytes(plan, group);
-  msm_accumulate(plan, group, sc.bases, sc.accum, wout, d->stream, d->ev + 1);
-  std::vector<Xyzz<F>> S(npts);
-  uint32_t entries = 0;
-  G16_CHECK(hipMemcpyAsync(S.data(), wout, sizeof(Xyzz<F>) * npts, hipMemcpyDeviceToHost,
-                           d->stream));
-  G16_CHECK(hipMemcpyAsync(&entries, plan.total, 4, hipMemcpyDeviceToHost, d->stream));
+  if (npts > ROWS_POINTS) throw ArgError{"more reduction rows than the device's buffer holds"};
+  uint32_t* entries_at = reinterpret_cast<uint32_t*>(d->host_rows + ROWS_BYTES);
+  G16_CHECK(hipMemcpyAsync(entries_at, plan.total, 4, hipMemcpyDeviceToHost, d->stream));
+  msm_accumulate(plan, group, sc.bases, sc.accum, d->host_rows_dev, d->stream, d->ev + 1);
   G16_CHECK(hipEventRecord(d->ev[5], d->stream));
   G16_CHECK(hipStreamSynchronize(d->stream));
+  const uint32_t entries = *entries_at;
   g16hip_msm_stats& st = d->stats;
   st.sort_ms = ev_ms(d->ev[0], d->ev[1]);
   st.accumulate_ms = ev_ms(d->ev[1], d->ev[2]);
@@ -175,7 +173,7 @@ static Xyzz<F> run_msm_on(g16hip_device* d, int group, const void* bases, const 
   st.c = (uint32_t)c;
   st.windows = (uint32_t)plan.windows;
   note_accumulate(d, group, entries, st.accumulate_ms);
-  return msm_combine(S.data(), plan);
+  return msm_combine(reinterpret_cast<const Xyzz<F>*>(d->host_rows), plan);
 }
 
 // The same with scratch the device owns and grows as needed.
@@ -433,6 +431,9 @@ g16hip_status g16hip_open(int ordinal, g16hip_device** out) {
     G16_CHECK(hipSetDevice(ordinal));
     G16_CHECK(hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking));
     for (auto& e : d->ev) G16_CHECK(hipEventCreate(&e));
+    G16_CHECK(hipHostMalloc((void**)&d->host_rows, ROWS_BYTES + 64,
+                            hipHostMallocMapped | hipHostMallocCoherent));
+    G16_CHECK(hipHostGetDevicePointer((void**)&d->host_rows_dev, d->host_rows, 0));
     *out = d;
     return G16HIP_OK;
   });
@@ -451,6 +452,7 @@ void g16hip_close(g16hip_device* d) {
   d->scratch_e.release();
   for (auto& e : d->ev)
     if (e) (void)hipEventDestroy(e);
+  if (d->host_rows) (void)hipHostFree(d->host_rows);
   (void)hipStreamDestroy(d->stream);
   delete d;
 }

@@ -197,6 +197,29 @@ Pt<F> pt_add(const Pt<F>& p, const Pt<F>& q) {
   return r;
 }
 
+// 2^n p: Jacobian doublings (dbl-2009-l: 2 products and 5 squares against XYZZ's 6 and 3) between
+// two conversions: (X ZZ^2, Y ZZ^3, ZZZ) is the point's Jacobian form, since ZZ^3 = ZZZ^2.
+template <class F>
+Pt<F> pt_dbl_n(const Pt<F>& p, int n) {
+  if (n < 3 || is_zero(p.ZZ)) {
+    Pt<F> r = p;
+    for (int i = 0; i < n; ++i) r = pt_dbl(r);
+    return r;
+  }
+  const F zz2 = sqr(p.ZZ);
+  F X = mul(p.X, zz2), Y = mul(p.Y, mul(zz2, p.ZZ)), Z = p.ZZZ;
+  for (int i = 0; i < n; ++i) {
+    const F A = sqr(X), B = sqr(Y), C = sqr(B);
+    const F D = dbl(sub(sub(sqr(add(X, B)), A), C)), E = add(dbl(A), A);
+    const F X3 = sub(sqr(E), dbl(D));
+    Z = dbl(mul(Y, Z));
+    Y = sub(mul(E, sub(D, X3)), dbl(dbl(dbl(C))));
+    X = X3;
+  }
+  const F ZZ = sqr(Z);
+  return {X, Y, ZZ, mul(ZZ, Z)};
+}
+
 // Rows come off the MSM kernels in the R' = 2^261 Montgomery form, below 2q: x_R = x_R' / 32,
 // one R-form product by 2^251 (= 2^256 / 32) after a conditional subtraction of q.
 inline Fq from_msm_form(Fq x) {
@@ -288,42 +311,6 @@ Aff<G> host_to_aff(const Xyzz<G>& p) {
   return a;
 }
 
-// The MSM from the reduction's rows (msm_accumulate, in the kernels' R' form): sum over
-// windows w and rows j of 2^e P[w][j], e = c w for row 0 and c w + lg + j - 1 for row
-// j >= 1 — one Horner pass over the exponents, one doubling each (the reference finishes
-// sum_w 2^(cw) S_w on the host the same way, crates/cuda/src/msm.rs:3976-4010).
-template <class F>
-Xyzz<F> msm_combine(const Xyzz<F>* P, const MsmPlan& p) {
-  typedef typename hx::Of<F>::T H;
-  static_assert(sizeof(H) == sizeof(F), "host field layouts");
-  int rows, lg;
-  msm_reduce_shape(p, &rows, &lg);
-  const int c = p.c, W = msm_bucket_sets(p);  // one set when the windows are merged
-  int emax = c * (W - 1) + (rows > 1 ? lg + rows - 2 : 0);
-  std::vector<hx::Pt<H>> E((size_t)emax + 1, hx::Pt<H>{});
-  for (int w = 0; w < W; ++w)
-    for (int j = 0; j < rows; ++j) {
-      int e = c * w + (j == 0 ? 0 : lg + j - 1);
-      hx::Pt<H> q;
-      const Xyzz<F>& s = P[(size_t)w * rows + j];
-      std::memcpy(&q.X, &s.X, sizeof(H));
-      std::memcpy(&q.Y, &s.Y, sizeof(H));
-      std::memcpy(&q.ZZ, &s.ZZ, sizeof(H));
-      std::memcpy(&q.ZZZ, &s.ZZZ, sizeof(H));
-      q = {hx::from_msm_form(q.X), hx::from_msm_form(q.Y), hx::from_msm_form(q.ZZ),
-           hx::from_msm_form(q.ZZZ)};
-      E[e] = hx::pt_add(E[e], q);
-    }
-  hx::Pt<H> acc = E[emax];
-  for (int e = emax - 1; e >= 0; --e) acc = hx::pt_add(hx::pt_dbl(acc), E[e]);
-  Xyzz<F> out;
-  std::memcpy(&out.X, &acc.X, sizeof(H));
-  std::memcpy(&out.Y, &acc.Y, sizeof(H));
-  std::memcpy(&out.ZZ, &acc.ZZ, sizeof(H));
-  std::memcpy(&out.ZZZ, &acc.ZZZ, sizeof(H));
-  return out;
-}
-
 inline float ev_ms(hipEvent_t a, hipEvent_t b) {
   float ms = 0;
   G16_CHECK(hipEventElapsedTime(&ms, a, b));
@@ -379,6 +366,70 @@ struct HostTask {
   std::shared_ptr<State> st_;
 };
 
+// The MSM from the reduction's rows (msm_accumulate, in the kernels' R' form). Set w's sum is
+// S_w = row 0 + sum_j 2^(lg + j - 1) row j, the MSM sum_w 2^(c w) S_w: a Horner pass over the sets,
+// 255 doublings one after the other, which cost more than a small MSM's kernels (G2 of 1021
+// points: 340 us of 650). The sets' own sums, as many additions again, are taken by pooled
+// threads from the top set down, just ahead of the pass; whoever needs one that nobody has
+// begun does it itself. (The reference finishes sum_w 2^(cw) S_w on the host the same way,
+// crates/cuda/src/msm.rs:3976-4010.)
+template <class F>
+Xyzz<F> msm_combine(const Xyzz<F>* P, const MsmPlan& p) {
+  typedef typename hx::Of<F>::T H;
+  static_assert(sizeof(H) == sizeof(F), "host field layouts");
+  int rows, lg;
+  msm_reduce_shape(p, &rows, &lg);
+  const int c = p.c, W = msm_bucket_sets(p);  // one set when the windows are merged
+  const auto row = [&](int w, int j) {
+    hx::Pt<H> q;
+    const Xyzz<F>& s = P[(size_t)w * rows + j];
+    std::memcpy(&q.X, &s.X, sizeof(H));
+    std::memcpy(&q.Y, &s.Y, sizeof(H));
+    std::memcpy(&q.ZZ, &s.ZZ, sizeof(H));
+    std::memcpy(&q.ZZZ, &s.ZZZ, sizeof(H));
+    return hx::Pt<H>{hx::from_msm_form(q.X), hx::from_msm_form(q.Y), hx::from_msm_form(q.ZZ),
+                     hx::from_msm_form(q.ZZZ)};
+  };
+  const auto set_sum = [&](int w) {
+    hx::Pt<H> acc = row(w, rows - 1);
+    for (int j = rows - 2; j >= 0; --j)
+      acc = hx::pt_add(hx::pt_dbl_n(acc, j == 0 ? lg : 1), row(w, j));
+    return acc;
+  };
+  hx::Pt<H> acc{};
+  if (W * rows < 32) {
+    for (int w = W - 1; w >= 0; --w) acc = hx::pt_add(hx::pt_dbl_n(acc, c), set_sum(w));
+  } else {
+    enum { FREE, TAKEN, DONE };
+    std::vector<hx::Pt<H>> S((size_t)W);
+    std::unique_ptr<std::atomic<int>[]> state(new std::atomic<int>[(size_t)W]);
+    for (int w = 0; w < W; ++w) state[w].store(FREE, std::memory_order_relaxed);
+    const auto take = [&](int w) {
+      int want = FREE;
+      if (!state[w].compare_exchange_strong(want, TAKEN)) return;
+      S[w] = set_sum(w);
+      state[w].store(DONE, std::memory_order_release);
+    };
+    std::vector<std::unique_ptr<HostTask>> helpers;
+    for (int h = 0; h < 3; ++h)
+      helpers.push_back(std::make_unique<HostTask>([&] {
+        for (int w = W - 1; w >= 0; --w) take(w);
+      }));
+    for (int w = W - 1; w >= 0; --w) {
+      take(w);
+      while (state[w].load(std::memory_order_acquire) != DONE) std::this_thread::yield();
+      acc = hx::pt_add(hx::pt_dbl_n(acc, c), S[w]);
+    }
+    for (auto& h : helpers) h->join();
+  }
+  Xyzz<F> out;
+  std::memcpy(&out.X, &acc.X, sizeof(H));
+  std::memcpy(&out.Y, &acc.Y, sizeof(H));
+  std::memcpy(&out.ZZ, &acc.ZZ, sizeof(H));
+  std::memcpy(&out.ZZZ, &acc.ZZZ, sizeof(H));
+  return out;
+}
+
 // ---- devices ---------------------------------------------------------------------------
 struct NttTables {
   // fwd, inv: per-pass twiddle tables (2^L - 1 entries); coset: shift^bitrev(p) / n; both in
@@ -400,6 +451,10 @@ struct g16hip_device {
   g16::DevBuf msm_bases;  // the standalone MSM's bases in the MSM kernels' R' form
   std::map<int, std::unique_ptr<g16::NttTables>> ntt;
   hipEvent_t ev[6] = {};
+  // The standalone MSM's reduction rows and entry count: page-locked memory the kernels write
+  // (mapped into the device), as large as any width's rows (ROWS_BYTES), allocated at open.
+  uint8_t* host_rows = nullptr;
+  uint8_t* host_rows_dev = nullptr;
   g16hip_msm_stats stats = {};
   std::mutex stats_mu;
   g16hip_kernel_stats kstats = {};
@@ -444,6 +499,10 @@ inline void note_accumulate(g16hip_device* d, int group, uint64_t entries, doubl
 }
 
 inline void set_device(const g16hip_device* d) { G16_CHECK(hipSetDevice(d->ordinal)); }
+
+// Rows of a standalone MSM: at most 128 sets of one row (width 2), 29 of 8 (width 9) and the
+// like; 512 G2 points hold any.
+constexpr size_t ROWS_POINTS = 512, ROWS_BYTES = 256 * ROWS_POINTS;
 
 // Device scratch of one standalone MSM: the sort's, the accumulation's (window sums behind
 // it) and the bases in the MSM kernels' form.
