@@ -36,6 +36,69 @@ __device__ __forceinline__ void register_heavy(const TailJob& j, uint32_t k, uin
   }
 }
 
+// The bucket accumulation (accumulate_segment's work, a segment per point) for MSMs whose
+// segments fill little of the device at one lane each: an addition is 2-4 us deep instead of 5
+// (G1) or 13 (G2), at 2.2 (G1) and 2.0 (G2) times the work.
+template <bool G2>
+__global__ void __launch_bounds__(TAIL_BLOCK) k_accumulate_quad(const AccQueue q) {
+  using Q = Quad<G2>;
+  const AccQueueJob& j = q.job[blockIdx.y];
+  if (blockIdx.x == 0 && threadIdx.x < 4) j.cnt[threadIdx.x] = 0;
+  const uint64_t t = (uint64_t)blockIdx.x * (TAIL_BLOCK / Q::LANES) + Q::slot();
+  const uint64_t T = j.total[0], b = t * j.seg;
+  const bool alive = t < j.nseg && b < T;
+  const uint64_t e = !alive ? b : b + j.seg < T ? b + j.seg : T;
+  const uint32_t len = (uint32_t)(e - b);
+  uint32_t cur = alive ? j.ent[b].x : 0u;
+  bool starts = alive && (b == 0 || j.ent[b - 1].x != cur);
+  bool first = true;  // the run began at the segment's start
+  // Lanes 0 and 1 of a quad read the base's x and y.
+  const uint32_t at = (Q::coord() & 1u) * (Q::POINT_WORDS / 4) + Q::comp() * 2;
+  const auto fetch = [&](uint32_t i, uint2& en, uint4& lo, uint4& hi) {
+    en = j.ent[b + i];
+    const uint4* p = j.bases + (size_t)(en.y >> 1) * (Q::POINT_WORDS / 2) + at;
+    lo = p[0];
+    hi = p[1];
+  };
+  Coord acc = Q::inf();
+  uint2 en = make_uint2(0, 0);
+  uint4 lo = make_uint4(0, 0, 0, 0), hi = lo;
+  if (len) fetch(0, en, lo, hi);
+#pragma unroll 1
+  for (uint32_t i = 0; __any(i < len); ++i) {
+    const bool live = i < len;
+    if (live && en.x != cur) {
+      if (starts) Q::store(j.buckets, cur, acc);
+      else Q::store(j.pfirst, t, acc);
+      acc = Q::inf();
+      cur = en.x;
+      starts = true;
+      first = false;
+    }
+    const Coord p = Q::from_affine(lo, hi, (en.y & 1u) != 0, live);
+    if (i + 1 < len) fetch(i + 1, en, lo, hi);
+    acc = Q::add(acc, p);
+  }
+  if (!alive) return;
+  const bool ends = e == T || j.ent[e].x != cur;
+  if (starts && ends) {
+    Q::store(j.buckets, cur, acc);
+  } else {
+    if (first) Q::store(j.pfirst, t, acc);
+    Q::store(j.plast, t, acc);
+  }
+}
+
+void accumulate_quad_jobs(int group, const AccQueue& q, uint64_t nseg, hipStream_t s) {
+  const auto launch = [&](auto kernel, uint32_t points) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((nseg + points - 1) / points), q.n),
+                       dim3(TAIL_BLOCK), 0, s, q);
+  };
+  if (group == 1) launch(k_accumulate_quad<false>, TAIL_BLOCK / Quad<false>::LANES);
+  else launch(k_accumulate_quad<true>, TAIL_BLOCK / Quad<true>::LANES);
+  G16_LAUNCH_CHECK("msm accumulate (points over lanes)");
+}
+
 // Buckets that span segments, L points each: point i of a bucket adds every L-th of its pieces
 // (plast of its first segment, pfirst of the rest), then the L points add up. A bucket past
 // MERGE_SPAN pieces per point goes to the heavy path. Empty buckets become infinity; a bucket

@@ -315,6 +315,9 @@ struct AccQueue {
   int n;
 };
 
+// The jobs' accumulation with each segment's sum spread over lanes (kernels_msm_tail.hip).
+void accumulate_quad_jobs(int group, const AccQueue& q, uint64_t nseg, hipStream_t s);
+
 // One launch over jobs of the same segment count (blockIdx.y picks the job).
 template <class F>
 __global__ void __launch_bounds__(128) k_accumulate(const AccQueue q) {
@@ -864,7 +867,13 @@ inline void accumulate_jobs_impl(int group, const MsmPlan* const* plans, const v
   } else {
     uint64_t nseg = 1;  // at least one workgroup: it clears the counters
     for (int d = 0; d < n; ++d) nseg = std::max(nseg, q.job[d].nseg);
-    hipLaunchKernelGGL(k_accumulate<F>, dim3((unsigned)((nseg + 127) / 128), n), dim3(128), 0, s, q);
+    // Segments' sums over 4 (G1) or 8 (G2) lanes each while those lanes take at most two waves
+    // per SIMD: there they end sooner than one lane each (G1 MSM of 4099 points 351 -> 324 us,
+    // G2 of 1021 points 511 -> 444); at sixteen the device is full and the extra work shows
+    // (65k-constraint prove 1.38 -> 1.74 ms).
+    const uint64_t lanes = nseg * n * (group == 1 ? 4 : 8);
+    if (lanes <= 131072) accumulate_quad_jobs(group, q, nseg, s);
+    else hipLaunchKernelGGL(k_accumulate<F>, dim3((unsigned)((nseg + 127) / 128), n), dim3(128), 0, s, q);
   }
   G16_LAUNCH_CHECK("msm accumulate");
   if (ev) G16_CHECK(hipEventRecord(ev[1], s));

@@ -209,6 +209,24 @@ struct Quad {
     limbs29_of(w, r.v);
     return r;
   }
+  // The affine point whose x lanes 0 hold and whose y lanes 1 hold as words (any values on the
+  // other lanes), negated or not, with ZZ = ZZZ = 1; infinity for (0, 0) or where `live` is false.
+  static __device__ __forceinline__ Coord from_affine(const uint4& lo, const uint4& hi, bool negate,
+                                                      bool live) {
+    const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    const uint32_t l = coord();
+    Coord p;
+    limbs29_of(w, p.v);
+    const bool none = zero_at<0>(p) && zero_at<1>(p);
+    const Coord m = sub<Kq3>(inf(), p);  // 3q - y < 3q
+    p = coord_sel(l == 1 && negate, m, p);
+#pragma unroll
+    for (int j = 0; j < 9; ++j) {
+      const uint32_t one = comp() == 0 ? one29(j) : 0u;
+      p.v[j] = !live || none ? 0u : l >= 2 ? one : p.v[j];
+    }
+    return p;
+  }
   static __device__ __forceinline__ void put(uint4* base, size_t i, const Coord& x) {
     uint32_t w[8];
     pack29(x.v, w);
