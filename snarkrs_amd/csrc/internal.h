@@ -187,6 +187,14 @@ struct TailJobs {
 };
 void tail_merge_jobs(int group, const TailJobs& t, hipStream_t s);
 void tail_reduce_jobs(int group, const TailJobs& t, hipStream_t s);
+
+// Blinding products of `proofs` proofs: r delta1, s alpha1, r beta1, rs delta1 and s delta2 as
+// XYZZ points (R' form, below 2q) 256 bytes apart, from tables of 2^w P for w < 256 (XYZZ, R'
+// form: delta1, alpha1, beta1, then delta2) and each proof's standard-form r, s, rs.
+constexpr size_t BLIND_TABLE_BYTES = 256 * (3 * 128 + 256);
+constexpr size_t BLIND_SCALAR_BYTES = 96, BLIND_OUT_BYTES = 5 * 256;
+void launch_blind(const void* tables, const void* scalars, void* out, uint32_t proofs,
+                  hipStream_t s);
 void msm_reduce_shape(const MsmPlan& p, int* rows, int* lg);
 // The MSM kernels keep coordinates in Montgomery form with R' = 2^261 (bn254.cuh Fm): bases go
 // in as 32 x mod q. dst may equal src; n_fq counts 32-byte coordinates.

@@ -280,6 +280,54 @@ __global__ void __launch_bounds__(64) k_tail_slices(const TailJobs jobs) {
   }
 }
 
+// The stage-11 products of key points and blinders: block x of proof y sums the entries of its
+// point's table of 256 doublings (2^w P, XYZZ) at the scalar's set bits, as a chain of four (G2:
+// eight) additions per point of the block and a tree: 25 us (G1) and 50 us (G2) beside the
+// proof's other kernels (MI355X). On the host they were five double-and-add chains on the
+// calling thread, 600 us, longer than all the kernels of a 1000-constraint proof.
+//   x: 0 r delta1, 1 s alpha1, 2 r beta1, 3 rs delta1, 4 s delta2
+template <bool G2>
+__device__ __forceinline__ void blind_product(const uint4* table, const uint32_t* scalar,
+                                              uint4* out) {
+  using Q = Quad<G2>;
+  constexpr uint32_t POINTS = TAIL_BLOCK / Q::LANES;
+  const auto term = [&](uint32_t w) {
+    return w < 256 && ((scalar[w >> 5] >> (w & 31u)) & 1u) ? Q::load(table, w) : Q::inf();
+  };
+  uint32_t w = Q::slot();
+  Coord acc = term(w);
+  acc = Q::template block_sum<TAIL_BLOCK>(acc, [&](Coord& b) {
+    w += POINTS;
+    if (w - Q::slot() >= 256) return false;
+    b = term(w);
+    return true;
+  });
+  if (Q::slot() == 0) {
+    Q::store_out(out, 0, acc);
+    __threadfence_system();  // `out` is pinned host memory the host reads next
+  }
+}
+
+__global__ void __launch_bounds__(TAIL_BLOCK) k_blind(const uint4* tables,
+                                                      const uint32_t* scalars, uint4* out) {
+  const uint32_t x = blockIdx.x, y = blockIdx.y;
+  const uint32_t point[5] = {0, 1, 2, 0, 0}, which[5] = {0, 1, 0, 2, 1};
+  __shared__ uint32_t k[8];  // the scalar, read from host memory once
+  if (threadIdx.x < 8) k[threadIdx.x] = scalars[(y * 3 + which[x]) * 8 + threadIdx.x];
+  __syncthreads();
+  uint4* o = out + (size_t)(y * 5 + x) * 16;
+  if (x < 4) blind_product<false>(tables + point[x] * 256 * 8, k, o);
+  else blind_product<true>(tables + 3 * 256 * 8, k, o);
+}
+
+void launch_blind(const void* tables, const void* scalars, void* out, uint32_t proofs,
+                  hipStream_t s) {
+  hipLaunchKernelGGL(k_blind, dim3(5, proofs), dim3(TAIL_BLOCK), 0, s,
+                     static_cast<const uint4*>(tables), static_cast<const uint32_t*>(scalars),
+                     static_cast<uint4*>(out));
+  G16_LAUNCH_CHECK("blinding products");
+}
+
 template <class Fn>
 static uint32_t most(const TailJobs& t, Fn f) {
   uint32_t m = 0;

@@ -26,6 +26,8 @@ using namespace g16;
 
 namespace g16 {
 
+constexpr size_t BLIND_AT = 512;  // the blinding tables' offset behind NttTables::scalars
+
 struct Slot {
   hipStream_t stream = nullptr;
   hipStream_t side[2] = {nullptr, nullptr};
@@ -43,6 +45,7 @@ struct Slot {
   // here (no copy on the stream, which would wait for CUs behind other streams' kernels).
   uint8_t* host_wout = nullptr;
   uint8_t* host_wout_dev = nullptr;
+  size_t blind_at = 0;  // there: r, s, rs for the blinding products, then the products
   // Page-locked staging for a host witness: the caller's (pageable) witness is copied here in
   // chunks and each chunk goes up by DMA as soon as it is in (the reference's pinned witness
   // staging, crates/cuda/src/stages.rs:946-985).
@@ -135,6 +138,7 @@ struct g16hip_circuit {
   DevBuf row_ptr[2], signal[2], value_id[2], values;
   DevBuf a_q, b1_q, b2_q, l_q, h_q;
   NttTables tables;
+  char* blind_tables() const { return tables.scalars.as<char>() + g16::BLIND_AT; }
   size_t key_bytes = 0;
   std::mutex mu;
   std::condition_variable cv;
@@ -329,6 +333,15 @@ static void upload_key(g16hip_circuit* C, const g16hip_key* k, const KeyPlan& pl
     msm_window_tables(2, C->b2_q.p, nv, C->cw, Ww, s);
     msm_window_tables(1, C->h_q.p, nh, C->ch, Wh, s);
   }
+  // The blinding products' tables sit behind the transforms' few scalars, in the same page.
+  std::vector<uint8_t> blind(BLIND_TABLE_BYTES);
+  host_doublings(xyzz_from_aff(C->delta_g1), blind.data());
+  host_doublings(xyzz_from_aff(C->alpha_g1), blind.data() + 256 * 128);
+  host_doublings(xyzz_from_aff(C->beta_g1), blind.data() + 2 * 256 * 128);
+  host_doublings(xyzz_from_aff(C->delta_g2), blind.data() + 3 * 256 * 128);
+  C->tables.scalars.alloc(BLIND_AT + BLIND_TABLE_BYTES);
+  G16_CHECK(hipMemcpyAsync(C->blind_tables(), blind.data(), BLIND_TABLE_BYTES,
+                           hipMemcpyHostToDevice, s));
   build_ntt_tables(C->tables, C->log_n, s);
   if (C->h_basis == 1) build_gnark_h_table(C->tables, C->log_n, s);
   G16_CHECK(hipStreamSynchronize(s));
@@ -398,7 +411,8 @@ static void size_slot(const g16hip_circuit* C, Slot* S, bool fast) {
   S->accum_w2.alloc(msm_accum_scratch_bytes(S->plan_w, 2));
   S->accum_h.alloc(msm_accum_scratch_bytes(S->plan_h, 1));
   size_t wbytes = 256 * (4 * msm_out_points(S->plan_w) + msm_out_points(S->plan_h));
-  G16_CHECK(hipHostMalloc((void**)&S->host_wout, wbytes + 64,
+  S->blind_at = (wbytes + 64 + 255) / 256 * 256;
+  G16_CHECK(hipHostMalloc((void**)&S->host_wout, S->blind_at + 256 + BLIND_OUT_BYTES,
                           hipHostMallocMapped | hipHostMallocCoherent));
   G16_CHECK(hipHostGetDevicePointer((void**)&S->host_wout_dev, S->host_wout, 0));
   S->host_witness_bytes = 32 * nv;
@@ -768,15 +782,11 @@ static void finish_msms(const g16hip_circuit* C, Slot* S, bool per_msm_events,
 }
 
 // Eager run with events: timings, kernel statistics, the optional per-proof timeline.
-// `beside` runs on the calling thread once the GPU work is enqueued (host work that overlaps
-// it without a thread of its own).
 static void run_timed(g16hip_circuit* C, Slot* S, bool with_h, void* h, g16hip_msm_out* out,
-                      g16hip_timings* t, BlindProducts* blind, const Rows* rows = nullptr,
-                      const std::function<void()>& beside = nullptr) {
+                      g16hip_timings* t, BlindProducts* blind, const Rows* rows = nullptr) {
   enqueue_stages(C, S, with_h, h, true, rows);
   std::exception_ptr err;
   try {
-    if (beside) beside();
     finish_msms(C, S, true, out, blind);
   } catch (...) {
     err = std::current_exception();
@@ -833,8 +843,7 @@ static void run_timed(g16hip_circuit* C, Slot* S, bool with_h, void* h, g16hip_m
 // the graph; there are no memset nodes: every clear is a fill kernel), then replayed.
 // Replays go on the slot's own main stream, which lives as long as the graph: launching a
 // slot's graph on a stream that is destroyed before the graph's next launch is not done.
-static void run_graph(g16hip_circuit* C, Slot* S, g16hip_msm_out* out, BlindProducts* blind,
-                      const std::function<void()>& beside = nullptr) {
+static void run_graph(g16hip_circuit* C, Slot* S, g16hip_msm_out* out, BlindProducts* blind) {
   if (!S->exec) {
     G16_CHECK(hipStreamBeginCapture(S->stream, hipStreamCaptureModeThreadLocal));
     try {
@@ -849,14 +858,7 @@ static void run_graph(g16hip_circuit* C, Slot* S, g16hip_msm_out* out, BlindProd
     G16_CHECK(hipGraphInstantiate(&S->exec, S->graph, nullptr, nullptr, 0));
   }
   G16_CHECK(hipGraphLaunch(S->exec, S->stream));
-  std::exception_ptr err;
-  try {
-    if (beside) beside();
-  } catch (...) {
-    err = std::current_exception();
-  }
   G16_CHECK(hipStreamSynchronize(S->stream));
-  if (err) std::rethrow_exception(err);
   finish_msms(C, S, false, out, blind);
 }
 
@@ -865,8 +867,8 @@ static void run_graph(g16hip_circuit* C, Slot* S, g16hip_msm_out* out, BlindProd
 //   pi_a = A + alpha1 + r delta1,  pi_b = B2 + beta2 + s delta2,
 //   pi_c = L + H + s pi_a + r (B1 + beta1 + s delta1) - r s delta1
 //        = L + H + s A + r B1 + (s alpha1 + r beta1 + r s delta1).
-// The key-only terms are computed beside the GPU work; s A and r B1 as soon as those MSMs
-// finish. Group elements are canonical, so the proof is the same point whatever order the
+// The key-only products come from a kernel of their own beside the proof's (launch_blind); s A
+// and r B1 from the host as soon as those MSMs finish. Group elements are canonical, so the proof is the same point whatever order the
 // terms are added in.
 // ---------------------------------------------------------------------------------------
 struct BlinderTerms {
@@ -874,14 +876,20 @@ struct BlinderTerms {
   G2X d2s;      // s delta2
 };
 
-static BlinderTerms blinder_terms(const g16hip_circuit* C, const Fr& r_std, const Fr& s_std,
-                                  const Fr& rs_std) {
+// A proof's standard-form r, s and rs where launch_blind reads them.
+static void put_blinders(uint8_t* at, const Fr& r_std, const Fr& s_std, const Fr& rs_std) {
+  std::memcpy(at, r_std.v, 32);
+  std::memcpy(at + 32, s_std.v, 32);
+  std::memcpy(at + 64, rs_std.v, 32);
+}
+
+// The terms from a proof's products (launch_blind).
+static BlinderTerms blinder_terms(const uint8_t* products) {
   BlinderTerms b;
-  b.d1r = host_mul(xyzz_from_aff(C->delta_g1), r_std.v);
-  b.k1 = host_add(host_add(host_mul(xyzz_from_aff(C->alpha_g1), s_std.v),
-                           host_mul(xyzz_from_aff(C->beta_g1), r_std.v)),
-                  host_mul(xyzz_from_aff(C->delta_g1), rs_std.v));
-  b.d2s = host_mul(xyzz_from_aff(C->delta_g2), s_std.v);
+  b.d1r = host_row<Fq>(products);
+  b.k1 = host_add(host_add(host_row<Fq>(products + 256), host_row<Fq>(products + 512)),
+                  host_row<Fq>(products + 768));
+  b.d2s = host_row<Fq2>(products + 1024);
   return b;
 }
 
@@ -925,18 +933,21 @@ static void prove_on_slot(g16hip_circuit* C, Slot* S, const void* w, size_t n, b
   bp.r_std = to_std(r);
   bp.s_std = to_std(s);
   Fr rs_std = to_std(mul(r, s));
-  BlinderTerms terms;
-  const std::function<void()> beside = [&] { terms = blinder_terms(C, bp.r_std, bp.s_std, rs_std); };
+  // On the stream of B2, which the proof's end waits for, or on the graph's.
+  put_blinders(S->host_wout + S->blind_at, bp.r_std, bp.s_std, rs_std);
+  launch_blind(C->blind_tables(), S->host_wout_dev + S->blind_at,
+               S->host_wout_dev + S->blind_at + 256, 1,
+               graph && !rows ? S->stream : S->side[1]);
   g16hip_msm_out m;
   load_witness(C, S, w, n, on_device);
-  if (graph && !rows) run_graph(C, S, &m, &bp, beside);
-  else run_timed(C, S, true, S->hbuf.p, &m, t, &bp, rows, beside);
+  if (graph && !rows) run_graph(C, S, &m, &bp);
+  else run_timed(C, S, true, S->hbuf.p, &m, t, &bp, rows);
   if (on_device) {  // the slot's streams are synchronised: the copy has landed
     std::memcpy(w0.v, w0_pinned, 32);
     if (!is_one(w0)) throw StatusError{G16HIP_CONSTANT_WIRE, "w[0] is the constant-one wire and must be 1"};
   }
   Timer ta;
-  assemble(C, m, terms, bp, proof);
+  assemble(C, m, blinder_terms(S->host_wout + S->blind_at + 256), bp, proof);
   if (t) t->assemble_us += ta.us();
 }
 
@@ -998,6 +1009,13 @@ static size_t wave_rows_offset(const WavePlans& P, uint32_t cap, int j, uint32_t
 static size_t wave_rows_bytes(const WavePlans& P, uint32_t cap) {
   return wave_rows_offset(P, cap, 4, cap);
 }
+// Behind the rows: cap proofs' blinders, then their blinding products.
+static size_t wave_blind_at(const WavePlans& P, uint32_t cap) {
+  return (wave_rows_bytes(P, cap) + 255) / 256 * 256;
+}
+static size_t wave_products_at(const WavePlans& P, uint32_t cap) {
+  return wave_blind_at(P, cap) + ((size_t)cap * BLIND_SCALAR_BYTES + 255) / 256 * 256;
+}
 
 static size_t wave_bytes_for(const g16hip_circuit* C, uint32_t cap, bool fast) {
   static char anchor;  // bound only to size the pieces
@@ -1044,7 +1062,7 @@ static std::unique_ptr<Wave> make_wave(g16hip_circuit* C, uint32_t cap) {
   W->accum_g1[3].alloc(msm_accum_scratch_bytes(P.h, 1));
   W->accum_w2.alloc(msm_accum_scratch_bytes(P.w, 2));
   W->queue.alloc(256);
-  W->wout_bytes = wave_rows_bytes(P, cap);
+  W->wout_bytes = wave_products_at(P, cap) + cap * BLIND_OUT_BYTES;
   for (int b = 0; b < 2; ++b) {
     G16_CHECK(hipHostMalloc((void**)&W->host_wout[b], W->wout_bytes + 64,
                             hipHostMallocMapped | hipHostMallocCoherent));
@@ -1095,6 +1113,8 @@ static void wave_device(g16hip_circuit* C, Wave* W, uint32_t m, int b) {
                    rows + wave_rows_offset(P, cap, 2, 0), rows + wave_rows_offset(P, cap, 4, 0)};
   msm_accumulate_g1_queue(plans, bases, scratch, outs, 4, W->queue.as<uint32_t>(), s);
   msm_accumulate(P.w, 2, C->b2_q.p, W->accum_w2.p, rows + wave_rows_offset(P, cap, 3, 0), s);
+  launch_blind(C->blind_tables(), rows + wave_blind_at(P, cap), rows + wave_products_at(P, cap), m,
+               s);
 }
 
 // Copies the wave's witnesses into page-locked staging with a few host threads and enqueues one
@@ -1104,6 +1124,13 @@ static void enqueue_wave(g16hip_circuit* C, Wave* W, const std::vector<WaveItem>
   const size_t nv = C->n_vars, wb = 32 * nv;
   hipStream_t s = W->stream;
   uint8_t* stage = W->staging[b];
+  {
+    static char anchor;
+    const WavePlans P = wave_plans(C, &anchor, &anchor, m, W->cap, W->fast);
+    for (uint32_t k = 0; k < m; ++k)
+      put_blinders(W->host_wout[b] + wave_blind_at(P, W->cap) + BLIND_SCALAR_BYTES * k,
+                   to_std(it[k].r), to_std(it[k].s), to_std(mul(it[k].r, it[k].s)));
+  }
   {
     std::atomic<uint32_t> next{0};
     auto copy = [&] {
@@ -1171,7 +1198,8 @@ static void finish_wave(g16hip_circuit* C, Wave* W, const std::vector<WaveItem>&
       g1_store(mo.h_g1, host_to_aff(g1(4, k, P.vh)));
       bp.sA = host_mul(A, bp.s_std.v);
       bp.rB1 = host_mul(B1, bp.r_std.v);
-      const BlinderTerms terms = blinder_terms(C, bp.r_std, bp.s_std, to_std(mul(w.r, w.s)));
+      const BlinderTerms terms =
+          blinder_terms(rows + wave_products_at(P, cap) + BLIND_OUT_BYTES * k);
       assemble(C, mo, terms, bp, &proofs[w.index]);
       return G16HIP_OK;
     });

@@ -229,6 +229,11 @@ inline Fq from_msm_form(Fq x) {
 inline Fq2 from_msm_form(const Fq2& x) {
   return {from_msm_form(x.c0), from_msm_form(x.c1)};
 }
+inline Fq to_msm_form(Fq x) {  // x_R' = 32 x_R
+  for (int k = 0; k < 5; ++k) x = add(x, x);
+  return x;
+}
+inline Fq2 to_msm_form(const Fq2& x) { return {to_msm_form(x.c0), to_msm_form(x.c1)}; }
 
 template <class F> struct Of;
 template <> struct Of<g16::Fq> { typedef Fq T; };
@@ -279,6 +284,27 @@ Xyzz<G> out(const Pt<typename Of<G>::T>& q) {
 template <class G>
 Xyzz<G> host_add(const Xyzz<G>& a, const Xyzz<G>& b) {
   return hx::out<G>(hx::pt_add(hx::in(a), hx::in(b)));
+}
+
+// A point the MSM kernels wrote for the host (XYZZ, R' form, below 2q), and 2^w p for w < 256 as
+// they read it (w-th of `out`).
+template <class G>
+Xyzz<G> host_row(const void* at) {
+  Xyzz<G> p;
+  std::memcpy(&p, at, sizeof p);
+  const auto q = hx::in(p);
+  return hx::out<G>({hx::from_msm_form(q.X), hx::from_msm_form(q.Y), hx::from_msm_form(q.ZZ),
+                     hx::from_msm_form(q.ZZZ)});
+}
+template <class G>
+void host_doublings(const Xyzz<G>& p, uint8_t* out) {
+  auto q = hx::in(p);
+  for (int w = 0; w < 256; ++w) {
+    const Xyzz<G> e = hx::out<G>({hx::to_msm_form(q.X), hx::to_msm_form(q.Y),
+                                  hx::to_msm_form(q.ZZ), hx::to_msm_form(q.ZZZ)});
+    std::memcpy(out + sizeof e * w, &e, sizeof e);
+    q = hx::pt_dbl(q);
+  }
 }
 
 // k * p for a plain (standard-form) 256-bit scalar, double-and-add from the top bit.
