@@ -163,6 +163,7 @@ void msm_accumulate(const MsmPlan& p, int group, const void* bases, void* scratc
 // side (ev as msm_accumulate's). _queue: ONE persistent accumulation launch whose workgroups
 // take tiles of segments of every job from a device-side counter (a device word of the caller,
 // 16 bytes, cleared by a kernel here).
+// _together takes constant-work plans too.
 void msm_accumulate_g1_together(const MsmPlan& p, const void* const* bases, void* const* scratch,
                                 void* const* window_out, int n, hipStream_t s, hipEvent_t* ev);
 void msm_accumulate_g1_queue(const MsmPlan* const* plans, const void* const* bases,
@@ -186,7 +187,8 @@ struct TailJobs {
   int n;
 };
 void tail_merge_jobs(int group, const TailJobs& t, hipStream_t s);
-void tail_reduce_jobs(int group, const TailJobs& t, hipStream_t s);
+// `constant`: the buckets are projective and no branch follows the data.
+void tail_reduce_jobs(int group, bool constant, const TailJobs& t, hipStream_t s);
 
 // Blinding products of `proofs` proofs: r delta1, s alpha1, r beta1, rs delta1 and s delta2 as
 // XYZZ points (R' form, below 2q) 256 bytes apart, from tables of 2^w P for w < 256 (XYZZ, R'

@@ -763,8 +763,8 @@ size_t msm_sort_scratch_bytes(uint32_t n, int c, bool lean, uint32_t batch) {
 // same number of rounds of waves at the prove's sizes and the fold starts from half the slots
 // (47.8-47.9 against 47.4-47.5 proofs/s).
 // A segment is a chain of dependent additions on one lane, 5 us each in G1 and 13 in G2 while
-// the device is not full, so a variable-work MSM whose segments would not fill it halves them
-// until they do, down to 8 (G1 over per-window buckets: 10). MI355X: G1 MSM of 4099 points
+// the device is not full, so an MSM whose segments would not fill it halves them until they do,
+// down to 8 (G1 over per-window buckets: 10; constant work: 16, 20). MI355X: G1 MSM of 4099 points
 // 562 -> 405 us, G2 of 1021 points 956 -> 622, 22k-constraint prove 1035 -> 850, 65k resident
 // 1616 -> 1530. 131072 lanes for G1 gave 868 and 1576 on the last two; 32768 for G2 966 and
 // 1652, 131072 the same as 65536; segments of 4 gained 3 % on the two MSMs and lost as much on
@@ -772,10 +772,10 @@ size_t msm_sort_scratch_bytes(uint32_t n, int c, bool lean, uint32_t batch) {
 static constexpr size_t SEG_LANES[2] = {262144, 65536};  // G1: four waves per SIMD; G2: one
 
 static uint32_t segment_length(const MsmPlan& p, int g, size_t at_once) {
-  if (p.constant && p.merged) return 64u;
-  uint32_t seg = !p.merged && g == 0 ? 40u : 32u;
-  if (p.constant || !at_once) return seg;  // constant work, or the least scratch
-  while (seg >= 16 && at_once / seg < SEG_LANES[g]) seg /= 2;
+  uint32_t seg = p.constant && p.merged ? 64u : !p.merged && g == 0 ? 40u : 32u;
+  if (!at_once) return seg;  // the least scratch
+  const uint32_t halve = p.constant ? 32 : 16;  // a constant-work segment adds two fold slots
+  while (seg >= halve && at_once / seg < SEG_LANES[g]) seg /= 2;
   return seg;
 }
 
@@ -919,14 +919,8 @@ size_t msm_accum_scratch_bytes(const MsmPlan& p, int group) {
 }
 
 template <>
-void ConstTail<Fm>::fold(const AccumPtrs& a, hipStream_t s) {
-  tail_fold_const<Fm>(a, s);
-}
-
-template <>
-void ConstTail<Fm>::reduce(const MsmPlan& p, const AccumPtrs& a, uint32_t B, void* window_out,
-                           hipStream_t s) {
-  tail_reduce_ops<Fm, COps<Fm>>(p, a, B, window_out, s);
+void ConstTail<Fm>::fold(const ConstJobs& jobs, size_t nseg, int n, hipStream_t s) {
+  tail_fold_const<Fm>(jobs, nseg, n, s);
 }
 
 // Window tables: entry w n + i = 2^(c w) P_i from P_i at entry i, one thread per point.
@@ -985,6 +979,10 @@ void msm_accumulate_g1_queue(const MsmPlan* const* plans, const void* const* bas
 
 void msm_accumulate_g1_together(const MsmPlan& p, const void* const* bases, void* const* scratch,
                                 void* const* window_out, int n, hipStream_t s, hipEvent_t* ev) {
+  if (p.constant) {
+    accumulate_const_impl<Fm>(1, p, bases, scratch, window_out, n, s, ev);
+    return;
+  }
   const MsmPlan* plans[TAIL_JOBS];
   for (int k = 0; k < TAIL_JOBS; ++k) plans[k] = &p;
   accumulate_jobs_impl<Fm>(1, plans, bases, scratch, window_out, n, nullptr, 0, s, ev);
@@ -993,7 +991,6 @@ void msm_accumulate_g1_together(const MsmPlan& p, const void* const* bases, void
 void msm_accumulate(const MsmPlan& p, int group, const void* bases, void* scratch,
                     void* window_out, hipStream_t s, hipEvent_t* ev) {
   if (group == 2) msm_accumulate_g2(p, bases, scratch, window_out, s, ev);
-  else if (p.constant) accumulate_const_impl<Fm>(p, bases, scratch, window_out, s, ev);
   else msm_accumulate_g1_together(p, &bases, &scratch, &window_out, 1, s, ev);
 }
 

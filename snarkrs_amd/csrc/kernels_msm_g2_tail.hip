@@ -4,8 +4,8 @@
 namespace g16 {
 
 template <>
-void ConstTail<Fm2i>::fold(const AccumPtrs& a, hipStream_t s) {
-  tail_fold_const<Fm2i>(a, s);
+void ConstTail<Fm2i>::fold(const ConstJobs& jobs, size_t nseg, int n, hipStream_t s) {
+  tail_fold_const<Fm2i>(jobs, nseg, n, s);
 }
 
 }  // namespace g16

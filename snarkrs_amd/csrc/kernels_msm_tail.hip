@@ -203,7 +203,7 @@ __global__ void __launch_bounds__(TAIL_BLOCK) k_tail_heavy_finish(const TailJobs
 
 // Level 1 of the window reduction (see msm_accum.cuh): group g's T = sum_i B_{gB+i} and
 // U = sum_i (i+1) B_{gB+i}, one point per group, 2 (B - 1) additions.
-template <bool G2>
+template <bool G2, bool CW>
 __global__ void __launch_bounds__(TAIL_BLOCK) k_tail_groups(const TailJobs jobs) {
   using Q = Quad<G2>;
   const TailJob& j = jobs.job[blockIdx.y];
@@ -212,11 +212,14 @@ __global__ void __launch_bounds__(TAIL_BLOCK) k_tail_groups(const TailJobs jobs)
   if (blockIdx.x * (TAIL_BLOCK / Q::LANES) >= n) return;
   const uint32_t g = t < n ? t : n - 1;  // past the last group: repeat it, store nothing
   const size_t base = (size_t)g * j.B;
-  Coord run = Q::load(j.buckets, base + j.B - 1), acc = run;
+  const auto bucket = [&](size_t i) {
+    return CW ? Q::load_proj(j.buckets, i) : Q::load(j.buckets, i);
+  };
+  Coord run = bucket(base + j.B - 1), acc = run;
 #pragma unroll 1
   for (int i = 2 * (int)j.B - 3; i >= 0; --i) {  // odd: run += B_{i/2}; even: acc += run
-    const Coord next = Q::load(j.buckets, base + (uint32_t)(i >> 1));
-    const Coord r = Q::add((i & 1) ? run : acc, (i & 1) ? next : run);
+    const Coord next = bucket(base + (uint32_t)(i >> 1));
+    const Coord r = Q::template add<CW>((i & 1) ? run : acc, (i & 1) ? next : run);
     if (i & 1) run = r;
     else acc = r;
   }
@@ -228,7 +231,7 @@ __global__ void __launch_bounds__(TAIL_BLOCK) k_tail_groups(const TailJobs jobs)
 
 // Level 2: block x = ((w rows + r) S + slice) sums its slice of row r of set w; S = 1 writes
 // the host's row, else a slice sum for k_tail_slices.
-template <bool G2>
+template <bool G2, bool CW>
 __global__ void __launch_bounds__(TAIL_BLOCK) k_tail_rows(const TailJobs jobs) {
   using Q = Quad<G2>;
   const TailJob& j = jobs.job[blockIdx.y];
@@ -246,7 +249,7 @@ __global__ void __launch_bounds__(TAIL_BLOCK) k_tail_rows(const TailJobs jobs) {
   };
   uint32_t m = sl * per + Q::slot();
   Coord acc = m < m1 ? item(m) : Q::inf();
-  acc = Q::template block_sum<TAIL_BLOCK>(acc, [&](Coord& b) {
+  acc = Q::template block_sum<TAIL_BLOCK, CW>(acc, [&](Coord& b) {
     m += POINTS;
     if (!__any(m < m1)) return false;
     b = m < m1 ? item(m) : Q::inf();
@@ -260,7 +263,7 @@ __global__ void __launch_bounds__(TAIL_BLOCK) k_tail_rows(const TailJobs jobs) {
 }
 
 // Row x = w rows + r: out[x] = sum of parts[x S .. x S + S), one wave per row.
-template <bool G2>
+template <bool G2, bool CW>
 __global__ void __launch_bounds__(64) k_tail_slices(const TailJobs jobs) {
   using Q = Quad<G2>;
   const TailJob& j = jobs.job[blockIdx.y];
@@ -268,7 +271,7 @@ __global__ void __launch_bounds__(64) k_tail_slices(const TailJobs jobs) {
   uint32_t i = Q::slot();
   const size_t base = (size_t)blockIdx.x * j.S;
   Coord acc = i < j.S ? Q::load(j.parts, base + i) : Q::inf();
-  acc = Q::template block_sum<64>(acc, [&](Coord& b) {
+  acc = Q::template block_sum<64, CW>(acc, [&](Coord& b) {
     i += Q::WAVE_POINTS;
     if (!__any(i < j.S)) return false;
     b = i < j.S ? Q::load(j.parts, base + i) : Q::inf();
@@ -357,19 +360,19 @@ static void merge_jobs(const TailJobs& t, hipStream_t s) {
   G16_LAUNCH_CHECK("msm heavy finish");
 }
 
-template <bool G2>
+template <bool G2, bool CW>
 static void reduce_jobs(const TailJobs& t, hipStream_t s) {
   constexpr uint32_t per = TAIL_BLOCK / Quad<G2>::LANES;
   const uint32_t groups = most(t, [](const TailJob& j) { return j.sets * j.G; });
-  hipLaunchKernelGGL(k_tail_groups<G2>, dim3((groups + per - 1) / per, t.n), dim3(TAIL_BLOCK), 0,
+  hipLaunchKernelGGL((k_tail_groups<G2, CW>), dim3((groups + per - 1) / per, t.n), dim3(TAIL_BLOCK), 0,
                      s, t);
   G16_LAUNCH_CHECK("msm reduce groups");
   const uint32_t rows = most(t, [](const TailJob& j) { return j.sets * j.rows * j.S; });
-  hipLaunchKernelGGL(k_tail_rows<G2>, dim3(rows, t.n), dim3(TAIL_BLOCK), 0, s, t);
+  hipLaunchKernelGGL((k_tail_rows<G2, CW>), dim3(rows, t.n), dim3(TAIL_BLOCK), 0, s, t);
   G16_LAUNCH_CHECK("msm reduce rows");
   if (most(t, [](const TailJob& j) { return j.S; }) > 1) {
     const uint32_t sr = most(t, [](const TailJob& j) { return j.sets * j.rows; });
-    hipLaunchKernelGGL(k_tail_slices<G2>, dim3(sr, t.n), dim3(64), 0, s, t);
+    hipLaunchKernelGGL((k_tail_slices<G2, CW>), dim3(sr, t.n), dim3(64), 0, s, t);
     G16_LAUNCH_CHECK("msm reduce slices");
   }
 }
@@ -379,9 +382,9 @@ void tail_merge_jobs(int group, const TailJobs& t, hipStream_t s) {
   else merge_jobs<true>(t, s);
 }
 
-void tail_reduce_jobs(int group, const TailJobs& t, hipStream_t s) {
-  if (group == 1) reduce_jobs<false>(t, s);
-  else reduce_jobs<true>(t, s);
+void tail_reduce_jobs(int group, bool constant, const TailJobs& t, hipStream_t s) {
+  if (group == 1) constant ? reduce_jobs<false, true>(t, s) : reduce_jobs<false, false>(t, s);
+  else constant ? reduce_jobs<true, true>(t, s) : reduce_jobs<true, false>(t, s);
 }
 
 }  // namespace g16

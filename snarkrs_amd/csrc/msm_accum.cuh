@@ -348,14 +348,24 @@ static constexpr uint32_t FOLD_NONE = 0xFFFFFFFFu;
 static constexpr uint32_t FOLD_LEN = 8;
 static_assert(FOLD_LEN > 2, "each fold level must shrink the slot count");
 
+// One launch serves up to TAIL_JOBS MSMs over one plan's entries (blockIdx.y).
+struct ConstJob {
+  const uint4* bases;
+  uint4 *buckets, *fold[2];
+  uint32_t* rows[2];
+};
+struct ConstJobs {
+  ConstJob job[TAIL_JOBS];
+};
+
 template <class F>
 __global__ void __launch_bounds__(128) k_accumulate_const(const uint2* __restrict__ ent,
                                                           const uint32_t* total, size_t nseg,
-                                                          uint32_t seg,
-                                                          const uint4* __restrict__ bases,
-                                                          uint4* buckets, uint4* slots,
-                                                          uint32_t* rows) {
+                                                          uint32_t seg, const ConstJobs jobs) {
   using O = COps<F>;
+  const uint4* __restrict__ bases = jobs.job[blockIdx.y].bases;
+  uint4 *buckets = jobs.job[blockIdx.y].buckets, *slots = jobs.job[blockIdx.y].fold[0];
+  uint32_t* rows = jobs.job[blockIdx.y].rows[0];
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nseg) return;
   const size_t b = t * seg, T = total[0];  // the plan's entry count: b < T for t < nseg
@@ -397,12 +407,15 @@ __global__ void __launch_bounds__(128) k_accumulate_const(const uint2* __restric
 // (exactly FOLD_LEN iterations; past m it repeats the last slot as empty), adding runs of equal
 // rows. A run that ends inside the group, other than its first, is complete (all of a bucket's
 // pieces are consecutive) and goes to its bucket; the group's first and last runs go to slots
-// 2g and 2g + 1 of the next level (k_scan_const finishes the last few hundred slots).
+// 2g and 2g + 1 of the next level (k_scan_const takes over at ScanSlots::FROM slots).
 template <class F>
-__global__ void __launch_bounds__(128) k_fold_const(const uint4* in, const uint32_t* in_rows,
-                                                    uint32_t m, uint4* out, uint32_t* out_rows,
-                                                    uint4* buckets) {
+__global__ void __launch_bounds__(128) k_fold_const(const ConstJobs jobs, int from, uint32_t m) {
   using O = COps<F>;
+  const ConstJob& job = jobs.job[blockIdx.y];
+  const uint4* in = job.fold[from];
+  const uint32_t* in_rows = job.rows[from];
+  uint4 *out = job.fold[1 - from], *buckets = job.buckets;
+  uint32_t* out_rows = job.rows[1 - from];
   const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t groups = (m + FOLD_LEN - 1) / FOLD_LEN;
   if (g >= groups) return;
@@ -436,21 +449,33 @@ __global__ void __launch_bounds__(128) k_fold_const(const uint4* in, const uint3
   out_rows[2 * (size_t)g + 1] = (has_run && !first) ? cur : FOLD_NONE;
 }
 
-// The fold's end, for at most BLOCK slots: one workgroup, a slot per thread. The non-empty
-// slots are packed to the front in order (their rows stay sorted, so each bucket's pieces are
-// adjacent), then a segmented inclusive scan in LDS runs one addition per level for every
-// thread: at distance d a thread adds the value d slots back where that slot has its row (the
-// slots between belong to the same run) and keeps its own otherwise. The last slot of a run
-// then holds the run's sum and stores it to its bucket. The level count depends on m only.
+// The fold's end: a workgroup per BLOCK slots, a slot per thread. The non-empty slots are packed
+// to the front in order (their rows stay sorted, so each bucket's pieces are adjacent), then a
+// segmented inclusive scan in LDS runs one addition per level for every thread: at distance d a
+// thread adds the value d slots back where that slot has its row (the slots between belong to
+// the same run) and keeps its own otherwise. The last slot of a run then holds the run's sum and
+// stores it to its bucket; with several workgroups a workgroup's first and last runs go to
+// slots 2b and 2b + 1 of the next level instead, as a fold group's do. A level of 512 slots to 2
+// is 9 additions deep, where fold levels are 8 deep for a factor of 4, at 9 times their work; so
+// folds run down to FROM slots (G1 131072, G2 32768: a level there is as long on the device as it is deep). The level count depends on m only.
 // BLOCK: slots per scan, as many threads as the point form's registers allow in one workgroup.
 template <class F>
 struct ScanSlots {
-  static constexpr uint32_t N = sizeof(typename COps<F>::P) > 128 ? 256 : 512;
+  static constexpr bool G2 = sizeof(typename COps<F>::P) > 128;
+  static constexpr uint32_t N = G2 ? 256 : 512;
+  static constexpr uint32_t FROM = G2 ? 32768 : 131072;
 };
 
 template <class F, uint32_t BLOCK>
-__global__ void __launch_bounds__(BLOCK) k_scan_const(const uint4* in, const uint32_t* in_rows,
-                                                      uint32_t m, uint4* buckets) {
+__global__ void __launch_bounds__(BLOCK) k_scan_const(const ConstJobs jobs, int from,
+                                                      uint32_t count) {
+  const ConstJob& job = jobs.job[blockIdx.y];
+  const size_t at = (size_t)blockIdx.x * BLOCK;  // below count
+  const uint4* in = job.fold[from] + at * Words<F>::N * 4;
+  const uint32_t* in_rows = job.rows[from] + at;
+  uint4* buckets = job.buckets;
+  const uint32_t m = count - at < BLOCK ? (uint32_t)(count - at) : BLOCK;
+  const bool last_level = gridDim.x == 1;
   using O = COps<F>;
   using P = typename O::P;
   __shared__ P sh[BLOCK];
@@ -494,14 +519,21 @@ __global__ void __launch_bounds__(BLOCK) k_scan_const(const uint4* in, const uin
     v = O::sel(take, sum, v);
   }
   const bool end = r != FOLD_NONE && (i + 1 == BLOCK || rows[i + 1] != r);
-  if (end) O::store(buckets, r, v);
+  const bool head = !last_level && r == rows[0], tail = !last_level && !head && i + 1 == total;
+  const size_t slot = 2 * (size_t)blockIdx.x + (tail ? 1 : 0);
+  if (end) O::store(head || tail ? job.fold[1 - from] : buckets, head || tail ? slot : r, v);
+  if (!last_level && i < 2) {  // the next level's rows: first run, last run if another
+    const uint32_t first = total ? rows[0] : FOLD_NONE, last = total ? rows[total - 1] : FOLD_NONE;
+    job.rows[1 - from][2 * (size_t)blockIdx.x + i] =
+        i == 0 ? first : (last != first ? last : FOLD_NONE);
+  }
 }
 
 // Every bucket starts as the identity (a bucket no entry names is never stored).
 template <class F>
-__global__ void k_fill_proj_inf(uint4* buckets, size_t K) {
+__global__ void k_fill_proj_inf(const ConstJobs jobs, size_t K) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < K) POps<F>::store(buckets, i, POps<F>::inf());
+  if (i < K) POps<F>::store(jobs.job[blockIdx.y].buckets, i, POps<F>::inf());
 }
 
 // Several MSMs' bucket accumulations as one persistent launch over a device-side work queue:
@@ -533,16 +565,6 @@ __global__ void __launch_bounds__(QUEUE_TILE) k_accumulate_queue(AccQueue q, uin
 // Interior segments per heavy-bucket task (kernels_msm_tail.hip).
 static constexpr uint32_t HEAVY_TASK = 256;
 
-// Sum of BLOCK per-thread values in LDS, left in sh[0].
-template <class Ops, int BLOCK>
-__device__ __forceinline__ void block_tree(typename Ops::P* sh) {
-  for (int off = BLOCK / 2; off > 0; off >>= 1) {
-    __syncthreads();
-    if ((int)threadIdx.x < off) sh[threadIdx.x] = Ops::add(sh[threadIdx.x], sh[threadIdx.x + off]);
-  }
-  __syncthreads();
-}
-
 // ---------------------------------------------------------------------------------------
 // window reduction: S_w = sum_j (j+1) B_{w,j}
 // ---------------------------------------------------------------------------------------
@@ -550,75 +572,11 @@ __device__ __forceinline__ void block_tree(typename Ops::P* sh) {
 // U_g = sum_i (i+1) B_{gB+i},
 //   S_w = sum_g U_g + B sum_g g T_g = sum_g U_g + sum_k 2^(k+lg) Q_k,
 //   Q_k = sum of T_g over the g whose bit k is set.
-// Level 1 (one thread per group, 2B additions) makes T and U; level 2 is a plain sum per
-// (window, row) — row 0 sums U, row k+1 is Q_k. A row's items are cut into S slices (S a
-// power of two, at most 64, dividing every row's count), one workgroup each: strided
-// per-thread sums and an LDS tree; with S > 1 the slice sums go to `out` = a scratch array
-// and k_reduce_slices adds each row's S of them, so a long row (one bucket set of 2^15
-// buckets: 8192 groups) costs two short trees rather than one long strided chain. Every
-// chain is short; the doublings of the bit weights happen once, in the host's Horner pass
-// over all windows.
-template <class F, class Ops>
-__global__ void __launch_bounds__(128) k_reduce_groups(const uint4* buckets, uint32_t nb,
-                                                       int W, uint32_t B, uint4* T,
-                                                       uint4* U) {
-  uint32_t G = nb / B;
-  uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (uint32_t)W * G) return;
-  size_t base = (size_t)t * B;  // = w * nb + g * B
-  typename Ops::P run = Ops::inf(), acc = Ops::inf();
-  for (int i = (int)B - 1; i >= 0; --i) {
-    run = Ops::add(run, Ops::load(buckets, base + i));
-    acc = Ops::add(acc, run);
-  }
-  Ops::store(T, t, run);
-  Ops::store(U, t, acc);
-}
-
-// Workgroup x = ((w rows + r) S + slice); writes out[x] (the host's XYZZ when S = 1, else a
-// slice sum in the policy's form for k_reduce_slices).
-template <class F, int BLOCK, class Ops>
-__global__ void __launch_bounds__(BLOCK) k_reduce_rows(const uint4* T, const uint4* U,
-                                                       uint32_t G, uint32_t rows, uint32_t S,
-                                                       uint4* out) {
-  __shared__ typename Ops::P sh[BLOCK];
-  const uint32_t sl = blockIdx.x % S, wr = blockIdx.x / S;
-  const uint32_t w = wr / rows, r = wr % rows;
-  size_t base = (size_t)w * G;
-  typename Ops::P acc = Ops::inf();
-  const uint4* src = r == 0 ? U : T;
-  const uint32_t k = r == 0 ? 0 : r - 1, low = (1u << k) - 1u, count = r == 0 ? G : G / 2;
-  const uint32_t per = count / S, m0 = sl * per;
-  for (uint32_t m = m0 + threadIdx.x; m < m0 + per; m += BLOCK) {
-    // row 0: every g; row k + 1: m with a 1 inserted at bit k
-    const uint32_t g = r == 0 ? m : ((m & ~low) << 1) | (1u << k) | (m & low);
-    acc = Ops::add(acc, Ops::load(src, base + g));
-  }
-  sh[threadIdx.x] = acc;
-  block_tree<Ops, BLOCK>(sh);
-  if (threadIdx.x == 0) {
-    if (S == 1) st_xyzz(out, blockIdx.x, Ops::out(sh[0]));
-    else Ops::store(out, blockIdx.x, sh[0]);
-    __threadfence_system();  // `out` may be pinned host memory the host reads next
-  }
-}
-
-// Row x = w rows + r: out[x] = sum of parts[x S .. x S + S), in the host's XYZZ.
-template <class F, int BLOCK, class Ops>
-__global__ void __launch_bounds__(BLOCK) k_reduce_slices(const uint4* parts, uint32_t S,
-                                                         uint4* out) {
-  __shared__ typename Ops::P sh[BLOCK];
-  typename Ops::P acc = Ops::inf();
-  for (uint32_t i = threadIdx.x; i < S; i += BLOCK)
-    acc = Ops::add(acc, Ops::load(parts, (size_t)blockIdx.x * S + i));
-  sh[threadIdx.x] = acc;
-  block_tree<Ops, BLOCK>(sh);
-  if (threadIdx.x == 0) {
-    st_xyzz(out, blockIdx.x, Ops::out(sh[0]));
-    __threadfence_system();  // `out` may be pinned host memory the host reads next
-  }
-}
-
+// Level 1 makes T and U; level 2 is a plain sum per (window, row) — row 0 sums U, row k+1 is
+// Q_k. A row's items are cut into S slices (S a power of two that divides every row's count), one
+// workgroup each; with S > 1 the slice sums go to a scratch array and each row's S of them are
+// added after. Every chain is short; the doublings of the bit weights happen once, in the host's
+// pass over all windows (kernels_msm_tail.hip).
 inline uint32_t reduce_group_size(const MsmPlan& p) { return p.nb < 4 ? p.nb : 4; }
 inline int ilog2_u32(uint32_t x) {
   int l = 0;
@@ -626,26 +584,8 @@ inline int ilog2_u32(uint32_t x) {
   return l;
 }
 
-// Slices per row of G groups over `sets` bucket sets (constant work: one lane per point): rows
-// hold G or G / 2 items, at least 512 and 256 per slice, and no more than 256 workgroups of four
-// waves (one wave per SIMD): past that, waves share SIMDs and every tree level slows by as much
-// as slicing saves. In practice only a single bucket set (merged windows) is sliced.
-// Past 8192 groups (bucket sets of 2^15 and more: widths above 16) a row is cut into slices of
-// about 2048 groups, up to 256 per row, so that the row sums run across the device instead of
-// in a few long chains.
-inline uint32_t reduce_slices(uint32_t G, uint32_t sets) {
-  const uint32_t rows = 1 + (uint32_t)ilog2_u32(G);
-  uint32_t S = 1;
-  if (G > 8192) {
-    while (S < 256 && S * 2048 < G) S *= 2;
-    return S;
-  }
-  while (S < 64 && 2 * S * 512 <= G && (uint64_t)2 * S * rows * sets <= 256) S *= 2;
-  return S;
-}
-
-// The same where a point takes `lanes` lanes (k_tail_rows: 256 / lanes points per workgroup). A
-// slice costs its chain of additions and a tree of log2(points): with at least two items per
+// Slices per row of G groups over `sets` bucket sets, a point taking `lanes` lanes (k_tail_rows:
+// 256 / lanes points per workgroup). A slice costs its chain of additions and a tree of log2(points): with at least two items per
 // point while the device has room (512 workgroups), eight beyond.
 inline uint32_t tail_slices(uint32_t G, uint32_t sets, uint32_t lanes) {
   const uint32_t rows = 1 + (uint32_t)ilog2_u32(G), points = 256 / lanes;
@@ -685,8 +625,8 @@ inline AccumLayout accum_layout(const MsmPlan& p, size_t pt) {
     return r;
   };
   L.buckets = take(pt * K);
-  L.pfirst = take(pt * (nseg + 1));
-  L.plast = take(pt * (nseg + 1));
+  L.pfirst = take(p.constant ? 0 : pt * (nseg + 1));  // constant work keeps slots instead
+  L.plast = take(p.constant ? 0 : pt * (nseg + 1));
   L.heavy = take(12 * max_heavy);
   L.tasks = take(8 * max_tasks);
   L.task_sum = take(pt * max_tasks);
@@ -708,8 +648,8 @@ inline size_t msm_accum_scratch_bytes_impl(const MsmPlan& p, int group) {
 // Pointers into one accumulation's scratch.
 struct AccumPtrs {
   uint4 *buckets, *pfirst, *plast, *task_sum, *gT, *gU;
-  // The reduction's slice sums: S per row, in the segment partials' place (no longer needed by
-  // then), so S is cut to what they hold.
+  // The reduction's slice sums: S per row, in the place of the segment partials (constant work:
+  // the slots), no longer needed by then, so S is cut to what they hold.
   uint4* parts;
   uint32_t S;
   uint32_t *heavy, *tasks, *cnt;
@@ -719,63 +659,36 @@ struct AccumPtrs {
   size_t nseg;
 };
 
-// Launchers of the constant-work fold and reduction over field F. The G1 ones are defined here;
-// the G2 ones (F = Fm2i, products expanded in place so the latency-bound tail does not spill)
-// live in kernels_msm_g2_tail.hip and kernels_msm_g2_reduce.hip, so the slow G2 kernels
-// compile in parallel translation units.
+// Launches the constant-work fold of n jobs over field F. The G1 one is defined here; the G2 one
+// (F = Fm2i, products expanded in place so the latency-bound fold does not spill) lives in
+// kernels_msm_g2_tail.hip, so the slow G2 kernels compile in parallel translation units.
 template <class F>
 struct ConstTail {
-  static void fold(const AccumPtrs& a, hipStream_t s);
-  static void reduce(const MsmPlan& p, const AccumPtrs& a, uint32_t B, void* window_out,
-                     hipStream_t s);
+  static void fold(const ConstJobs& jobs, size_t nseg, int n, hipStream_t s);
 };
 
 template <class F>
-inline void tail_fold_const(const AccumPtrs& a, hipStream_t s) {
-  // Fold levels (2 nseg slots, then 2 per group of FOLD_LEN) until one workgroup's scan holds
-  // the rest.
+inline void tail_fold_const(const ConstJobs& jobs, size_t nseg, int n, hipStream_t s) {
+  // Fold levels (2 nseg slots, then 2 per group of FOLD_LEN), then scan levels (2 per
+  // workgroup), until one workgroup's scan holds the rest.
   constexpr uint32_t SCAN = ScanSlots<F>::N;
-  size_t m = fold_slots0(a.nseg);
+  size_t m = fold_slots0(nseg);
   if (m == 0) return;
-  const uint4* in = a.fold0;
-  const uint32_t* in_rows = a.frows0;
-  bool to1 = true;
-  while (m > SCAN) {
+  int from = 0;
+  for (; m > ScanSlots<F>::FROM; from = 1 - from) {
     const size_t groups = (m + FOLD_LEN - 1) / FOLD_LEN;
-    uint4* out = to1 ? a.fold1 : a.fold0;
-    uint32_t* out_rows = to1 ? a.frows1 : a.frows0;
-    hipLaunchKernelGGL(k_fold_const<F>, dim3((unsigned)((groups + 127) / 128)), dim3(128), 0, s,
-                       in, in_rows, (uint32_t)m, out, out_rows, a.buckets);
+    hipLaunchKernelGGL(k_fold_const<F>, dim3((unsigned)((groups + 127) / 128), n), dim3(128), 0, s,
+                       jobs, from, (uint32_t)m);
     G16_LAUNCH_CHECK("msm fold (constant work)");
-    in = out;
-    in_rows = out_rows;
     m = 2 * groups;
-    to1 = !to1;
   }
-  hipLaunchKernelGGL((k_scan_const<F, SCAN>), dim3(1), dim3(SCAN), 0, s, in, in_rows,
-                     (uint32_t)m, a.buckets);
-  G16_LAUNCH_CHECK("msm fold scan (constant work)");
-}
-
-template <class F, class Ops>
-inline void tail_reduce_ops(const MsmPlan& p, const AccumPtrs& a, uint32_t B, void* window_out,
-                            hipStream_t s) {
-  uint32_t G = p.nb / B;
-  uint32_t rows = 1 + (uint32_t)ilog2_u32(G);
-  const int sets = msm_bucket_sets(p);
-  uint32_t nthreads = (uint32_t)sets * G;
-  hipLaunchKernelGGL((k_reduce_groups<F, Ops>), dim3((nthreads + 127) / 128), dim3(128), 0, s,
-                     a.buckets, p.nb, sets, B, a.gT, a.gU);
-  G16_LAUNCH_CHECK("msm reduce groups");
-  const uint32_t S = a.S;
-  uint4* wout = static_cast<uint4*>(window_out);
-  hipLaunchKernelGGL((k_reduce_rows<F, 256, Ops>), dim3((unsigned)sets * rows * S), dim3(256), 0,
-                     s, a.gT, a.gU, G, rows, S, S > 1 ? a.parts : wout);
-  G16_LAUNCH_CHECK("msm reduce rows");
-  if (S > 1) {
-    hipLaunchKernelGGL((k_reduce_slices<F, 64, Ops>), dim3((unsigned)sets * rows), dim3(64), 0, s,
-                       a.parts, S, wout);
-    G16_LAUNCH_CHECK("msm reduce slices");
+  for (;; from = 1 - from) {
+    const size_t blocks = (m + SCAN - 1) / SCAN;
+    hipLaunchKernelGGL((k_scan_const<F, SCAN>), dim3((unsigned)blocks, n), dim3(SCAN), 0, s, jobs,
+                       from, (uint32_t)m);
+    G16_LAUNCH_CHECK("msm fold scan (constant work)");
+    if (blocks == 1) return;
+    m = 2 * blocks;
   }
 }
 
@@ -795,7 +708,6 @@ inline AccumPtrs accum_ptrs(const MsmPlan& p, void* scratch) {
   a.task_sum = reinterpret_cast<uint4*>(q + L.task_sum);
   a.gT = reinterpret_cast<uint4*>(q + L.gT);
   a.gU = reinterpret_cast<uint4*>(q + L.gU);
-  a.parts = a.pfirst;
   a.cnt = reinterpret_cast<uint32_t*>(q + L.cnt);
   a.fold0 = reinterpret_cast<uint4*>(q + L.fold0);
   a.frows0 = reinterpret_cast<uint32_t*>(q + L.frows0);
@@ -805,8 +717,9 @@ inline AccumPtrs accum_ptrs(const MsmPlan& p, void* scratch) {
   a.nseg = (p.max_entries + a.seg - 1) / a.seg;
   const uint32_t G = p.nb / reduce_group_size(p), sets = (uint32_t)msm_bucket_sets(p);
   const uint64_t rows = (uint64_t)(1 + ilog2_u32(G)) * sets;
-  a.S = p.constant ? reduce_slices(G, sets) : tail_slices(G, sets, PT == 128 ? 4 : 8);
-  while (a.S > 1 && a.S * rows > 2 * (a.nseg + 1)) a.S /= 2;
+  a.S = tail_slices(G, sets, PT == 128 ? 4 : 8);
+  a.parts = p.constant ? a.fold0 : a.pfirst;
+  while (a.S > 1 && a.S * rows > 2 * a.nseg) a.S /= 2;
   return a;
 }
 
@@ -879,32 +792,41 @@ inline void accumulate_jobs_impl(int group, const MsmPlan* const* plans, const v
   if (ev) G16_CHECK(hipEventRecord(ev[1], s));
   tail_merge_jobs(group, t, s);
   if (ev) G16_CHECK(hipEventRecord(ev[2], s));
-  tail_reduce_jobs(group, t, s);
+  tail_reduce_jobs(group, false, t, s);
   if (ev) G16_CHECK(hipEventRecord(ev[3], s));
 }
 
-// One constant-work MSM.
+// Up to TAIL_JOBS constant-work MSMs over one plan's entries, every launch over all of them.
 template <class F>
-inline void accumulate_const_impl(const MsmPlan& p, const void* bases, void* scratch,
-                                  void* window_out, hipStream_t s, hipEvent_t* ev) {
-  const AccumPtrs a = accum_ptrs<F>(p, scratch);
-  const uint32_t B = reduce_group_size(p);
-  auto bp = static_cast<const uint4*>(bases);
+inline void accumulate_const_impl(int group, const MsmPlan& p, const void* const* bases,
+                                  void* const* scratch, void* const* window_out, int n,
+                                  hipStream_t s, hipEvent_t* ev) {
+  if (n < 1 || n > TAIL_JOBS) throw ArgError{"accumulation of " + std::to_string(n) + " jobs"};
+  ConstJobs jobs{};
+  TailJobs t{};
+  t.n = n;
+  AccumPtrs a{};
+  for (int d = 0; d < n; ++d) {
+    a = accum_ptrs<F>(p, scratch[d]);
+    jobs.job[d] = ConstJob{static_cast<const uint4*>(bases[d]), a.buckets, {a.fold0, a.fold1},
+                           {a.frows0, a.frows1}};
+    t.job[d] = tail_job(p, a, window_out[d]);
+  }
   const unsigned grid = (unsigned)((a.nseg + 127) / 128);
   const size_t K = (size_t)msm_bucket_sets(p) * p.nb;
   if (ev) G16_CHECK(hipEventRecord(ev[0], s));
-  hipLaunchKernelGGL(k_fill_proj_inf<F>, dim3((unsigned)((K + 255) / 256)), dim3(256), 0, s,
-                     a.buckets, K);
+  hipLaunchKernelGGL(k_fill_proj_inf<F>, dim3((unsigned)((K + 255) / 256), n), dim3(256), 0, s,
+                     jobs, K);
   G16_LAUNCH_CHECK("msm buckets (constant work)");
   if (a.nseg) {
-    hipLaunchKernelGGL(k_accumulate_const<F>, dim3(grid), dim3(128), 0, s, p.ent, p.total,
-                       a.nseg, a.seg, bp, a.buckets, a.fold0, a.frows0);
+    hipLaunchKernelGGL(k_accumulate_const<F>, dim3(grid, n), dim3(128), 0, s, p.ent, p.total,
+                       a.nseg, a.seg, jobs);
     G16_LAUNCH_CHECK("msm accumulate (constant work)");
   }
   if (ev) G16_CHECK(hipEventRecord(ev[1], s));
-  ConstTail<F>::fold(a, s);
+  ConstTail<F>::fold(jobs, a.nseg, n, s);
   if (ev) G16_CHECK(hipEventRecord(ev[2], s));
-  ConstTail<F>::reduce(p, a, B, window_out, s);
+  tail_reduce_jobs(group, true, t, s);
   if (ev) G16_CHECK(hipEventRecord(ev[3], s));
 }
 

@@ -167,7 +167,9 @@ struct Quad {
   }
 
   // a + b. Every lane of the wave that reaches this takes part; the rare doubling or
-  // cancellation of any of them is resolved by all of them together.
+  // cancellation of any of them is resolved by all of them together. Constant work (CW)
+  // computes the doubling every time and picks the result by selects.
+  template <bool CW = false>
   static __device__ __forceinline__ Coord add(const Coord& a, const Coord& b) {
     const uint32_t l = coord();
     const bool ia = zero_at<2>(a), ib = zero_at<2>(b);
@@ -192,10 +194,10 @@ struct Quad {
     Coord r = coord_sel(l == 0, perm<1, 1, 1, 1>(X3), Y3);
     r = coord_sel(l == 2, t3, r);
     r = coord_sel(l == 3, t4, r);
-    if (__any(same_x)) {
+    if (CW || __any(same_x)) {
       const bool same_y = zero_at<1>(t2);
       const Coord d2 = dbl(a);
-      if (same_x) r = coord_sel(same_y, d2, inf());
+      r = coord_sel(same_x, coord_sel(same_y, d2, inf()), r);
     }
     r = coord_sel(ib, a, r);
     return coord_sel(ia, b, r);
@@ -226,6 +228,14 @@ struct Quad {
       p.v[j] = !live || none ? 0u : l >= 2 ? one : p.v[j];
     }
     return p;
+  }
+  // A constant-work slot (X, Y, Z, 0) of the point (X : Y : Z) as (X Z, Y Z^2, Z^2, Z^3).
+  static __device__ __forceinline__ Coord load_proj(const uint4* base, size_t i) {
+    const uint32_t l = coord();
+    const Coord a = load(base, i), z = perm<2, 2, 2, 2>(a);
+    const Coord t1 = mul(coord_sel(l == 3, z, a), z);  // X Z | Y Z | Z^2 | Z^2
+    const Coord t2 = mul(t1, z);                       // - | Y Z^2 | - | Z^3
+    return coord_sel((l & 1u) != 0, t2, t1);
   }
   static __device__ __forceinline__ void put(uint4* base, size_t i, const Coord& x) {
     uint32_t w[8];
@@ -264,7 +274,7 @@ struct Quad {
   // returns whether any point of the wave had one. Chain, tree across the wave and tree across
   // the waves share one addition site. Every lane of the block must arrive; the caller puts a
   // barrier before the next use.
-  template <int BLOCK, class Next>
+  template <int BLOCK, bool CW = false, class Next>
   static __device__ __forceinline__ Coord block_sum(Coord acc, Next next) {
     constexpr int WAVES = BLOCK / 64;
     __shared__ uint32_t sh[WAVES][9][LANES];
@@ -297,7 +307,7 @@ struct Quad {
         b = from_below(acc, off, q < off);
         off >>= 1;
       }
-      acc = add(acc, b);
+      acc = add<CW>(acc, b);
     }
     return acc;
   }

@@ -393,7 +393,7 @@ static void slot_plans(MsmPlan& w, MsmPlan& h, void* sort_w, void* sort_h, uint3
 // Bytes of a slot's G1 witness scratch: one MSM's, or three when they run together.
 static size_t accum_w1_bytes(const MsmPlan& w, bool fast) {
   const size_t one = (msm_accum_scratch_bytes(w, 1) + 255) & ~(size_t)255;
-  return fast && !w.constant && 3 * one <= TOGETHER_BYTES ? 3 * one : one;
+  return fast && 3 * one <= TOGETHER_BYTES ? 3 * one : one;
 }
 
 // Per-proof scratch for one slot, sized once so a proof allocates nothing.

@@ -66,3 +66,24 @@ def test_sort_of_small_msms(dev, n, constant):
         dev.set_constant_work(False)
     total = sum(k * s for k, s in zip(ks, ss)) % R_MOD
     assert (got == dev.fixed_base(1, fr_array([total]))[0]).all()
+
+
+@pytest.mark.parametrize("group,n", [(1, 33), (1, 1999), (1, 30011), (1, 65537), (2, 33),
+                                     (2, 1999), (2, 20011)])
+@pytest.mark.parametrize("same", [True, False])
+def test_constant_work_runs(dev, group, n, same):
+    # Runs that span several scan workgroups and fold groups (every scalar equal) or none, and the
+    # branch-free reduction over mostly empty buckets.
+    rng = SplitMix64(80 + n)
+    ks = [rng.next_fr() for _ in range(257)]
+    s0 = rng.next_fr()
+    ss = [s0] * n if same else [rng.next_fr() for _ in range(n)]
+    base = dev.fixed_base(group, fr_array(ks))
+    bases = base[[i % 257 for i in range(n)]]
+    dev.set_constant_work(True)
+    try:
+        got = dev.msm(group, bases, fr_array(ss))
+    finally:
+        dev.set_constant_work(False)
+    total = sum(ks[i % 257] * s for i, s in enumerate(ss)) % R_MOD
+    assert (got == dev.fixed_base(group, fr_array([total]))[0]).all()
