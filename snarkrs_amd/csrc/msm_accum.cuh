@@ -577,7 +577,13 @@ static constexpr uint32_t HEAVY_TASK = 256;
 // workgroup each; with S > 1 the slice sums go to a scratch array and each row's S of them are
 // added after. Every chain is short; the doublings of the bit weights happen once, in the host's
 // pass over all windows (kernels_msm_tail.hip).
-inline uint32_t reduce_group_size(const MsmPlan& p) { return p.nb < 4 ? p.nb : 4; }
+// Buckets per group. A group's chain is 2 (B - 1) additions and the rows' trees cost more per
+// point than chains do, so many sets of many buckets (a large standalone MSM) take 8: whole G1
+// MSM 2^20 1637 -> 1606 us, whole G2 MSM 2^18 1547 -> 1524 (MI355X).
+inline uint32_t reduce_group_size(const MsmPlan& p) {
+  const uint32_t B = !p.merged && (size_t)p.windows * p.nb >= 65536 ? 8u : 4u;
+  return p.nb < B ? p.nb : B;
+}
 inline int ilog2_u32(uint32_t x) {
   int l = 0;
   while ((2u << l) <= x) ++l;
@@ -585,8 +591,9 @@ inline int ilog2_u32(uint32_t x) {
 }
 
 // Slices per row of G groups over `sets` bucket sets, a point taking `lanes` lanes (k_tail_rows:
-// 256 / lanes points per workgroup). A slice costs its chain of additions and a tree of log2(points): with at least two items per
-// point while the device has room (512 workgroups), eight beyond.
+// 256 / lanes points per workgroup). A slice costs its chain of additions and a tree of
+// log2(points): with at least two items per point while the device has room (512 workgroups),
+// eight beyond.
 inline uint32_t tail_slices(uint32_t G, uint32_t sets, uint32_t lanes) {
   const uint32_t rows = 1 + (uint32_t)ilog2_u32(G), points = 256 / lanes;
   uint32_t S = 1;

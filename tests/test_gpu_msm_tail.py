@@ -87,3 +87,26 @@ def test_constant_work_runs(dev, group, n, same):
         dev.set_constant_work(False)
     total = sum(ks[i % 257] * s for i, s in enumerate(ss)) % R_MOD
     assert (got == dev.fixed_base(group, fr_array([total]))[0]).all()
+
+
+@pytest.mark.parametrize("group", [1, 2])
+@pytest.mark.parametrize("c", [2, 3, 4, 12, 13, 16])
+@pytest.mark.parametrize("constant", [False, True])
+def test_reduction_group_widths(dev, group, c, constant):
+    # Windows either side of 2^16 buckets in all (groups of 4 and of 8), and windows of fewer
+    # buckets than a group.
+    from snarkrs_amd.devmem import DeviceArray
+
+    n = 3001
+    rng = SplitMix64(60 + c)
+    ks = [rng.next_fr() for _ in range(n)]
+    ss = [rng.next_fr() if i % 5 else i % 2 for i in range(n)]
+    bases = DeviceArray(dev.fixed_base(group, fr_array(ks)))
+    scalars = DeviceArray(fr_array(ss))
+    dev.set_constant_work(constant)
+    try:
+        got = dev.msm_device(group, bases.addr, scalars.addr, n, c)
+    finally:
+        dev.set_constant_work(False)
+    total = sum(k * s for k, s in zip(ks, ss)) % R_MOD
+    assert (got == dev.fixed_base(group, fr_array([total]))[0]).all()
