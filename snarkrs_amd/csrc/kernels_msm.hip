@@ -12,7 +12,7 @@
 //               to side arrays and a merge pass folds them (heavy buckets, e.g. every 1
 //               scalar in bucket 0 of window 0, are cut into tasks summed by trees);
 //   4. reduce:  per window S_w = sum_j (j+1) B_j, as group sums and weighted group sums of
-//               4 buckets, then one tree per (window, bit of the group index); the host
+//               4 (or 8) buckets, then one tree per (window, bit of the group index); the host
 //               finishes with one Horner pass over every window and bit.
 // Merges and reduction (kernels_msm_tail.hip) work on points spread over lanes (msm_quad.cuh).
 // Zero scalars produce no entries and a scalar equal to 1 produces one (window 0, bucket 0),
@@ -686,7 +686,7 @@ static size_t align_up(size_t x) { return (x + 255) & ~(size_t)255; }
 // coarse bins at most MAX_CBINS), and chunks of SORT_CHUNK scalars, doubled until the count array
 // fits the scan (1024 SCAN_BLOCK), or halved, down to SORT_CHUNK_MIN, while the coarse kernels
 // would have under 256 workgroups (the counts' scratch grows; `lean` keeps SORT_CHUNK):
-// coarse count and scatter of H at 65k constraints 18 + 44 us with 32 workgroups, 6 + 13 with 256.
+// coarse count and scatter of H at 65k constraints 18 + 44 us with 32 workgroups, 8 + 14 with 256.
 struct SortGeom {
   int shift = 0;
   uint32_t cbins = 1, rows_per_set = 1, sets = 1, rows = 1, cs = SORT_CHUNK, chunks = 1;

@@ -4,7 +4,8 @@
 // additions once, not one after the other.
 //
 // What bounds these kernels is the length of their chains: a few hundred waves at most, each
-// addition waiting for the last. MI355X, one lane per point -> points over lanes, us:
+// addition waiting for the last. MI355X, one lane per point -> points over lanes, us
+// (reduction groups of 4; see reduce_group_size for the last two):
 //                                merge       heavy buckets   groups      rows and slices
 //   G1, 1000-constraint prove    34 -> 12    40 -> 31        47 -> 20    60 -> 24
 //   G2, 1000-constraint prove    91 -> 16    126 -> 46       140 -> 27   156 -> 44
@@ -38,7 +39,8 @@ __device__ __forceinline__ void register_heavy(const TailJob& j, uint32_t k, uin
 
 // The bucket accumulation (accumulate_segment's work, a segment per point) for MSMs whose
 // segments fill little of the device at one lane each: an addition is 2-4 us deep instead of 5
-// (G1) or 13 (G2), at 2.2 (G1) and 2.0 (G2) times the work.
+// (G1) or 13 (G2), with the slots of 16 products (G1) where a lane's mixed addition takes 10, and
+// the moves.
 template <bool G2>
 __global__ void __launch_bounds__(TAIL_BLOCK) k_accumulate_quad(const AccQueue q) {
   using Q = Quad<G2>;
@@ -285,9 +287,9 @@ __global__ void __launch_bounds__(64) k_tail_slices(const TailJobs jobs) {
 
 // The stage-11 products of key points and blinders: block x of proof y sums the entries of its
 // point's table of 256 doublings (2^w P, XYZZ) at the scalar's set bits, as a chain of four (G2:
-// eight) additions per point of the block and a tree: 25 us (G1) and 50 us (G2) beside the
-// proof's other kernels (MI355X). On the host they were five double-and-add chains on the
-// calling thread, 600 us, longer than all the kernels of a 1000-constraint proof.
+// eight) additions per point of the block and a tree: 57 us for the five products of 16 proofs,
+// 59-67 us beside one proof's other kernels (MI355X). On the host they were five double-and-add
+// chains on the calling thread, 600 us, longer than all the kernels of a 1000-constraint proof.
 //   x: 0 r delta1, 1 s alpha1, 2 r beta1, 3 rs delta1, 4 s delta2
 template <bool G2>
 __device__ __forceinline__ void blind_product(const uint4* table, const uint32_t* scalar,
