@@ -400,13 +400,22 @@ struct HostTask {
 // begun does it itself. (The reference finishes sum_w 2^(cw) S_w on the host the same way,
 // crates/cuda/src/msm.rs:3976-4010.)
 template <class F>
-Xyzz<F> msm_combine(const Xyzz<F>* P, const MsmPlan& p) {
+struct SetSums {
   typedef typename hx::Of<F>::T H;
   static_assert(sizeof(H) == sizeof(F), "host field layouts");
-  int rows, lg;
-  msm_reduce_shape(p, &rows, &lg);
-  const int c = p.c, W = msm_bucket_sets(p);  // one set when the windows are merged
-  const auto row = [&](int w, int j) {
+  enum { FREE, TAKEN, DONE };
+  const Xyzz<F>* P;  // the rows: read only between a FREE -> TAKEN step and its DONE
+  int W, rows, lg;
+  std::vector<hx::Pt<H>> S;
+  std::unique_ptr<std::atomic<int>[]> state;
+
+  SetSums(const Xyzz<F>* rows_at, const MsmPlan& p) : P(rows_at), W(msm_bucket_sets(p)) {
+    msm_reduce_shape(p, &rows, &lg);
+    S.resize((size_t)W);
+    state.reset(new std::atomic<int>[(size_t)W]);
+    for (int w = 0; w < W; ++w) state[w].store(FREE, std::memory_order_relaxed);
+  }
+  hx::Pt<H> row(int w, int j) const {
     hx::Pt<H> q;
     const Xyzz<F>& s = P[(size_t)w * rows + j];
     std::memcpy(&q.X, &s.X, sizeof(H));
@@ -415,38 +424,60 @@ Xyzz<F> msm_combine(const Xyzz<F>* P, const MsmPlan& p) {
     std::memcpy(&q.ZZZ, &s.ZZZ, sizeof(H));
     return hx::Pt<H>{hx::from_msm_form(q.X), hx::from_msm_form(q.Y), hx::from_msm_form(q.ZZ),
                      hx::from_msm_form(q.ZZZ)};
-  };
-  const auto set_sum = [&](int w) {
+  }
+  hx::Pt<H> sum(int w) const {
     hx::Pt<H> acc = row(w, rows - 1);
     for (int j = rows - 2; j >= 0; --j)
       acc = hx::pt_add(hx::pt_dbl_n(acc, j == 0 ? lg : 1), row(w, j));
     return acc;
-  };
+  }
+  void take(int w) {
+    int want = FREE;
+    if (!state[w].compare_exchange_strong(want, TAKEN)) return;
+    S[w] = sum(w);
+    state[w].store(DONE, std::memory_order_release);
+  }
+};
+
+// One queued or running helper of msm_combine, of the process's few: every thread that finishes
+// a proof of a wave would ask for three.
+struct CombineHelp {
+  static constexpr int MOST = 8;
+  static inline std::atomic<int> in_use{0};
+  CombineHelp() { ++in_use; }
+  CombineHelp(const CombineHelp&) = delete;
+  CombineHelp& operator=(const CombineHelp&) = delete;
+  ~CombineHelp() { --in_use; }
+};
+
+template <class F>
+Xyzz<F> msm_combine(const Xyzz<F>* P, const MsmPlan& p) {
+  typedef typename SetSums<F>::H H;
+  const auto sums = std::make_shared<SetSums<F>>(P, p);
+  const int c = p.c, W = sums->W;  // one set when the windows are merged
   hx::Pt<H> acc{};
-  if (W * rows < 32) {
-    for (int w = W - 1; w >= 0; --w) acc = hx::pt_add(hx::pt_dbl_n(acc, c), set_sum(w));
+  if (W * sums->rows < 32) {
+    for (int w = W - 1; w >= 0; --w) acc = hx::pt_add(hx::pt_dbl_n(acc, c), sums->sum(w));
   } else {
-    enum { FREE, TAKEN, DONE };
-    std::vector<hx::Pt<H>> S((size_t)W);
-    std::unique_ptr<std::atomic<int>[]> state(new std::atomic<int>[(size_t)W]);
-    for (int w = 0; w < W; ++w) state[w].store(FREE, std::memory_order_relaxed);
-    const auto take = [&](int w) {
-      int want = FREE;
-      if (!state[w].compare_exchange_strong(want, TAKEN)) return;
-      S[w] = set_sum(w);
-      state[w].store(DONE, std::memory_order_release);
-    };
-    std::vector<std::unique_ptr<HostTask>> helpers;
-    for (int h = 0; h < 3; ++h)
-      helpers.push_back(std::make_unique<HostTask>([&] {
-        for (int w = W - 1; w >= 0; --w) take(w);
-      }));
-    for (int w = W - 1; w >= 0; --w) {
-      take(w);
-      while (state[w].load(std::memory_order_acquire) != DONE) std::this_thread::yield();
-      acc = hx::pt_add(hx::pt_dbl_n(acc, c), S[w]);
+    // Nothing waits for a helper that has not begun: the pass ends with every sum taken, the
+    // helpers share the state's ownership, and one that starts later finds nothing to take and
+    // never reads the rows. Without a helper (none left, no thread to be had) the pass does all
+    // of them.
+    try {
+      for (int h = 0; h < 3 && CombineHelp::in_use.load() < CombineHelp::MOST; ++h) {
+        const auto help = std::make_shared<CombineHelp>();
+        host_pool_run([sums, help] {
+          for (int w = sums->W - 1; w >= 0; --w) sums->take(w);
+        });
+      }
+    } catch (...) {
     }
-    for (auto& h : helpers) h->join();
+    for (int w = W - 1; w >= 0; --w) {
+      sums->take(w);
+      while (sums->state[w].load(std::memory_order_acquire) != SetSums<F>::DONE)
+        std::this_thread::yield();
+      acc = hx::pt_add(hx::pt_dbl_n(acc, c), sums->S[w]);
+    }
   }
   Xyzz<F> out;
   std::memcpy(&out.X, &acc.X, sizeof(H));
