@@ -21,6 +21,11 @@
 #include "bn254.cuh"
 #include "internal.h"
 
+// The moves below must stay moves: see the Makefile's NEEDED.
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(G16_NO_DPP_COMBINE)
+#error "compile with -mllvm -amdgpu-dpp-combine=0 -DG16_NO_DPP_COMBINE"
+#endif
+
 namespace g16 {
 
 template <int CTRL>
