@@ -206,7 +206,7 @@ struct KeyPlan {
   bool merged = false;
   size_t key_bytes = 0, slot_bytes = 0;  // slot_bytes: the least scratch a slot works with
   size_t fast_slot_bytes = 0;            // with short segments and shared launches
-  bool fast = false;                     // the budget holds those
+  bool fast = false;                     // the budget keeps SPARE_BYTES free after those
   size_t total() const { return key_bytes + slot_bytes; }
 };
 
@@ -247,23 +247,25 @@ static KeyPlan plan_key(const g16hip_key* k, bool merged, bool constant) {
   return P;
 }
 
-// Window tables take W times the bases' memory; they are used when the device keeps 8 GiB of
-// its budget free after the key and a slot (G16HIP_WINDOW_TABLES=0 turns them off). A key
-// that does not fit even without them is refused before anything is allocated.
+// Window tables take W times the bases' memory, and a slot of short segments and shared launches
+// up to half a GiB more than the least; each is used when the device keeps SPARE_BYTES of its
+// budget free after the key and that slot (G16HIP_WINDOW_TABLES=0 turns the tables off), so that
+// neither takes the room of what comes next. A key that does not fit without both is refused
+// before anything is allocated.
 static KeyPlan choose_plan(const g16hip_device* d, const g16hip_key* k) {
   const size_t budget = device_budget(d);
   const char* wt = std::getenv("G16HIP_WINDOW_TABLES");
   if (!(wt && wt[0] == '0')) {
     KeyPlan P = plan_key(k, true, d->constant_work);
-    if (P.total() + (8ull << 30) <= budget) {
-      P.fast = P.key_bytes + P.fast_slot_bytes <= budget;
+    if (P.total() + SPARE_BYTES <= budget) {
+      P.fast = P.key_bytes + P.fast_slot_bytes + SPARE_BYTES <= budget;
       return P;
     }
   }
   KeyPlan P = plan_key(k, false, d->constant_work);
   if (P.total() > budget)
     throw too_big(P.total(), budget, "this key's resident data and one proof's stage scratch");
-  P.fast = P.key_bytes + P.fast_slot_bytes <= budget;
+  P.fast = P.key_bytes + P.fast_slot_bytes + SPARE_BYTES <= budget;
   return P;
 }
 
@@ -447,7 +449,7 @@ static size_t slot_bytes_estimate(const g16hip_circuit* C, bool fast) {
   return slot_bytes_for(C->n_vars, C->domain, C->n_h, C->cw, C->ch, C->merged, C->constant, fast);
 }
 
-static bool try_add_slot(g16hip_circuit* C, size_t reserve);
+static bool try_add_slot(g16hip_circuit* C, size_t reserve, uint32_t more);
 
 // Exclusive use of one of the circuit's slots. Waits for a free one; with `cap` > 0, first
 // adds a slot (up to `cap` in all, while the device keeps `reserve` bytes free) when every
@@ -464,10 +466,11 @@ struct SlotLease {
       if (idx < C->busy.size()) break;
       if (C->slots.size() + C->growing < cap) {
         C->growing++;
+        const uint32_t more = cap - (uint32_t)(C->slots.size() + C->growing);
         lk.unlock();
         bool added = false;
         try {
-          added = try_add_slot(C, reserve);
+          added = try_add_slot(C, reserve, more);
         } catch (...) {
           lk.lock();
           C->growing--;
@@ -1042,10 +1045,11 @@ static uint32_t wave_cap_of(const g16hip_circuit* C) {
   return cap ? cap : default_wave_cap(C);
 }
 
-// Builds a wave for cap proofs, refused before allocating when the device budget cannot hold it.
+// Builds a wave for cap proofs, refused before allocating when the device budget cannot hold it;
+// with short segments where SPARE_BYTES stay free after them.
 static std::unique_ptr<Wave> make_wave(g16hip_circuit* C, uint32_t cap) {
   const size_t budget = device_budget(C->dev);
-  const bool fast = wave_bytes_for(C, cap, true) <= budget;
+  const bool fast = wave_bytes_for(C, cap, true) + SPARE_BYTES <= budget;
   const size_t need = wave_bytes_for(C, cap, fast);
   if (need > budget) throw too_big(need, budget, "a wave of " + std::to_string(cap) + " proofs");
   auto W = std::make_unique<Wave>();
@@ -1298,11 +1302,14 @@ struct g16hip_server {
 namespace g16 {
 
 // Adds one slot to `C` if the device keeps `reserve` bytes free after it (admission by free
-// device memory); returns whether it did.
-static bool try_add_slot(g16hip_circuit* C, size_t reserve) {
-  const size_t budget = device_budget(C->dev);
-  if (budget < slot_bytes_estimate(C, false) + reserve) return false;
-  auto S = make_slot(C, budget >= slot_bytes_estimate(C, true) + reserve);
+// device memory); returns whether it did. It takes the larger scratch if SPARE_BYTES and the
+// least scratch of the `more` slots that may follow stay free besides, so that as many are
+// admitted as with the least.
+static bool try_add_slot(g16hip_circuit* C, size_t reserve, uint32_t more) {
+  const size_t budget = device_budget(C->dev), least = slot_bytes_estimate(C, false);
+  if (budget < least + reserve) return false;
+  auto S = make_slot(C, budget >= slot_bytes_estimate(C, true) + least * more + reserve +
+                                      SPARE_BYTES);
   std::lock_guard<std::mutex> lk(C->mu);
   C->slots.push_back(std::move(S));
   C->busy.push_back(false);
@@ -1459,7 +1466,7 @@ g16hip_status g16hip_circuit_add_slots(g16hip_circuit* C, uint32_t count, size_t
     if (!C) throw ArgError{"null circuit"};
     set_device(C->dev);
     for (uint32_t i = 0; i < count; ++i)
-      if (!try_add_slot(C, reserve_bytes)) break;
+      if (!try_add_slot(C, reserve_bytes, count - i - 1)) break;
     if (total_slots) {
       std::lock_guard<std::mutex> lk(C->mu);
       *total_slots = (uint32_t)C->slots.size();

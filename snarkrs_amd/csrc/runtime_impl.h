@@ -528,6 +528,9 @@ namespace g16 {
 // the reserve, capped by the device's limit (the reference's device_budget,
 // crates/cuda/src/msm.rs:1057-1091).
 constexpr size_t VRAM_HEADROOM = 256ull << 20;
+// Left free of the budget by what only makes proofs and MSMs faster: the window tables, the
+// scratch of short segments and shared launches.
+constexpr size_t SPARE_BYTES = 8ull << 30;
 inline size_t device_budget(const g16hip_device* d) {
   size_t free_b = 0, total_b = 0;
   G16_CHECK(hipMemGetInfo(&free_b, &total_b));

@@ -102,3 +102,36 @@ def test_key_over_the_vram_budget_is_refused_before_allocating(dev, orc):
         circ.release()
     finally:
         dev.set_vram_limit(0)
+
+
+def _slot_memory(dev, key, wit):
+    """Device bytes of a prepared key with its slot, of two more slots, and of its first wave."""
+    circ = dev.prepare(key)
+    try:
+        first = circ.resident_bytes()
+        assert circ.add_slots(2, reserve_bytes=0) == 3
+        more = circ.resident_bytes() - first
+        free = dev.mem_info()[0]
+        native.prove_batch([(circ, wit, *RS)] * 2)
+        return first, more, free - dev.mem_info()[0]
+    finally:
+        circ.release()
+
+
+def test_larger_scratch_only_while_memory_is_spare(dev, orc, monkeypatch):
+    # A budget that holds the larger scratch of short segments but not 8 GiB besides: slots and
+    # waves take the least, so that what is prepared next finds the room it found before.
+    monkeypatch.setenv("G16HIP_WINDOW_TABLES", "0")
+    syn = Synth(orc, 20_000, n_public=2, n_private_in=2000, bool_permille=300,
+                input_bool_permille=300, seed=97, setup_seed=98)
+    key, wit = syn.key()
+    need = native.key_resident_bytes(key, window_tables=False)
+    _slot_memory(dev, key, wit)  # what the runtime allocates with a first launch
+    roomy = _slot_memory(dev, key, wit)
+    try:
+        dev.set_vram_limit(need + (4 << 30))
+        short = _slot_memory(dev, key, wit)
+    finally:
+        dev.set_vram_limit(0)
+    assert short[0] <= need < roomy[0]
+    assert short[1] < roomy[1] and short[2] < roomy[2]
