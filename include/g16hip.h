@@ -150,9 +150,10 @@ g16hip_status g16hip_set_vram_limit(g16hip_device* dev, size_t bytes);
  * free memory less a 256 MiB headroom and the reserve, capped by the limit. */
 g16hip_status g16hip_device_budget(g16hip_device* dev, size_t* bytes);
 /* resident_bytes (crates/cuda/src/backend.rs:626-643): device bytes `key` and one proof slot take
- * once prepared, with (window_tables != 0) or without the per-window base tables, each buffer
- * rounded up to 2 MiB pages. g16hip_prepare uses the tables only when the budget keeps 8 GiB
- * free after them. */
+ * once prepared, each buffer rounded up to 2 MiB pages. With window_tables != 0: with the
+ * per-window base tables and the slot's larger scratch (short segments, shared launches), which
+ * g16hip_prepare uses when the budget keeps 8 GiB free after them. With 0: the least a key is
+ * prepared with, without either; under this it is refused. */
 g16hip_status g16hip_key_resident_bytes(const g16hip_key* key, int window_tables, size_t* bytes);
 
 /* Backend::prepare (crates/groth16/src/lib.rs:371-378): validates the key

@@ -1429,7 +1429,8 @@ g16hip_status g16hip_key_resident_bytes(const g16hip_key* key, int window_tables
   return guarded([&] {
     if (!bytes) throw ArgError{"null argument"};
     validate_key(key);
-    *bytes = plan_key(key, window_tables != 0, false).total();
+    const KeyPlan P = plan_key(key, window_tables != 0, false);
+    *bytes = window_tables ? P.key_bytes + P.fast_slot_bytes : P.total();
     return G16HIP_OK;
   });
 }

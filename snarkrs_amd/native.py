@@ -443,7 +443,8 @@ class Device:
 
 def key_resident_bytes(key: ProvingKey, window_tables: bool = False) -> int:
     """Device bytes ``key`` and one proof slot take once prepared (``resident_bytes``,
-    crates/cuda/src/backend.rs:626-643), with or without the per-window base tables."""
+    crates/cuda/src/backend.rs:626-643): with the per-window base tables and the slot's larger
+    scratch, used while the budget keeps 8 GiB free after them, or the least without either."""
     st = key.struct()
     b = ctypes.c_size_t()
     _check(load().g16hip_key_resident_bytes(ctypes.byref(st), int(window_tables), ctypes.byref(b)))

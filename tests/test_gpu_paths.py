@@ -135,3 +135,17 @@ def test_larger_scratch_only_while_memory_is_spare(dev, orc, monkeypatch):
         dev.set_vram_limit(0)
     assert short[0] <= need < roomy[0]
     assert short[1] < roomy[1] and short[2] < roomy[2]
+
+
+def test_key_and_slot_take_what_is_predicted(dev, orc):
+    syn = Synth(orc, 20_000, n_public=2, n_private_in=2000, bool_permille=300,
+                input_bool_permille=300, seed=99, setup_seed=100)
+    key, _ = syn.key()
+    predicted = native.key_resident_bytes(key, window_tables=True)
+    assert dev.budget() > predicted + (8 << 30), "the GPU is not free enough for the tables"
+    circ = dev.prepare(key)
+    try:
+        # every buffer may be up to a page of 2 MiB short of its share
+        assert predicted - 40 * (2 << 20) < circ.resident_bytes() <= predicted
+    finally:
+        circ.release()
