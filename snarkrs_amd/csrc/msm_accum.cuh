@@ -109,8 +109,7 @@ __device__ __forceinline__ void st_xyzz(uint4* base, size_t i, const Xyzz<F>& r)
 }
 
 // How the constant-work kernels see a point: (X : Y : Z) with the complete formulas (POps in
-// words; COps below runs them on limbs), stored in an XYZZ-sized slot as (X, Y, Z, 0). `out` is
-// the form the host reads (XYZZ).
+// words; COps below runs them on limbs), stored in an XYZZ-sized slot as (X, Y, Z, 0).
 template <class F>
 struct POps {
   using P = Proj<F>;
@@ -123,7 +122,6 @@ struct POps {
   static __device__ __forceinline__ void store(uint4* base, size_t i, const P& p) {
     st_xyzz(base, i, Xyzz<F>{p.X, p.Y, p.Z, f_zero<F>()});
   }
-  static __device__ __forceinline__ Xyzz<F> out(const P& p) { return proj_to_xyzz(p); }
   static __device__ __forceinline__ P sel(bool c, const P& a, const P& b) { return proj_sel(c, a, b); }
   static __device__ __forceinline__ P add_aff(const P& p, const Aff<F>& a) { return proj_add_aff(p, a); }
 };
@@ -144,9 +142,6 @@ struct COps<Fm2i> {
   static __device__ __forceinline__ void store(uint4* base, size_t i, const P& p) {
     POps<Fm2i>::store(base, i, p2l_out(p));
   }
-  static __device__ __forceinline__ Xyzz<Fm2i> out(const P& p) {
-    return proj_to_xyzz(p2l_out(p));
-  }
   static __device__ __forceinline__ P sel(bool c, const P& a, const P& b) { return p2l_sel(c, a, b); }
   static __device__ __forceinline__ P add_aff(const P& p, const Aff<Fm2i>& a) {
     F2L x, y;
@@ -166,7 +161,6 @@ struct COps<Fm> {
   static __device__ __forceinline__ void store(uint4* base, size_t i, const P& p) {
     POps<Fm>::store(base, i, p1l_out(p));
   }
-  static __device__ __forceinline__ Xyzz<Fm> out(const P& p) { return proj_to_xyzz(p1l_out(p)); }
   static __device__ __forceinline__ P sel(bool c, const P& a, const P& b) { return p1l_sel(c, a, b); }
   static __device__ __forceinline__ P add_aff(const P& p, const Aff<Fm>& a) {
     uint32_t x[9], y[9];

@@ -1,8 +1,8 @@
 // Host check of the limb-form point arithmetic (G1L, G2L, P1L, P2L in snarkrs_amd/csrc/bn254.cuh)
 // against the word-form XYZZ formulas of the same header: chains of mixed additions with
-// random signs, repeated points (doublings) and opposite points (cancellations), general
-// additions of such sums (including p + p and p + (-p)), and every value's bound after every
-// step (G1 X < 9q, G2 X < 5q, the rest < 2q, limbs as the header states); the complete
+// random signs, repeated points (doublings) and opposite points (cancellations), and every
+// value's bound after every step (G1 X < 9q, G2 X < 5q, the rest < 2q, limbs as the header
+// states); general additions are msm_quad.cuh's (quad_points.cpp); the complete
 // formulas on limbs (P1L, P2L) against proj_add_aff / proj_add, coordinate by coordinate,
 // including every coordinate at 2q - 1, and G1's b3 step on its own. Points are random
 // field elements, not curve points: the formulas are compared as algebra, not the group law.
@@ -86,10 +86,36 @@ static bool g2_bounds(const G2L& a) {
   return true;
 }
 
-// One chain of mixed additions in both forms; returns the limb sum and the word-form sum.
+// The packed sum (X below 5q) in the word form's range: X by a product with one.
+static Fm word_x(const uint32_t X[9]) {
+  uint32_t one[9], x[9];
+  for (int j = 0; j < 9; ++j) one[j] = one29(j);
+  mont29_limbs<Fq29>(X, one, x);
+  Fm w;
+  pack29(x, w.v);
+  return w;
+}
+static Xyzz<Fm> g1_word(const G1L& p) {
+  Xyzz<Fm> r = g1l_pack(p);
+  uint32_t X[9];
+  limbs29_of(r.X.v, X);
+  r.X = word_x(X);
+  return r;
+}
+static Xyzz<Fm2i> g2_word(const G2L& p) {
+  Xyzz<Fm2i> r = g2l_pack(p);
+  uint32_t X[9];
+  limbs29_of(r.X.c0.v, X);
+  r.X.c0 = word_x(X);
+  limbs29_of(r.X.c1.v, X);
+  r.X.c1 = word_x(X);
+  return r;
+}
+
+// Chains of mixed additions in both forms.
 template <class F, class L, class Madd, class Out, class Bounds, class Inf>
 static void chains(const char* name, const std::vector<Aff<F>>& B, int n_chains, Madd madd,
-                   Out out, Bounds bounds, Inf inf, std::vector<std::pair<L, Xyzz<F>>>* keep) {
+                   Out out, Bounds bounds, Inf inf) {
   for (int ch = 0; ch < n_chains; ++ch) {
     Xyzz<F> ref = xyzz_inf<F>();
     L acc = inf();
@@ -111,23 +137,6 @@ static void chains(const char* name, const std::vector<Aff<F>>& B, int n_chains,
       prev = i;
       prev_neg = ng;
     }
-    if (keep) keep->push_back({acc, ref});
-  }
-}
-
-template <class F, class L, class Add, class Out, class Bounds>
-static void sums(const char* name, const std::vector<std::pair<L, Xyzz<F>>>& pts, Add add,
-                 Out out, Bounds bounds) {
-  for (size_t i = 0; i + 1 < pts.size(); ++i) {
-    const auto& p = pts[i];
-    const auto& q = pts[i + 1];
-    const L r = add(p.first, q.first);
-    ++steps;
-    if (!same(out(r), xyzz_add(p.second, q.second))) report(name, (int)i, 0);
-    if (!bounds(r)) report("bounds (add)", (int)i, 0);
-    const L d = add(p.first, p.first);  // the doubling case
-    if (!same(out(d), xyzz_add(p.second, p.second))) report(name, (int)i, 1);
-    if (!bounds(d)) report("bounds (add)", (int)i, 1);
   }
 }
 
@@ -299,33 +308,14 @@ static void complete_g2(const std::vector<Aff<Fm2i>>& B) {
 int main() {
   std::vector<Aff<Fm>> B1(24);
   for (auto& b : B1) rnd_below_2q(b.x), rnd_below_2q(b.y);
-  std::vector<std::pair<G1L, Xyzz<Fm>>> k1;
-  chains<Fm, G1L>("G1 madd", B1, 600, g1l_madd, g1l_out, g1_bounds, g1l_inf, &k1);
-  // p + (-p) through the general addition: negate Y (word form) and convert back.
-  for (size_t i = 0; i < 40 && i < k1.size(); ++i) {
-    Xyzz<Fm> w = g1l_out(k1[i].first);
-    w.Y = neg(w.Y);
-    const G1L r = g1l_add(k1[i].first, g1l_from(w));
-    ++steps;
-    if (!is_zero(g1l_out(r).ZZ) && !is_zero(k1[i].second.ZZ)) report("G1 p + (-p)", (int)i, 0);
-  }
-  sums<Fm, G1L>("G1 add", k1, g1l_add, g1l_out, g1_bounds);
+  chains<Fm, G1L>("G1 madd", B1, 600, g1l_madd, g1_word, g1_bounds, g1l_inf);
   b3_g1();
   complete_g1(B1);
 
   std::vector<Aff<Fm2i>> B2(24);
   for (auto& b : B2) rnd_below_2q(b.x.c0), rnd_below_2q(b.x.c1), rnd_below_2q(b.y.c0),
       rnd_below_2q(b.y.c1);
-  std::vector<std::pair<G2L, Xyzz<Fm2i>>> k2;
-  chains<Fm2i, G2L>("G2 madd", B2, 300, g2l_madd, g2l_out, g2_bounds, g2l_inf, &k2);
-  for (size_t i = 0; i < 20 && i < k2.size(); ++i) {
-    Xyzz<Fm2i> w = g2l_out(k2[i].first);
-    w.Y = neg(w.Y);
-    const G2L r = g2l_add(k2[i].first, g2l_from(w));
-    ++steps;
-    if (!is_zero(g2l_out(r).ZZ) && !is_zero(k2[i].second.ZZ)) report("G2 p + (-p)", (int)i, 0);
-  }
-  sums<Fm2i, G2L>("G2 add", k2, g2l_add, g2l_out, g2_bounds);
+  chains<Fm2i, G2L>("G2 madd", B2, 300, g2l_madd, g2_word, g2_bounds, g2l_inf);
   complete_g2(B2);
 
   if (bad) {
