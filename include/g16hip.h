@@ -429,8 +429,9 @@ void g16hip_ceremony_close(g16hip_ceremony* c);
 /* group 1 or 2; out: the affine sum (64 or 128 bytes). Empty input is infinity. */
 g16hip_status g16hip_ceremony_msm(g16hip_ceremony* c, int group, const uint8_t* bases,
                                   const uint8_t* scalars, size_t n, uint8_t* out);
-/* Device bytes a standalone MSM of n points takes (uploaded inputs, the bases' MSM form,
- * sort and accumulation scratch): what vram_limit is compared with. */
+/* Device bytes a standalone MSM of n points takes at least (uploaded inputs, the bases' MSM
+ * form, sort and accumulation scratch): what vram_limit is compared with. Small MSMs take more
+ * scratch, for speed, where that fits the limit and leaves 8 GiB of the device budget free. */
 g16hip_status g16hip_msm_scratch_bytes(int group, size_t n, size_t* bytes);
 /* Runs the last call took (CudaMsmBackend::last_runs), and the running tally. */
 g16hip_status g16hip_ceremony_last_runs(g16hip_ceremony* c, uint64_t* runs);

@@ -176,12 +176,29 @@ static Xyzz<F> run_msm_on(g16hip_device* d, int group, const void* bases, const 
   return msm_combine(reinterpret_cast<const Xyzz<F>*>(d->host_rows), plan);
 }
 
-// The same with scratch the device owns and grows as needed.
+// Whether the device's scratch holds z, or can grow to it and leave SPARE_BYTES of the budget.
+static bool scratch_to_spare(const g16hip_device* d, const MsmScratchSizes& z) {
+  size_t grow = 0;
+  const auto need = [&](const DevBuf& b, size_t bytes) {
+    if (bytes > b.bytes) grow += bytes - b.bytes;
+  };
+  need(d->scratch_d, z.sort);
+  need(d->scratch_e, z.accum);
+  need(d->msm_bases, z.bases);
+  return grow == 0 || grow + SPARE_BYTES <= device_budget(d);
+}
+
+// The same with scratch the device owns and grows as needed: the least where the larger scratch
+// of short segments would leave less than SPARE_BYTES (or `lean` asks for it).
 template <class F>
 static Xyzz<F> run_msm(g16hip_device* d, int group, const void* bases, const void* scalars,
                        uint32_t n, int c, bool lean = false) {
   c = msm_width(n, c);
-  const MsmScratchSizes z = msm_scratch_sizes(group, n, c, d->constant_work, lean);
+  MsmScratchSizes z = msm_scratch_sizes(group, n, c, d->constant_work, lean);
+  if (!lean && !scratch_to_spare(d, z)) {
+    lean = true;
+    z = msm_scratch_sizes(group, n, c, d->constant_work, lean);
+  }
   d->scratch_d.alloc(z.sort);
   d->scratch_e.alloc(z.accum);
   d->msm_bases.alloc(z.bases);

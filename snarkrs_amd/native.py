@@ -656,7 +656,7 @@ class CeremonyMsm:
 
     @staticmethod
     def scratch_bytes(group: int, n: int) -> int:
-        """Device bytes one run of n points takes (what ``vram_limit`` is compared with)."""
+        """Device bytes one run of n points takes at least (what ``vram_limit`` is compared with)."""
         b = ctypes.c_size_t()
         _check(load().g16hip_msm_scratch_bytes(group, n, ctypes.byref(b)))
         return b.value

@@ -7,7 +7,8 @@
 * a prove from a snarkjs .zkey / .wtns pair written to disk and read back by the codec
   (the reference's warm bench input path, bin/snarkrs/src/bench.rs:461-467);
 * the device-memory budget: a key over it is refused as DeviceMemory with nothing allocated,
-  a key at it prepares and proves (crates/cuda/src/backend.rs:722-771);
+  a key at it prepares and proves (crates/cuda/src/backend.rs:722-771); slots, waves and MSMs
+  that take no more than is reported for them where less than 8 GiB would stay free;
 * H MSM widths above 16 over window tables (G16HIP_C_H = 17 and 20: buckets of 2^16 and 2^19,
   the 24-bit digit code, rows cut into many slices), which the width model does not pick.
 """
@@ -15,7 +16,7 @@ import numpy as np
 import pytest
 
 from oracle.oracle import Synth
-from snarkrs_amd import native
+from snarkrs_amd import native, synth
 from snarkrs_amd.wire import MONT_R, R_MOD, fr_array, fr_ints
 from snarkrs_amd.zkey import load_wtns, load_zkey, write_wtns, write_zkey
 
@@ -149,3 +150,27 @@ def test_key_and_slot_take_what_is_predicted(dev, orc):
         assert predicted - 40 * (2 << 20) < circ.resident_bytes() <= predicted
     finally:
         circ.release()
+
+
+@pytest.mark.parametrize("group,n", [(1, 1 << 18), (2, 1 << 16)])
+def test_msm_scratch_without_spare_memory(dev, group, n):
+    # With less than 8 GiB to spare a standalone MSM takes no more than the figure reported for
+    # it, so that one that fits a nearly full device is not refused for the sake of speed.
+    from snarkrs_amd.devmem import DeviceArray
+
+    bases = DeviceArray(dev.fixed_base(group, synth.scalars(41, n, 0)))
+    scalars = DeviceArray(synth.scalars(42, n, 300))
+    got, used = [], []
+    for limit in (0, 0, 1 << 30):  # the first call also pays for what the runtime keeps
+        d = native.Device(0)
+        try:
+            d.set_vram_limit(limit)
+            free = d.mem_info()[0]
+            got.append(d.msm_device(group, bases.addr, scalars.addr, n))
+            used.append(free - d.mem_info()[0])
+            got.append(d.msm_device(group, bases.addr, scalars.addr, n))
+        finally:
+            d.close()
+    assert all((g == got[0]).all() for g in got)
+    inputs = n * (32 + 64 * group)  # counted in the figure, held by the caller here
+    assert used[2] <= native.CeremonyMsm.scratch_bytes(group, n) - inputs + 4 * (2 << 20) < used[1]
