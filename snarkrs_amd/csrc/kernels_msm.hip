@@ -533,11 +533,15 @@ __global__ void k_scan_fix(uint32_t* offset, const uint32_t* bsum, uint32_t K) {
 
 // The whole sort of a small MSM in one workgroup: every bucket's count in LDS, a scan, then the
 // entries to their places (the digits are computed twice instead of stored). It is bound by one
-// compute unit's instruction issue, 35 us for 30 thousand entries, as long as the general path's
-// ten kernels together, but those spend as much again between their launches: the
-// 1000-constraint prove, which sorts twice, 895 -> 810 us (MI355X). Up to TINY_ENTRIES entries
-// and TINY_BUCKETS buckets.
-static constexpr uint32_t TINY_ENTRIES = 131072;
+// compute unit's instruction issue, so it pays while that is shorter than the general path's ten
+// kernels and the time between their launches. Whole calls, one workgroup against the general
+// path, us (MI355X, medians of five runs of each in turn):
+//   G1 MSM   10 200 entries 242 : 256   30 100 278 : 286   34 400 308 : 285    55 500 316 : 286
+//   G2 MSM   10 200         355 : 387   20 400 389 : 386   34 400 406 : 386    55 500 446 : 417
+//   prove     9 600         428 : 439   25 600 512 : 509   31 300 630 : 601   100 000 835 : 691
+// (a proof's witness entries, and about as many of H). Up to TINY_ENTRIES entries, where the two
+// are within 3 % of each other, and TINY_BUCKETS buckets.
+static constexpr uint32_t TINY_ENTRIES = 32768;
 static constexpr uint32_t TINY_BUCKETS = 15360;  // 60 KB of LDS
 
 __global__ void __launch_bounds__(SORT_THREADS) k_sort_tiny(const uint4* scalars, uint32_t n,

@@ -50,10 +50,11 @@ def test_least_scratch_runs_in_one_piece(dev, group, n):
 
 
 @pytest.mark.parametrize("constant", [False, True])
-@pytest.mark.parametrize("n", [1, 63, 1023, 1024, 1025, 4095, 4096, 4097, 6000])
+@pytest.mark.parametrize("n", [1, 63, 762, 763, 1023, 1024, 1025, 4095, 4096, 4097, 6000])
 def test_sort_of_small_msms(dev, n, constant):
-    # The one-workgroup sort and the general one either side of their limits, on boolean-heavy
-    # scalars (most entries in one bucket).
+    # The one-workgroup sort and the general one either side of their limit (762 points of 43
+    # windows are its last) and of a round of threads, on boolean-heavy scalars (most entries in
+    # one bucket).
     rng = SplitMix64(70 + n)
     ks = [rng.next_fr() for _ in range(n)]
     ss = [rng.next_fr() if i % 4 == 0 else i % 2 for i in range(n)]
