@@ -453,11 +453,14 @@ static bool try_add_slot(g16hip_circuit* C, size_t reserve, uint32_t more);
 
 // Exclusive use of one of the circuit's slots. Waits for a free one; with `cap` > 0, first
 // adds a slot (up to `cap` in all, while the device keeps `reserve` bytes free) when every
-// slot is busy.
+// slot is busy. A call that fails with work of its own on the slot's streams waits for it before
+// the slot is free again: the next proof writes the pinned memory that this work reads and writes
+// (the blinders and their products, the staged witness).
 struct SlotLease {
   g16hip_circuit* C;
   size_t idx;
   Slot* S;
+  const int unwinding = std::uncaught_exceptions();
   explicit SlotLease(g16hip_circuit* c, uint32_t cap = 0, size_t reserve = 0) : C(c) {
     std::unique_lock<std::mutex> lk(C->mu);
     for (;;) {
@@ -487,6 +490,8 @@ struct SlotLease {
     S = C->slots[idx].get();
   }
   ~SlotLease() {
+    if (std::uncaught_exceptions() > unwinding)
+      for (hipStream_t st : {S->stream, S->side[0], S->side[1]}) (void)hipStreamSynchronize(st);
     {
       std::lock_guard<std::mutex> lk(C->mu);
       C->busy[idx] = false;
