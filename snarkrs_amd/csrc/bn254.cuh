@@ -227,8 +227,10 @@ HD Fp<C> mul(const Fp<C>& a, const Fp<C>& b) {
 
 // Montgomery product for R' = 2^261: CIOS over nine 29-bit limbs with 64-bit column
 // accumulators. Every partial product is one 29x29+64 multiply-add; the columns take the
-// carries lazily (each stays below 2^63: at most 18 products of 2^58 land in one column), so
-// the loop has no carry flags at all, which the 32-bit form above needs on every step. On
+// carries lazily, so the loop has no carry flags at all, which the 32-bit form above needs on
+// every step. A column holds at most nine products of limbs below 2^29 + 8 and what the reduction
+// below adds: under 22.0 2^58 over Fq and 37.2 2^58 over Fr, so below 2^64 but not 2^63, and
+// every shift of a column is unsigned. On
 // gfx950 this runs 1.42x the 32-bit form's products per second. Inputs and output are the
 // usual 8 x 32-bit limbs, the output fully reduced. M29 gives the modulus in 29-bit limbs,
 // -modulus^-1 mod 2^29 and w = 2^-29 mod the modulus.
@@ -252,7 +254,7 @@ struct Fq29 {
   static constexpr uint32_t N29 = 0x04866389u;
   // 2^-29 + 2q mod 2^261: of the small multiples of q added to 2^-29 mod q, the one whose
   // limbs are smallest (any seven consecutive ones sum to at most 1.65 2^29).
-  static HD uint32_t w29(int j) {
+  static constexpr HD uint32_t w29(int j) {
     constexpr uint32_t W[9] = {0x0872952du, 0x0808854au, 0x065124e0u, 0x029b9885u, 0x03f6b850u,
                                0x148e9764u, 0x02b3e954u, 0x0843f777u, 0x0067a061u};
     return W[j];
@@ -267,7 +269,8 @@ struct Fr29 {
     return P[j];
   }
   static constexpr uint32_t N29 = 0x0fffffffu;
-  static HD uint32_t w29(int j) {  // 2^-29 mod r
+  // 2^-29 mod r: seven consecutive limbs sum to 3.58 2^29, too much for redc29.
+  static constexpr HD uint32_t w29(int j) {
     constexpr uint32_t W[9] = {0x18f05361u, 0x012bb1feu, 0x0f5d8135u, 0x1e6275f6u, 0x07e7a880u,
                                0x10c6bf1fu, 0x11f74a6cu, 0x06fdaecbu, 0x00183227u};
     return W[j];
@@ -378,6 +381,18 @@ HD void wide_msub(uint64_t t[17], const uint32_t A[9], const uint32_t B[9]) {
   }
 }
 
+// Whether seven consecutive limbs of w sum to at most 1.75 2^29, which the bounds of the lazy
+// reductions below count on: the steps add that times 2^32 to a column.
+template <class M29>
+constexpr bool w29_small() {
+  for (int i = 0; i < 3; ++i) {
+    uint64_t sum = 0;
+    for (int j = 0; j < 7; ++j) sum += M29::w29(i + j);
+    if (sum > 7ull << 27) return false;
+  }
+  return true;
+}
+
 // t 2^-261 mod the modulus as nine 29-bit limbs in [0, 2 modulus), for a wide value
 // V = sum_k t[k] 2^(29 k), |V| < (1 - 2^-24) 2^261 modulus, that sums at most two products
 // of each sign (operands below 16 modulus in limbs below 2^29 + 8). A column then holds at most
@@ -388,6 +403,7 @@ HD void wide_msub(uint64_t t[17], const uint32_t A[9], const uint32_t B[9]) {
 // modulus added (NEG = false: V >= 0, nothing to add).
 template <class M29, bool NEG = true>
 HD void redc29(uint64_t t[17], uint32_t R[9]) {
+  static_assert(w29_small<M29>(), "a column would leave int64");
   constexpr uint32_t MASK = (1u << 29) - 1u;
 #pragma unroll
   for (int i = 0; i < 9; ++i) {
@@ -1683,6 +1699,7 @@ struct P2L {
 // carries shift unsigned. The value is below (1 - 2^-24) 2^261 q, the result below 2q.
 template <class M29>
 HD void redc29u(uint64_t t[17], uint32_t R[9]) {
+  static_assert(w29_small<M29>(), "the columns' bound is for small limbs of w");
   constexpr uint32_t MASK = (1u << 29) - 1u;
 #pragma unroll
   for (int i = 0; i < 9; ++i) {

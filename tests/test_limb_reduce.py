@@ -96,6 +96,51 @@ def test_sums(run, op, bounds):
         assert got < 2 * Q_MOD and (got * 2**261 - want) % Q_MOD == 0
 
 
+def column_bound(m, products, limb, top):
+    """The largest any column of a sum of so many products gets in the reduction, where every
+    dropped low word is 2^32 - 1 and every digit 2^29 - 1."""
+    w = limbs(pow(2, -29, m) + (2 * m if m == Q_MOD else 0))
+    op = [limb] * 8 + [top]
+    t = [0] * 18
+    for i in range(9):
+        for j in range(9):
+            t[i + j] += products * op[i] * op[j]
+    most = max(t)
+    for i in range(9):
+        if i < 7:
+            t[i + 1] += 8 * (t[i] >> 32)
+            for j in range(9):
+                t[i + 1 + j] += (2**32 - 1) * w[j]
+        else:
+            for j in range(9):
+                t[i + j] += (2**29 - 1) * limbs(m)[j]
+            t[i + 1] += t[i] >> 29
+        most = max(most, max(t))
+    return most
+
+
+def test_column_bounds():
+    limb, top = 2**29 + 7, 2**26
+    assert column_bound(Q_MOD, 1, limb, top) < 22.0 * 2**58
+    assert 2**63 < column_bound(R_MOD, 1, limb, top) < 37.2 * 2**58  # unsigned, below 2^64
+    assert column_bound(Q_MOD, 2, limb, top) < 31.4 * 2**58          # redc29: signed
+    assert column_bound(Q_MOD, 4, limb, top) < 51.3 * 2**58          # redc29u
+    assert column_bound(R_MOD, 2, limb, top) > 2**63                 # not redc29's
+
+
+@pytest.mark.parametrize("call", ["redc29", "redc29u"])
+def test_lazy_reductions_refuse_large_limbs(tmp_path, call):
+    header = os.path.join(HERE, "..", "snarkrs_amd", "csrc", "bn254.cuh")
+    for field, fits in (("Fq29", True), ("Fr29", False)):
+        src = tmp_path / "reduce.cpp"
+        src.write_text(f'#include "{header}"\nusing namespace g16;\n'
+                       f"void f(uint64_t* t, uint32_t* r) {{ {call}<{field}>(t, r); }}\n")
+        r = subprocess.run([HIPCC, "-std=c++17", "--cuda-host-only", "-x", "hip", "-fsyntax-only",
+                            str(src)], capture_output=True, text=True, timeout=300)
+        assert (r.returncode == 0) == fits, r.stderr
+        assert fits or "static assertion failed" in r.stderr
+
+
 def test_pack(run):
     rng = random.Random(7)
     xs = operands(Q_MOD, 9, rng)
