@@ -111,3 +111,19 @@ def test_reduction_group_widths(dev, group, c, constant):
         dev.set_constant_work(False)
     total = sum(k * s for k, s in zip(ks, ss)) % R_MOD
     assert (got == dev.fixed_base(group, fr_array([total]))[0]).all()
+
+
+@pytest.mark.parametrize("group,n", [(1, 20480), (1, 20481), (2, 8192), (2, 8193)])
+def test_segment_sums_over_lanes_and_not(dev, group, n):
+    # Sixteen windows: the segments of the smaller n take 131072 lanes, the most that are spread,
+    # and those of the next n one lane each.
+    from snarkrs_amd.devmem import DeviceArray
+
+    rng = SplitMix64(50 + n)
+    ks = [rng.next_fr() for _ in range(257)]
+    ss = [rng.next_fr() for _ in range(n)]
+    base = dev.fixed_base(group, fr_array(ks))
+    bases = DeviceArray(base[[i % 257 for i in range(n)]])
+    got = dev.msm_device(group, bases.addr, DeviceArray(fr_array(ss)).addr, n, 16)
+    total = sum(ks[i % 257] * s for i, s in enumerate(ss)) % R_MOD
+    assert (got == dev.fixed_base(group, fr_array([total]))[0]).all()

@@ -56,6 +56,19 @@ def test_repeated_proofs_are_identical(dev, orc, small):
         assert (circ.prove_with_blinders(wit, r, s) == first).all()
 
 
+def test_blinders_at_the_ends_of_their_range(dev, orc, small):
+    # The blinding products' scalars r, s and rs: one bit, every bit of r - 1, the top bit alone.
+    _, key, wit = small
+    circ = dev.prepare(key)
+    pairs = [(1, 1), (1, R_MOD - 1), (R_MOD - 1, R_MOD - 1), (1 << 253, 2), (3, 1 << 128)]
+    items = [(circ, wit, fr_array([r]), fr_array([s])) for r, s in pairs]
+    want = [orc.prove(key, wit, r, s)[1] for r, s in pairs]
+    for (_, _, r, s), w in zip(items, want):
+        assert (circ.prove_with_blinders(wit, r, s) == w).all()
+    for got, w in zip(native.prove_batch(items), want):
+        assert (got == w).all()
+
+
 def test_concurrent_proofs_on_one_circuit(dev, orc, small):
     _, key, wit = small
     circ = dev.prepare(key)
