@@ -104,7 +104,7 @@ struct MsmPlan {
   // discarded, and the accumulation computes its addition and keeps the old sum by a select.
   // Entry values are then index << 2 | discard << 1 | sign (index < 2^30).
   bool constant = false;
-  // Entries per accumulation segment, for G1 and G2 bases (msm_segments).
+  // Entries per accumulation segment, for G1 and G2 bases (segment_length, kernels_msm.hip).
   uint32_t seg[2] = {0, 0};
   // device scratch (owned by the caller)
   uint32_t* offset = nullptr;   // [K + 1] first entry of each bucket (K = sets * nb); [K] = total

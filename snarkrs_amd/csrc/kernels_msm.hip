@@ -763,9 +763,9 @@ size_t msm_sort_scratch_bytes(uint32_t n, int c, bool lean, uint32_t batch) {
 // Entries per segment: 32, and 40 for a G1 MSM over per-window buckets, whose merges are one or
 // two additions per bucket, so fewer and longer segments pay there (the 2^20 G1 MSM: 2.13
 // against 2.25-2.30 ms; G2 and the prove's merged MSMs were slower).
-// Constant-work MSMs over window tables (the prove's) take 64: their accumulation runs the
-// same number of rounds of waves at the prove's sizes and the fold starts from half the slots
-// (47.8-47.9 against 47.4-47.5 proofs/s).
+// Constant-work MSMs over window tables (the prove's) take 64, so that the fold starts from half
+// the slots: the 1.1M-constraint prove 21.2 ms against 21.7 with 32, but 300k 7.18 against 6.75,
+// where 64 leaves G2 at 82 thousand lanes, just past the halving below.
 // A segment is a chain of dependent additions on one lane, 5 us each in G1 and 13 in G2 while
 // the device is not full, so an MSM whose segments would not fill it halves them until they do,
 // down to 8 (G1 over per-window buckets: 10; constant work: 16, 20). MI355X: G1 MSM of 4099 points

@@ -351,7 +351,11 @@ static void launch_merge(const TailJobs& t, hipStream_t s) {
 
 template <bool G2>
 static void merge_jobs(const TailJobs& t, hipStream_t s) {
-  // Points per bucket from the average pieces per bucket.
+  // Points per bucket from the average pieces per bucket. With both lines at half as many pieces
+  // G2 MSMs of 2^16 and 2^18 take 865 and 1721 us for 773 and 1533 and a batch of sixteen
+  // 60k-constraint proofs 12.2 ms for 11.0; at twice as many the 1.1M-constraint prove takes 15.0
+  // ms for 11.7 and the 5000-constraint one 753 us for 707, though G1 MSMs of 2^16 and 2^18
+  // gain (478 for 510 us, 708 for 775): one pair of lines is a compromise (MI355X).
   const uint32_t m = most(t, [](const TailJob& j) { return j.avg_pieces; });
   if (m < 3) launch_merge<G2, 1>(t, s);
   else if (m < 24) launch_merge<G2, 4>(t, s);

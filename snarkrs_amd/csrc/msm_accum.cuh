@@ -451,7 +451,12 @@ __global__ void __launch_bounds__(128) k_fold_const(const ConstJobs jobs, int fr
 // stores it to its bucket; with several workgroups a workgroup's first and last runs go to
 // slots 2b and 2b + 1 of the next level instead, as a fold group's do. A level of 512 slots to 2
 // is 9 additions deep, where fold levels are 8 deep for a factor of 4, at 9 times their work; so
-// folds run down to FROM slots (G1 131072, G2 32768: a level there is as long on the device as it is deep). The level count depends on m only.
+// folds run down to FROM slots (G1 131072, G2 32768: a level there is about as long on the device
+// as it is deep). The level count depends on m only. Other lines, MI355X: G1 at 65536, MSM of 2^15
+// 688 us for 658 and 2^18 1154 for 1127; at 262144, the 100k-constraint prove 3.61 ms for 3.35. G2
+// at 16384, MSM of 2^15 1381 us for 1265 and 2^18 3727 for 3593; at 65536, 2^14 1111 for 1209, 2^16
+// 1783 for 1888, and the 131k prove 4.27 ms for 4.39, with 300k and 450k within 0.4 %: the better
+// line for G2 lies between.
 // BLOCK: slots per scan, as many threads as the point form's registers allow in one workgroup.
 template <class F>
 struct ScanSlots {

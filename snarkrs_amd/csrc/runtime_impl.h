@@ -560,8 +560,8 @@ inline void note_accumulate(g16hip_device* d, int group, uint64_t entries, doubl
 
 inline void set_device(const g16hip_device* d) { G16_CHECK(hipSetDevice(d->ordinal)); }
 
-// Rows of a standalone MSM: at most 128 sets of one row (width 2), 29 of 8 (width 9) and the
-// like; 512 G2 points hold any.
+// Rows of a standalone MSM: 22 sets of 10 rows at width 12 are the most of any width in [2, 16];
+// 512 G2 points hold them, and run_msm_on checks.
 constexpr size_t ROWS_POINTS = 512, ROWS_BYTES = 256 * ROWS_POINTS;
 
 // Device scratch of one standalone MSM: the sort's, the accumulation's (window sums behind
