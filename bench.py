@@ -41,9 +41,9 @@ PEAK_MUL32_PER_S = 256 * 4 * 16 * 2.4e9
 # 28 (G2: 3 Fq products per Fq2 product); one Fq product = 136 32x32 partial products (CIOS).
 MUL32_PER_MADD = {1: 10 * 136, 2: 28 * 136}
 # HBM bytes per k_accumulate<Fm> launch in the 1.1M-constraint prove (FETCH_SIZE + WRITE_SIZE,
-# scaled by the counters' reading of a 256 MiB device copy: fetch x2, write x1), from the
+# scaled by the counters' reading of a device copy: fetch x2, write x1), from the
 # rocprofv3 --pmc runs in profiles/k_accumulate_traffic_1_1M.txt.
-ACCUMULATE_TRAFFIC_BYTES_1_1M = 3.39e9
+ACCUMULATE_TRAFFIC_BYTES_1_1M = 3.57e9
 # Reference, CUDA back end on a Tesla T4: single prove, synthetic key, domain 2^21, warm:
 # 1263 ms (bench/results/cuda-size-sweep-2026-11-10.md:26).
 REFERENCE_T4_PROVE_MS_2_21 = 1263.0
