@@ -444,7 +444,8 @@ struct SetSums {
 struct CombineHelp {
   static constexpr int MOST = 8;
   static inline std::atomic<int> in_use{0};
-  CombineHelp() { ++in_use; }
+  const bool got;  // counted: one of the MOST
+  CombineHelp() : got(in_use.fetch_add(1) < MOST) {}
   CombineHelp(const CombineHelp&) = delete;
   CombineHelp& operator=(const CombineHelp&) = delete;
   ~CombineHelp() { --in_use; }
@@ -464,8 +465,9 @@ Xyzz<F> msm_combine(const Xyzz<F>* P, const MsmPlan& p) {
     // never reads the rows. Without a helper (none left, no thread to be had) the pass does all
     // of them.
     try {
-      for (int h = 0; h < 3 && CombineHelp::in_use.load() < CombineHelp::MOST; ++h) {
+      for (int h = 0; h < 3; ++h) {
         const auto help = std::make_shared<CombineHelp>();
+        if (!help->got) break;
         host_pool_run([sums, help] {
           for (int w = sums->W - 1; w >= 0; --w) sums->take(w);
         });
