@@ -1190,8 +1190,12 @@ static void finish_wave(g16hip_circuit* C, Wave* W, const std::vector<WaveItem>&
   static char anchor;
   const WavePlans P = wave_plans(C, &anchor, &anchor, m, cap, W->fast);
   const uint8_t* rows = W->host_wout[b];
+  // The wave's own threads finish side by side: fewer helpers each. Sixteen proofs of 22k
+  // constraints without window tables: one 9.47 ms, none 9.79, three 10.1 (MI355X).
+  const int helpers = std::max(1, std::min(3, 8 / (int)m));
   auto g1 = [&](int j, uint32_t k, const MsmPlan& v) {
-    return msm_combine(reinterpret_cast<const G1X*>(rows + wave_rows_offset(P, cap, j, k)), v);
+    return msm_combine(reinterpret_cast<const G1X*>(rows + wave_rows_offset(P, cap, j, k)), v,
+                       helpers);
   };
   auto one = [&](uint32_t k) {
     const WaveItem& w = it[k];
@@ -1207,7 +1211,7 @@ static void finish_wave(g16hip_circuit* C, Wave* W, const std::vector<WaveItem>&
       g1_store(mo.l_g1, host_to_aff(g1(2, k, P.vw)));
       g2_store(mo.b_g2, host_to_aff(msm_combine(
                             reinterpret_cast<const G2X*>(rows + wave_rows_offset(P, cap, 3, k)),
-                            P.vw)));
+                            P.vw, helpers)));
       g1_store(mo.h_g1, host_to_aff(g1(4, k, P.vh)));
       bp.sA = host_mul(A, bp.s_std.v);
       bp.rB1 = host_mul(B1, bp.r_std.v);

@@ -439,20 +439,9 @@ struct SetSums {
   }
 };
 
-// One queued or running helper of msm_combine, of the process's few: every thread that finishes
-// a proof of a wave would ask for three.
-struct CombineHelp {
-  static constexpr int MOST = 8;
-  static inline std::atomic<int> in_use{0};
-  const bool got;  // counted: one of the MOST
-  CombineHelp() : got(in_use.fetch_add(1) < MOST) {}
-  CombineHelp(const CombineHelp&) = delete;
-  CombineHelp& operator=(const CombineHelp&) = delete;
-  ~CombineHelp() { --in_use; }
-};
-
+// `helpers`: how many pooled threads may take sets' sums.
 template <class F>
-Xyzz<F> msm_combine(const Xyzz<F>* P, const MsmPlan& p) {
+Xyzz<F> msm_combine(const Xyzz<F>* P, const MsmPlan& p, int helpers = 3) {
   typedef typename SetSums<F>::H H;
   const auto sums = std::make_shared<SetSums<F>>(P, p);
   const int c = p.c, W = sums->W;  // one set when the windows are merged
@@ -462,16 +451,12 @@ Xyzz<F> msm_combine(const Xyzz<F>* P, const MsmPlan& p) {
   } else {
     // Nothing waits for a helper that has not begun: the pass ends with every sum taken, the
     // helpers share the state's ownership, and one that starts later finds nothing to take and
-    // never reads the rows. Without a helper (none left, no thread to be had) the pass does all
-    // of them.
+    // never reads the rows. Without a helper (no thread to be had) the pass does all of them.
     try {
-      for (int h = 0; h < 3; ++h) {
-        const auto help = std::make_shared<CombineHelp>();
-        if (!help->got) break;
-        host_pool_run([sums, help] {
+      for (int h = 0; h < helpers; ++h)
+        host_pool_run([sums] {
           for (int w = sums->W - 1; w >= 0; --w) sums->take(w);
         });
-      }
     } catch (...) {
     }
     for (int w = W - 1; w >= 0; --w) {

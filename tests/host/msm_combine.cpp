@@ -1,8 +1,7 @@
 // msm_combine (snarkrs_amd/csrc/runtime_impl.h) with the helper pool in this file's hands, for
 // tests/test_msm_combine.py: rows k G of known k, combined while the pool
 //   run    starts a thread per task,
-//   late   starts none until the result is there and the rows are gone (of eight calls at a
-//          time, which may queue eight helpers between them),
+//   late   starts none until the results are there and the rows are gone,
 //   throw  refuses every task.
 // Prints "ok" when every sum is the point it should be.
 #include <cstdio>
@@ -78,13 +77,13 @@ int main(int, char** argv) {
     const Aff<Fq> ref = host_to_aff(host_mul(G, want));
     std::atomic<int> wrong{0};
     const auto call = [&] {
-      const Aff<Fq> got = host_to_aff(msm_combine(at.data(), p));
+      const Aff<Fq> got = host_to_aff(msm_combine(at.data(), p, 1 + rep % 3));
       wrong += std::memcmp(&got, &ref, sizeof got) != 0;
     };
     std::vector<std::thread> callers;
     for (int k = 0; k < 8; ++k) callers.emplace_back(call);
     for (auto& t : callers) t.join();
-    bad += wrong.load() + (tasks.size() > 8);
+    bad += wrong.load() + (tasks.size() > 8u * (1 + rep % 3));
     at = std::vector<Xyzz<Fq>>();  // a helper that starts now must not need the rows
     for (auto& t : tasks) t();
     tasks.clear();
